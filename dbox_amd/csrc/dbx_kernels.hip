@@ -3238,7 +3238,7 @@ __device__ __forceinline__ int bp_pairs(const float4 *gfat, const int *gmoved, i
     // along the axis (a container wall) does not serialise the sweep.  Found
     // pairs are collected as (a << 32 | b) keys and sorted, which is the
     // b2PairLessThan order.
-    if (stage) {
+    {
         __shared__ int s_np;
         if (tid == 0) s_np = 0;
         for (int p = tid; p < n; p += BS) {
@@ -4745,13 +4745,207 @@ static hipError_t launch_wide(const Dev &d, const WideBp &b, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------
+// Stand-alone broadphase on caller-given AABBs (dbx_broadphase_pairs*): every
+// i < j that overlaps with i or j moved, in (i, j) order, over the whole device.
+//
+// All pairs are tested instead of sorted and swept: the pair set then does not
+// depend on how the boxes lie, each row meets its partners in ascending order (no
+// sort of the pairs either), and the 134 M tests of 16,384 proxies are less than
+// the launches of a device-wide sort.  A wave holds 128 rows in its lanes, two each,
+// and 64 proxies j in its lanes, whose AABBs it reads out by v_readlane: no memory
+// access between the tests (j through the scalar cache waited for it at every
+// fourth test).  The first launch counts per row and segment of j and keeps each
+// tile's first kBp1Hits hits, the second turns counts into places, the third writes
+// the kept hits (a tile with more of them tests again).  At 16,000 proxies with two
+// pairs each: 60 + 8 + 4 us, against 17,600 us for the one-workgroup sort and sweep in
+// global memory before; the whole call 18,065 -> 81 us.  Bound by vector issue of the
+// tests (about 34 us of it at full clock and perfect balance) at the largest sizes, by
+// the three launches below about 4,000 proxies.
+// ---------------------------------------------------------------------------
+constexpr int kBp1Segs = 64; // segments of j per row; the tests of a row are split over them
+constexpr int kBp1Hits = 64; // hits kept per tile of 128 rows and segment, one per lane of the write
+struct Bp1 {
+    int nblk, nseg, S; // 256-row blocks, segments, proxies per segment (a multiple of 64)
+    int *cnt;          // [nseg][256 nblk] hits per segment and row, then the row's hits before the segment
+    int *nhit;         // [nseg][2 nblk] hits per segment and tile
+    uint2 *hits;       // [nseg][2 nblk][kBp1Hits]: row in the tile | place in the row's segment << 7, j
+    int *row;          // [256 nblk] hits of the block's rows before this one
+    int *sum;          // [nblk] hits of the block
+};
+__host__ __device__ inline Bp1 bp1_carve(char *p, int n, size_t &bytes) {
+    Bp1 b;
+    b.nblk = (n + 255) / 256;
+    b.S = ((n + kBp1Segs - 1) / kBp1Segs + 63) / 64 * 64;
+    b.nseg = n > 0 ? (n + b.S - 1) / b.S : 0;
+    const size_t rows = 256 * (size_t)b.nblk;
+    char *q = p;
+    b.cnt = (int *)q; q += 4 * rows * b.nseg;
+    b.hits = (uint2 *)q; q += 8 * kBp1Hits * 2 * (size_t)b.nblk * b.nseg;
+    b.row = (int *)q; q += 4 * rows;
+    b.nhit = (int *)q; q += isl_align(8 * (size_t)b.nblk * b.nseg);
+    b.sum = (int *)q; q += isl_align(4 * (size_t)b.nblk);
+    bytes = (size_t)(q - p);
+    return b;
+}
+// The row blocks of a segment that can hold a pair: their first row comes before the
+// segment's last proxy.  Only these (block, segment) cells are launched, one
+// workgroup each in segment order: with the others launched too and returning at
+// once, the working ones came to lie unevenly on the CUs (169,000 busy cycles against
+// 81,000 of vector issue).
+__host__ __device__ __forceinline__ int bp1_live(const Bp1 &b, int seg) {
+    const int l = (b.S * (seg + 1) + 254) / 256;
+    return l < b.nblk ? l : b.nblk;
+}
+static_assert(kBp1Segs == 64, "bp1_cell takes a segment per lane");
+__device__ __forceinline__ void bp1_cell(const Bp1 &b, int cell, int &blk, int &seg) {
+    const int lane = threadIdx.x & 63, mine = lane < b.nseg ? bp1_live(b, lane) : 0;
+    const int end = wave_incl_scan(mine);
+    seg = __popcll(__builtin_amdgcn_ballot_w64(end <= cell));
+    blk = cell - (seg > 0 ? __builtin_amdgcn_readlane(end, seg - 1) : 0);
+}
+// Positive exactly when a and f do not overlap (b2TestOverlap, overlap()): the
+// largest of the four gaps.  The constant stands for a gap that is not a number
+// (infinity minus infinity), which overlap() does not take for a separation either.
+__device__ __forceinline__ float bp1_gap(float4 a, float4 f) {
+    return __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(f.x - a.z, f.y - a.w), a.x - f.z),
+                           __builtin_fmaxf(a.y - f.w, -1.0f));
+}
+__device__ __forceinline__ float lane_value(float x, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
+// Calls found(u, rows, j) for each j of [j0, j1) in turn and u = 0, 1 with the rows
+// (a lane mask) of the wave's rows r0 + 64 u + lane that pair with j.  Four proxies
+// per step; only a step with an overlap looks at the moved flags and the order.
+template <class F>
+__device__ __forceinline__ void bp1_tests(const float4 *__restrict__ fat, const int *__restrict__ moved, int n, int r0,
+                                          int j0, int j1, F &&found) {
+    const int lane = threadIdx.x & 63;
+    float4 a[2];
+    unsigned long long vm[2], mm[2]; // the rows below n, and those of them that moved
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int i = r0 + 64 * u + lane;
+        a[u] = fat[min(i, n - 1)];
+        vm[u] = __builtin_amdgcn_ballot_w64(i < n);
+        mm[u] = vm[u] & __builtin_amdgcn_ballot_w64(moved[min(i, n - 1)] != 0);
+    }
+    for (int c = j0; c < j1; c += 64) {
+        const int q = min(c + lane, n - 1), len = min(64, j1 - c);
+        const float4 g = fat[q];
+        const unsigned long long jm = __builtin_amdgcn_ballot_w64(moved[q] != 0);
+        for (int l = 0; l < len; l += 4) { // lanes past len hold a proxy of the segment or the last one: not reported
+            float gap[4][2], least = 1.0f;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float4 f = make_float4(lane_value(g.x, l + v), lane_value(g.y, l + v), lane_value(g.z, l + v),
+                                             lane_value(g.w, l + v));
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    gap[v][u] = bp1_gap(a[u], f);
+                    least = __builtin_fminf(least, gap[v][u]);
+                }
+            }
+            if (!__builtin_amdgcn_ballot_w64(least <= 0.0f)) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int j = c + l + v;
+                if (l + v >= len) break;
+                const bool mj = ((jm >> (l + v)) & 1ull) != 0;
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const unsigned long long rows = __builtin_amdgcn_ballot_w64(gap[v][u] <= 0.0f) &
+                                                    (mj ? vm[u] : mm[u]) &
+                                                    __builtin_amdgcn_ballot_w64(j > r0 + 64 * u + lane);
+                    if (rows) found(u, rows, j);
+                }
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(128) void k_bp1_count(const float4 *__restrict__ fat, const int *__restrict__ moved, int n,
+                                                   Bp1 b) {
+    const int lane = threadIdx.x & 63;
+    int blk, seg;
+    bp1_cell(b, blockIdx.x, blk, seg);
+    const int tile = 2 * blk + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r0 = 128 * tile;
+    const size_t t = (size_t)seg * 2 * b.nblk + tile;
+    int cnt[2] = {0, 0}, nh = 0;
+    bp1_tests(fat, moved, n, r0, b.S * seg, min(b.S * (seg + 1), n), [&](int u, unsigned long long rows, int j) {
+        if ((rows >> lane) & 1ull) {
+            const int slot = nh + __popcll(rows & ((1ull << lane) - 1ull));
+            if (slot < kBp1Hits)
+                b.hits[t * kBp1Hits + slot] = make_uint2((unsigned)(64 * u + lane) | (unsigned)cnt[u] << 7, (unsigned)j);
+            ++cnt[u];
+        }
+        nh += __popcll(rows);
+    });
+    int *c = b.cnt + (size_t)seg * 256 * b.nblk + r0 + lane;
+    c[0] = cnt[0];
+    c[64] = cnt[1];
+    if (lane == 0) b.nhit[t] = nh;
+}
+
+__global__ __launch_bounds__(256) void k_bp1_scan(Bp1 b) {
+    __shared__ int s_tmp[5];
+    const int blk = blockIdx.x, i = 256 * blk + (int)threadIdx.x;
+    int v[kBp1Segs], run = 0;
+#pragma unroll
+    for (int seg = 0; seg < kBp1Segs; ++seg) // all loads in flight before the first store
+        v[seg] = seg < b.nseg && blk < bp1_live(b, seg) ? b.cnt[(size_t)seg * 256 * b.nblk + i] : 0;
+#pragma unroll
+    for (int seg = 0; seg < kBp1Segs; ++seg) {
+        if (seg < b.nseg && blk < bp1_live(b, seg)) b.cnt[(size_t)seg * 256 * b.nblk + i] = run;
+        run += v[seg];
+    }
+    int tot;
+    const int off = block_excl_scan(run, tot, s_tmp);
+    b.row[i] = off;
+    if (threadIdx.x == 0) b.sum[blk] = tot;
+}
+
+// Pairs are written only when all of them fit in cap; *total is the count either way.
+__global__ __launch_bounds__(128) void k_bp1_write(const float4 *__restrict__ fat, const int *__restrict__ moved, int n,
+                                                   Bp1 b, int2 *__restrict__ out, int cap, int *__restrict__ total) {
+    const int lane = threadIdx.x & 63;
+    int blk, seg;
+    bp1_cell(b, blockIdx.x, blk, seg);
+    long long before = 0, all = 0;
+    for (int k = lane; k < b.nblk; k += 64) {
+        const int v = b.sum[k];
+        all += v;
+        if (k < blk) before += v;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        all += __shfl_xor(all, o, 64);
+        before += __shfl_xor(before, o, 64);
+    }
+    if (blk == 0 && seg == 0 && threadIdx.x == 0) *total = all < INT_MAX ? (int)all : INT_MAX;
+    if (all > cap || b.nblk == 0) return;
+    const int tile = 2 * blk + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r0 = 128 * tile;
+    const size_t t = (size_t)seg * 2 * b.nblk + tile;
+    const int nh = __builtin_amdgcn_readfirstlane(b.nhit[t]);
+    const int *place = b.cnt + (size_t)seg * 256 * b.nblk; // of a row's first hit in this segment, after row[]
+    if (nh <= kBp1Hits) {
+        if (lane < nh) {
+            const uint2 h = b.hits[t * kBp1Hits + lane];
+            const int i = r0 + (int)(h.x & 127u);
+            out[before + b.row[i] + place[i] + (int)(h.x >> 7)] = make_int2(i, (int)h.y);
+        }
+        return;
+    }
+    int2 *at[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) at[u] = out + before + b.row[r0 + 64 * u + lane] + place[r0 + 64 * u + lane];
+    bp1_tests(fat, moved, n, r0, b.S * seg, min(b.S * (seg + 1), n), [&](int u, unsigned long long rows, int j) {
+        if ((rows >> lane) & 1ull) *at[u]++ = make_int2(r0 + 64 * u + lane, j);
+    });
+}
+
+// ---------------------------------------------------------------------------
 // Stand-alone kernels used by the tests.
 // ---------------------------------------------------------------------------
-__global__ void k_bp_single(const float4 *fat, const int *moved, int n, char *scratch, int2 *out, int cap, int *total) {
-    __shared__ int s_tmp[kMaxBlock / 64 + 1];
-    int t = bp_pairs(fat, moved, n, bp_carve(scratch, n), out, cap, nullptr, 0, s_tmp);
-    if (threadIdx.x == 0) *total = t;
-}
 
 __global__ void k_collide_pairs(const Shape *sa, const float *xa, const Shape *sb, const float *xb, int n, float *out) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -5293,9 +5487,22 @@ hipError_t launch_refit(const Dev &d, int w, hipStream_t s) {
     hipLaunchKernelGGL(k_refit, dim3(1), dim3(256), 0, s, d, w);
     return hipGetLastError();
 }
+size_t bp_single_scratch_bytes(int n) {
+    size_t bytes = 0;
+    (void)bp1_carve(nullptr, n, bytes);
+    return bytes;
+}
 hipError_t launch_bp_single(const float4 *fat, const int *moved, int n, char *scratch, int2 *out, int cap, int *total,
                             hipStream_t s) {
-    hipLaunchKernelGGL(k_bp_single, dim3(1), dim3(256), 0, s, fat, moved, n, scratch, out, cap, total);
+    size_t bytes = 0;
+    const Bp1 b = bp1_carve(scratch, n, bytes);
+    int cells = 0;
+    for (int seg = 0; seg < b.nseg; ++seg) cells += bp1_live(b, seg);
+    if (n > 0) {
+        hipLaunchKernelGGL(k_bp1_count, dim3(cells), dim3(128), 0, s, fat, moved, n, b);
+        hipLaunchKernelGGL(k_bp1_scan, dim3(b.nblk), dim3(256), 0, s, b);
+    }
+    hipLaunchKernelGGL(k_bp1_write, dim3(cells > 0 ? cells : 1), dim3(128), 0, s, fat, moved, n, b, out, cap, total);
     return hipGetLastError();
 }
 hipError_t launch_collide_pairs(const Shape *sa, const float *xa, const Shape *sb, const float *xb, int n, float *out,

@@ -27,14 +27,13 @@ using namespace dbx;
 
 // ---------------------------------------------------------------------------
 // Scratch of dbx_broadphase_pairs_noalloc: a fixed device array (each GPU holds
-// its own copy until the process ends), big enough for the sort-and-sweep of
-// DBX_NOALLOC_MAX_PROXIES proxies (keys 8 B per slot of the power of two above
-// the proxy count, fat AABB copy 16 B, three int arrays 12 B per proxy).  Host
-// code never passes `scratch` itself to a kernel: its device address on the
+// its own copy until the process ends), big enough for the counts and kept hits of
+// DBX_NOALLOC_MAX_PROXIES proxies (bp_single_scratch_bytes, checked on every call).
+// Host code never passes `scratch` itself to a kernel: its device address on the
 // current GPU comes from hipGetSymbolAddress, looked up once per device when a
 // handle is created there.
 // ---------------------------------------------------------------------------
-constexpr size_t kNoAllocScratchBytes = 36u * (size_t)DBX_NOALLOC_MAX_PROXIES;
+constexpr size_t kNoAllocScratchBytes = 528u * (size_t)DBX_NOALLOC_MAX_PROXIES;
 static __device__ __align__(256) char scratch[kNoAllocScratchBytes];
 
 namespace {
@@ -2159,7 +2158,7 @@ dbx_status dbx_broadphase_pairs(dbx_handle *h, const float *fat_aabbs, const uin
     size_t m = (size_t)std::max(1, n);
     hipError_t e = hipMalloc(&dfat, m * sizeof(float4));
     if (e == hipSuccess) e = hipMalloc(&dmv, m * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&dcnt, broadphase_scratch_bytes(std::max(1, n)));
+    if (e == hipSuccess) e = hipMalloc(&dcnt, bp_single_scratch_bytes(std::max(1, n)));
     if (e == hipSuccess) e = hipMalloc(&dtot, sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&dout, (size_t)std::max(1, cap) * sizeof(int2));
     if (e == hipSuccess && n) e = hipMemcpy(dfat, fat_aabbs, n * sizeof(float4), hipMemcpyHostToDevice);
@@ -2187,7 +2186,7 @@ dbx_status dbx_broadphase_pairs_noalloc(dbx_handle *h, const float *fat_aabbs, c
         return fail(h, DBX_E_INVALID_ARG, "bad broadphase arguments");
     if (((uintptr_t)fat_aabbs & 15) || ((uintptr_t)pairs & 7) || ((uintptr_t)moved & 3) || ((uintptr_t)count & 3))
         return fail(h, DBX_E_INVALID_ARG, "misaligned device pointer (fat AABBs need 16 bytes, pairs 8, ints 4)");
-    if (n > DBX_NOALLOC_MAX_PROXIES || broadphase_scratch_bytes(n) > kNoAllocScratchBytes)
+    if (n > DBX_NOALLOC_MAX_PROXIES || bp_single_scratch_bytes(n) > kNoAllocScratchBytes)
         return fail(h, DBX_E_CAPACITY, "more proxies than the fixed scratch holds (DBX_NOALLOC_MAX_PROXIES)");
     if (!h->noallocScratch) return fail(h, DBX_E_HIP, "no device address for the fixed scratch on this GPU");
     DBX_HIP(h, hipSetDevice(h->cfg.device));
