@@ -70,7 +70,6 @@ size_t wide_scratch_bytes(const WideBp &b);
 void wide_carve(WideBp &b, char *p);
 hipError_t launch_broadphase(const Dev &d, int cur, int worldOffset, int nworlds, int ldsBytes, int block, bool lead,
                              hipStream_t s, const WideBp *wide = nullptr, int nwide = 0);
-hipError_t launch_refit(const Dev &d, int world, hipStream_t s);
 // b2World.SolveTOI (continuous physics) after the step's broadphase.
 hipError_t launch_toi(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, bool lead,
                       hipStream_t s, const WideBp *wide, int nwide);
@@ -81,5 +80,53 @@ hipError_t launch_bp_single(const float4 *fat, const int *moved, int n, char *sc
 hipError_t launch_collide_pairs(const Shape *sa, const float *xa, const Shape *sb, const float *xb, int n, float *out,
                                 hipStream_t s);
 hipError_t launch_max_penetration(const Dev &d, int cur, float *out, hipStream_t s);
+
+// Read-backs and body writes through pinned host memory that the kernels write and
+// read themselves.  Each launch ends by storing `seq` to *flag (host memory) once all
+// its data are there; count: a zeroed device word of the handle.
+struct HostSignal {
+    unsigned *flag;
+    unsigned *count;
+    unsigned seq;
+};
+// dbx_body_state records of the bodies [base, base + n)
+hipError_t launch_read_bodies(const Dev &d, int base, int n, void *out, HostSignal sig, hipStream_t s);
+// *head = the world's contact count; its dbx_contact records, newest first, when
+// they fit in outBytes.  rows: an estimate of the count, for the launch's size only
+hipError_t launch_read_contacts(const Dev &d, int buf, int w, int rows, int *head, void *out, size_t outBytes,
+                                HostSignal sig, hipStream_t s);
+// What dbx_read_events assembles its list from, one after the other behind the
+// world's state in *head: the list Collide walked, the same before Collide (pre, or
+// null), each solved constraint's contact slot, its contact (zero flags for a slot out
+// of range), the continuous pass's log (log 0: none).  Written when they fit in outBytes.
+struct EventRead {
+    int walkedBuf, nowBuf, w;
+    const Contact *pre;
+    int solved, log; // whether constraints were solved and whether the pass's log is valid
+};
+__host__ __device__ inline void event_sizes(const EventRead &r, const WorldState &S, int logCap, int &walked, int &solved,
+                                            int &log) {
+    walked = S.collideCount;
+    solved = r.solved ? S.constraints : 0;
+    log = r.log ? (S.toiCallbacks < logCap ? S.toiCallbacks : logCap) : 0;
+}
+__host__ __device__ inline size_t event_words(const EventRead &r, int walked, int solved, int log) {
+    return 20 * (size_t)walked * (r.pre ? 2 : 1) + 21 * (size_t)solved + 8 * (size_t)log;
+}
+hipError_t launch_read_events(const Dev &d, const EventRead &r, int rows, WorldState *head, void *out, size_t outBytes,
+                              HostSignal sig, hipStream_t s);
+// What dbx_sync looks at: the phase-stamp counter, the first world with an error and
+// its error word, then the stamps of the steps seen .. seen + steps - 1 (the last
+// kProfSlots of them)
+struct SyncHead {
+    unsigned long long profCount;
+    int errorWorld, error; // -1: none
+};
+hipError_t launch_read_sync(const Dev &d, unsigned long long seen, int steps, SyncHead *head, unsigned long long *stamps,
+                            HostSignal sig, hipStream_t s);
+// dbx_write_bodies from n dbx_body_state records (and force / torque triples, or
+// null) in pinned memory, with the fixtures' refit
+hipError_t launch_write_bodies(const Dev &d, int w, int bodies, int fixtures, const void *in, const float *force3,
+                               hipStream_t s);
 
 } // namespace dbx

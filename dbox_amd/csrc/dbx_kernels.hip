@@ -5466,27 +5466,196 @@ hipError_t launch_broadphase(const Dev &d, int cur, int worldOffset, int nworlds
     DBX_LAUNCH(k_broadphase, lead, dim3(nworlds), dim3(block), ldsBytes, s, d, cur, worldOffset, ldsBytes);
     return hipGetLastError();
 }
-// b2Body.SetTransform's b2Fixture.Synchronize(xf, xf) (b2body.d:430-454,
-// b2fixture.d:480-502): after the host rewrote body poses, every fixture whose
-// fat AABB no longer contains its tight AABB gets a new fat AABB (no
-// displacement term) and enters the move buffer.
-__global__ void k_refit(Dev d, int w) {
+// ---------------------------------------------------------------------------
+// Read-backs and body writes.  One launch per call packs what the call returns into
+// the records of the C ABI and stores them straight into pinned host memory, where
+// the host finds them without a copy: six or more hipMemcpy calls of 10-15 us each
+// were the whole cost of a small world's read.  Bound by the launch and the host
+// link's latency below about 100 KB, by its bandwidth above.  A world of two bodies,
+// before and after: dbx_sync 42 and 9 us, bodies 73 and 12, contacts 39 (count, then
+// rows) and 11, events 74 and 12, dbx_write_bodies 88 and 8 (no longer waited for).
+// ---------------------------------------------------------------------------
+// Ends a kernel that wrote host memory: after the last workgroup's data have left,
+// the sequence number goes to the host's flag.
+__device__ __forceinline__ void host_signal(const HostSignal &sig) {
+    __builtin_amdgcn_s_waitcnt(0); // this wave's stores are done
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    __threadfence_system();
+    if (atomicAdd(sig.count, 1u) + 1 != gridDim.x) return;
+    *sig.count = 0;
+    __threadfence_system();
+    __hip_atomic_store(sig.flag, sig.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// Workgroups of 256 threads for n threads' worth of work, at most `most`.
+static unsigned read_grid(size_t n, unsigned most) {
+    const size_t g = (n + 255) / 256;
+    return g < 1 ? 1u : (g < most ? (unsigned)g : most);
+}
+
+// Four threads per body, one per 16 bytes of its record.
+__global__ __launch_bounds__(256) void k_read_bodies(Dev d, int base, int n, float4 *out, HostSignal sig) {
+    for (size_t t = blockIdx.x * 256 + threadIdx.x; t < 4 * (size_t)n; t += gridDim.x * 256) {
+        const int b = base + (int)(t >> 2), part = (int)(t & 3);
+        float4 v;
+        if (part == 0) v = d.bxf[b];
+        else if (part == 1) v = d.bpos[b];
+        else if (part == 2) {
+            v = d.bvel[b];
+            v.w = __uint_as_float(d.bflags[b] & 0xffffu);
+        } else {
+            v = d.bpos0[b];
+            v.w = d.bmass[b].x;
+        }
+        out[t] = v;
+    }
+    host_signal(sig);
+}
+
+// A thread per word; the table gives each dbx_contact word its place in Contact.
+static __constant__ unsigned char kContactWord[21] = {0,  1,  2,  3,  3,  8,  9,  10, 11, 12, 13,
+                                                      16, 17, 14, 18, 15, 19, 6,  7,  4,  5};
+__global__ __launch_bounds__(256) void k_read_contacts(Dev d, int buf, int w, int *head, unsigned *out, size_t outBytes,
+                                                       HostSignal sig) {
+    const int n = d.S[w].contactCount;
+    const unsigned *c = reinterpret_cast<const unsigned *>(d.cont[buf] + d.W[w].contactBase);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *head = n;
+    if (84 * (size_t)n <= outBytes)
+        for (size_t t = blockIdx.x * 256 + threadIdx.x; t < 21 * (size_t)n; t += gridDim.x * 256) {
+            const int k = (int)(t / 21), f = (int)(t % 21);
+            unsigned v = c[20 * (size_t)(n - 1 - k) + kContactWord[f]];
+            if (f == 2) v &= kContactTouching | kContactEnabled;
+            if (f == 3) v &= 0xfu;
+            if (f == 4) v = (v >> 4) & 0xfu;
+            out[t] = v;
+        }
+    host_signal(sig);
+}
+
+__global__ __launch_bounds__(256) void k_read_events(Dev d, EventRead r, WorldState *head, unsigned *out, size_t outBytes,
+                                                     HostSignal sig) {
+    const WorldDesc wd = d.W[r.w];
+    const WorldState S = d.S[r.w];
+    const int logCap = d.toiLogOff[r.w + 1] - d.toiLogOff[r.w];
+    int walked, solved, log;
+    event_sizes(r, S, logCap, walked, solved, log);
+    const int tid = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
+    if (tid < (int)(sizeof(WorldState) / 4))
+        reinterpret_cast<int *>(head)[tid] = reinterpret_cast<const int *>(d.S + r.w)[tid];
+    if (4 * event_words(r, walked, solved, log) <= outBytes) {
+        auto words = [&](const void *src, size_t n) {
+            const unsigned *p = static_cast<const unsigned *>(src);
+            for (size_t t = tid; t < n; t += step) out[t] = p[t];
+            out += n;
+        };
+        words(d.cont[r.walkedBuf] + wd.contactBase, 20 * (size_t)walked);
+        if (r.pre) words(r.pre + wd.contactBase, 20 * (size_t)walked);
+        const int *ord = d.ordC + wd.contactBase;
+        words(ord, solved);
+        const unsigned *now = reinterpret_cast<const unsigned *>(d.cont[r.nowBuf] + wd.contactBase);
+        for (size_t t = tid; t < 20 * (size_t)solved; t += step) {
+            const int c = ord[t / 20];
+            out[t] = c >= 0 && c < S.contactCount ? now[20 * (size_t)c + t % 20] : 0u;
+        }
+        out += 20 * (size_t)solved;
+        words(d.toiLog + d.toiLogOff[r.w], 8 * (size_t)log);
+    }
+    host_signal(sig);
+}
+
+__global__ __launch_bounds__(1024) void k_read_sync(Dev d, unsigned long long seen, int steps, SyncHead *head,
+                                                    unsigned long long *stamps, HostSignal sig) {
+    __shared__ int s_world;
+    if (threadIdx.x == 0) s_world = INT_MAX;
+    __syncthreads();
+    int first = INT_MAX;
+    for (int w = threadIdx.x; w < d.nworlds; w += 1024)
+        if (d.S[w].error) {
+            first = w;
+            break;
+        }
+    if (first != INT_MAX) atomicMin(&s_world, first);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        head->profCount = d.prof[0];
+        head->errorWorld = s_world == INT_MAX ? -1 : s_world;
+        head->error = s_world == INT_MAX ? 0 : d.S[s_world].error;
+    }
+    const int from = steps > kProfSlots ? steps - kProfSlots : 0;
+    for (int t = threadIdx.x; t < kProfStamps * (steps - from); t += 1024) {
+        const unsigned long long slot = seen + (unsigned)(from + t / kProfStamps);
+        stamps[t] = d.prof[kProfStamps * (slot % kProfSlots + 1) + t % kProfStamps];
+    }
+    host_signal(sig);
+}
+
+// A body's record and a fixture's refit per thread.  The refit is b2Body.
+// SetTransform's b2Fixture.Synchronize(xf, xf) (b2body.d:430-454, b2fixture.d:
+// 480-502): a fixture whose fat AABB no longer contains its tight AABB gets a new fat
+// AABB (no displacement term) and enters the move buffer; it takes the transform
+// from the record, so it need not wait for the body's stores.
+__global__ __launch_bounds__(256) void k_write_bodies(Dev d, int w, const float4 *__restrict__ in,
+                                                      const float *__restrict__ force3) {
     const WorldDesc wd = d.W[w];
-    for (int f = threadIdx.x; f < wd.fixCount; f += blockDim.x) {
-        const int b = d.fbody[wd.fixBase + f];
-        const Xf x = load_xf(d.bxf + wd.bodyBase, b);
-        const float4 aabb = shape_aabb(d.fshape + wd.fixBase + f, x);
-        const float4 fa = d.ffat[wd.fixBase + f];
+    const int step = gridDim.x * 256;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < wd.bodyCount; i += step) {
+        const int b = wd.bodyBase + i;
+        const float4 xf = in[4 * (size_t)i], pos = in[4 * (size_t)i + 1], vel = in[4 * (size_t)i + 2],
+                     p0 = in[4 * (size_t)i + 3];
+        d.bxf[b] = xf;
+        d.bpos[b] = pos;
+        d.bvel[b] = make_float4(vel.x, vel.y, vel.z, 0.0f);
+        d.bpos0[b] = make_float4(p0.x, p0.y, p0.z, 0.0f);
+        d.bflags[b] = (d.bflags[b] & ~(uint32_t)kBodyAwake) | (__float_as_uint(vel.w) & kBodyAwake);
+        if (force3)
+            d.bforce[b] =
+                make_float4(force3[3 * (size_t)i], force3[3 * (size_t)i + 1], force3[3 * (size_t)i + 2], 0.0f);
+    }
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < wd.fixCount; i += step) {
+        const int f = wd.fixBase + i;
+        const float4 t = in[4 * (size_t)d.fbody[f]];
+        Xf x;
+        x.p = v2(t.x, t.y);
+        x.q.s = t.z;
+        x.q.c = t.w;
+        const float4 aabb = shape_aabb(d.fshape + f, x);
+        const float4 fa = d.ffat[f];
         if (fa.x <= aabb.x && fa.y <= aabb.y && aabb.z <= fa.z && aabb.w <= fa.w) continue;
-        d.ffat[wd.fixBase + f] = make_float4(aabb.x - kAabbExtension, aabb.y - kAabbExtension, aabb.z + kAabbExtension,
-                                             aabb.w + kAabbExtension);
-        d.fmoved[wd.fixBase + f] = 1;
+        d.ffat[f] = make_float4(aabb.x - kAabbExtension, aabb.y - kAabbExtension, aabb.z + kAabbExtension,
+                                aabb.w + kAabbExtension);
+        d.fmoved[f] = 1;
     }
 }
-hipError_t launch_refit(const Dev &d, int w, hipStream_t s) {
-    hipLaunchKernelGGL(k_refit, dim3(1), dim3(256), 0, s, d, w);
+
+hipError_t launch_read_bodies(const Dev &d, int base, int n, void *out, HostSignal sig, hipStream_t s) {
+    hipLaunchKernelGGL(k_read_bodies, dim3(read_grid(4 * (size_t)n, 512)), dim3(256), 0, s, d, base, n, (float4 *)out,
+                       sig);
     return hipGetLastError();
 }
+hipError_t launch_read_contacts(const Dev &d, int buf, int w, int rows, int *head, void *out, size_t outBytes,
+                                HostSignal sig, hipStream_t s) {
+    hipLaunchKernelGGL(k_read_contacts, dim3(read_grid(21 * (size_t)rows, 512)), dim3(256), 0, s, d, buf, w, head,
+                       (unsigned *)out, outBytes, sig);
+    return hipGetLastError();
+}
+hipError_t launch_read_events(const Dev &d, const EventRead &r, int rows, WorldState *head, void *out, size_t outBytes,
+                              HostSignal sig, hipStream_t s) {
+    hipLaunchKernelGGL(k_read_events, dim3(read_grid(20 * (size_t)rows, 512)), dim3(256), 0, s, d, r, head,
+                       (unsigned *)out, outBytes, sig);
+    return hipGetLastError();
+}
+hipError_t launch_read_sync(const Dev &d, unsigned long long seen, int steps, SyncHead *head, unsigned long long *stamps,
+                            HostSignal sig, hipStream_t s) {
+    hipLaunchKernelGGL(k_read_sync, dim3(1), dim3(1024), 0, s, d, seen, steps, head, stamps, sig);
+    return hipGetLastError();
+}
+hipError_t launch_write_bodies(const Dev &d, int w, int bodies, int fixtures, const void *in, const float *force3,
+                               hipStream_t s) {
+    hipLaunchKernelGGL(k_write_bodies, dim3(read_grid(bodies > fixtures ? bodies : fixtures, 512)), dim3(256), 0, s, d, w,
+                       (const float4 *)in, force3);
+    return hipGetLastError();
+}
+
 size_t bp_single_scratch_bytes(int n) {
     size_t bytes = 0;
     (void)bp1_carve(nullptr, n, bytes);

@@ -695,6 +695,15 @@ struct dbx_handle {
     void *noallocScratch = nullptr; // device address of `scratch` on this handle's GPU
     std::vector<char> ringSolved;   // per ring entry: the step ran the island solve (dt > 0)
     unsigned long long profSeen = 0; // phase-stamp slots of the solve kernels already read
+    // pinned host memory that kernels write read-backs into (read) and take body writes
+    // from (write, filled from writeAt on since the stream was last known to be idle)
+    struct Pinned {
+        char *host = nullptr, *dev = nullptr;
+        size_t bytes = 0;
+    } read, write;
+    size_t writeAt = 0;
+    unsigned *signalHost = nullptr, *signalDev = nullptr, *signalCount = nullptr; // HostSignal's words
+    unsigned signalSeq = 0;
     double wallKHz = 100000.0;      // rate of the kernels' wall_clock64 stamps
     int cuCount = 0;                // compute units of the device
     bool leadCus = false;           // the lead tier runs on CUs of its own (CU-masked streams)
@@ -740,6 +749,55 @@ template <class T>
 hipError_t upload(dbx_handle *h, T *dst, const std::vector<T> &src) {
     if (src.empty()) return hipSuccess;
     return hipMemcpyAsync(dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice, h->stream);
+}
+
+hipError_t pinned_alloc(void **host, void **dev, size_t bytes) {
+    hipError_t e = hipHostMalloc(host, bytes, hipHostMallocMapped | hipHostMallocCoherent);
+    if (e == hipSuccess) e = hipHostGetDevicePointer(dev, *host, 0);
+    return e;
+}
+// At least `bytes` of p, which no launched kernel uses any more when this returns.
+hipError_t pinned_reserve(dbx_handle *h, dbx_handle::Pinned &p, size_t bytes) {
+    if (p.bytes >= bytes) return hipSuccess;
+    hipError_t e = hipStreamSynchronize(h->stream);
+    if (e != hipSuccess) return e;
+    if (p.host) (void)hipHostFree(p.host);
+    p = dbx_handle::Pinned{};
+    const size_t n = std::max<size_t>((bytes + bytes / 2 + 4095) & ~(size_t)4095, 1u << 18);
+    e = pinned_alloc((void **)&p.host, (void **)&p.dev, n);
+    if (e == hipSuccess) p.bytes = n;
+    return e;
+}
+// Runs launch(signal), a kernel that fills h->read (reserved to `bytes`) and signals,
+// and waits for it, which everything before it on the stream has finished by then.
+// The host looks at the signal itself for a while, which sees a short step's end some
+// microseconds sooner than a stream synchronisation; a long step, or one that
+// failed and never signals, is waited for by the synchronisation.
+template <class F>
+dbx_status pinned_read(dbx_handle *h, size_t bytes, F &&launch) {
+    DBX_HIP(h, hipSetDevice(h->cfg.device));
+    if (!h->signalCount) {
+        if (!h->signalHost) {
+            DBX_HIP(h, pinned_alloc((void **)&h->signalHost, (void **)&h->signalDev, 64));
+            *h->signalHost = 0;
+        }
+        DBX_HIP(h, dalloc(h, &h->signalCount, 1));
+    }
+    DBX_HIP(h, pinned_reserve(h, h->read, bytes));
+    const unsigned seq = ++h->signalSeq;
+    DBX_HIP(h, launch(HostSignal{h->signalDev, h->signalCount, seq}));
+    constexpr int kSpins = 4000; // about 0.2 ms
+    for (int i = 0; i < kSpins; ++i) {
+        if (__atomic_load_n(h->signalHost, __ATOMIC_ACQUIRE) == seq) {
+            h->writeAt = 0;
+            return DBX_OK;
+        }
+        __builtin_ia32_pause();
+    }
+    DBX_HIP(h, hipStreamSynchronize(h->stream));
+    h->writeAt = 0;
+    if (__atomic_load_n(h->signalHost, __ATOMIC_ACQUIRE) != seq) return fail(h, DBX_E_HIP, "a read-back kernel did not finish");
+    return DBX_OK;
 }
 
 } // namespace
@@ -802,6 +860,8 @@ void dbx_destroy(dbx_handle *h) {
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     mlp_release(h->mlp);
     for (void *p : h->allocs) (void)hipFree(p);
+    for (void *p : {(void *)h->read.host, (void *)h->write.host, (void *)h->signalHost})
+        if (p) (void)hipHostFree(p);
     for (auto &e : h->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto &e : h->ring) (void)hipEventDestroy(e);
@@ -1579,29 +1639,35 @@ dbx_status dbx_write_contact_settings(dbx_handle *h, int32_t world, const dbx_co
 dbx_status dbx_sync(dbx_handle *h) {
     if (!h) return DBX_E_INVALID_ARG;
     DBX_HIP(h, hipSetDevice(h->cfg.device));
-    DBX_HIP(h, hipStreamSynchronize(h->stream));
-    if (!h->finalized) return DBX_OK;
-    std::vector<WorldState> S(h->nworlds);
-    DBX_HIP(h, hipMemcpy(S.data(), h->d.S, h->nworlds * sizeof(WorldState), hipMemcpyDeviceToHost));
-    for (int w = 0; w < h->nworlds; ++w) {
-        if (S[w].error) {
-            // bit 1: contact slots; bit 2: the step's broadphase pair list; bit 4: the
-            // continuous pass's per-event lists (pairs of the moved proxies, moved proxies)
-            char buf[160];
-            const int e = S[w].error;
-            snprintf(buf, sizeof buf, "world %d exceeded its %s capacity", w,
-                     (e & 1) ? "contact" : (e & 2) ? "broadphase pair" : "continuous-pass pair/moved-proxy list");
-            return fail(h, DBX_E_CAPACITY, buf);
-        }
+    if (!h->finalized) {
+        DBX_HIP(h, hipStreamSynchronize(h->stream));
+        return DBX_OK;
+    }
+    int solvedSteps = 0;
+    for (int k = 0; k < h->ringUsed; ++k) solvedSteps += h->ringSolved[k] ? 1 : 0;
+    const int kept = std::min(solvedSteps, kProfSlots);
+    dbx_status rs = pinned_read(h, 64 + (size_t)kProfStamps * sizeof(unsigned long long) * kept, [&](HostSignal sig) {
+        return launch_read_sync(h->d, h->profSeen, solvedSteps, (SyncHead *)h->read.dev,
+                                (unsigned long long *)(h->read.dev + 64), sig, h->stream);
+    });
+    if (rs != DBX_OK) return rs;
+    const SyncHead head = *(const SyncHead *)h->read.host;
+    if (head.errorWorld >= 0) {
+        // bit 1: contact slots; bit 2: the step's broadphase pair list; bit 4: the
+        // continuous pass's per-event lists (pairs of the moved proxies, moved proxies)
+        char buf[160];
+        const int e = head.error;
+        snprintf(buf, sizeof buf, "world %d exceeded its %s capacity", head.errorWorld,
+                 (e & 1) ? "contact" : (e & 2) ? "broadphase pair" : "continuous-pass pair/moved-proxy list");
+        return fail(h, DBX_E_CAPACITY, buf);
     }
     // b2Profile's island-solve phases (b2island.d:118-237) from the stamps the largest
     // world's solve left: one slot per step that ran the solve, in step order.
-    std::vector<unsigned long long> stamps((size_t)kProfStamps * (kProfSlots + 1));
-    DBX_HIP(h, hipMemcpy(stamps.data(), h->d.prof, stamps.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-    const unsigned long long profCount = stamps[0];
-    int solvedSteps = 0;
-    for (int k = 0; k < h->ringUsed; ++k) solvedSteps += h->ringSolved[k] ? 1 : 0;
+    const unsigned long long *stamps = (const unsigned long long *)(h->read.host + 64);
+    const unsigned long long profCount = head.profCount, firstKept = h->profSeen + (solvedSteps - kept);
     const bool stampsMatch = profCount - h->profSeen == (unsigned long long)solvedSteps;
+    if (h->ringUsed > 0) // its timing is read below
+        DBX_HIP(h, hipEventSynchronize(h->ring[kStepEvents * h->ringUsed - 1]));
     unsigned long long nextSlot = h->profSeen;
     h->profSeen = profCount;
     for (int k = 0; k < h->ringUsed; ++k) {
@@ -1610,8 +1676,8 @@ dbx_status dbx_sync(dbx_handle *h) {
         float phase[3] = {0, 0, 0};
         if (h->ringSolved[k]) {
             const unsigned long long slot = nextSlot++;
-            if (stampsMatch && profCount - slot <= (unsigned long long)kProfSlots) {
-                const unsigned long long *t = &stamps[(size_t)kProfStamps * (slot % kProfSlots + 1)];
+            if (stampsMatch && slot >= firstKept) {
+                const unsigned long long *t = stamps + kProfStamps * (slot - firstKept);
                 const double perMs = h->wallKHz;
                 phase[0] = (float)((double)(t[kProfVel0] - t[kProfInit0]) / perMs);
                 phase[1] = (float)((double)(t[kProfVel1] - t[kProfVel0]) / perMs);
@@ -1732,76 +1798,46 @@ dbx_status dbx_read_bodies(dbx_handle *h, int32_t world, dbx_body_state *out, in
     if (st) return st;
     const WorldDesc &D = h->W[world];
     if (!out || n < D.bodyCount) return fail(h, DBX_E_INVALID_ARG, "output too small");
-    int nb = D.bodyCount, b0 = D.bodyBase;
-    std::vector<uint32_t> fl(nb);
-    std::vector<float4> xf(nb), pos(nb), pos0(nb), vel(nb), ms(nb);
-    DBX_HIP(h, hipStreamSynchronize(h->stream));
-    DBX_HIP(h, hipMemcpy(fl.data(), h->d.bflags + b0, nb * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    DBX_HIP(h, hipMemcpy(xf.data(), h->d.bxf + b0, nb * sizeof(float4), hipMemcpyDeviceToHost));
-    DBX_HIP(h, hipMemcpy(pos.data(), h->d.bpos + b0, nb * sizeof(float4), hipMemcpyDeviceToHost));
-    DBX_HIP(h, hipMemcpy(pos0.data(), h->d.bpos0 + b0, nb * sizeof(float4), hipMemcpyDeviceToHost));
-    DBX_HIP(h, hipMemcpy(vel.data(), h->d.bvel + b0, nb * sizeof(float4), hipMemcpyDeviceToHost));
-    DBX_HIP(h, hipMemcpy(ms.data(), h->d.bmass + b0, nb * sizeof(float4), hipMemcpyDeviceToHost));
-    for (int i = 0; i < nb; ++i) {
-        dbx_body_state &s = out[i];
-        s.px = xf[i].x;
-        s.py = xf[i].y;
-        s.qs = xf[i].z;
-        s.qc = xf[i].w;
-        s.cx = pos[i].x;
-        s.cy = pos[i].y;
-        s.a = pos[i].z;
-        s.sleep_time = pos[i].w;
-        s.vx = vel[i].x;
-        s.vy = vel[i].y;
-        s.w = vel[i].z;
-        s.flags = (int32_t)(fl[i] & 0xffffu);
-        s.c0x = pos0[i].x;
-        s.c0y = pos0[i].y;
-        s.a0 = pos0[i].z;
-        s.inv_mass = ms[i].x;
-    }
-    return DBX_OK;
+    static_assert(sizeof(dbx_body_state) == 64, "k_read_bodies writes four float4 per body");
+    const size_t bytes = (size_t)D.bodyCount * sizeof(dbx_body_state);
+    st = pinned_read(h, bytes, [&](HostSignal sig) {
+        return launch_read_bodies(h->d, D.bodyBase, D.bodyCount, h->read.dev, sig, h->stream);
+    });
+    if (st == DBX_OK) memcpy(out, h->read.host, bytes);
+    return st;
 }
 
 dbx_status dbx_write_bodies(dbx_handle *h, int32_t world, const dbx_body_state *in, const float *force3, int32_t n) {
     dbx_status st = check_world(h, world);
-    if (h->splitWaiting) return fail(h, DBX_E_STATE, "a PRESOLVE step is waiting for dbx_step_finish");
     if (st) return st;
+    if (h->splitWaiting) return fail(h, DBX_E_STATE, "a PRESOLVE step is waiting for dbx_step_finish");
     const WorldDesc &D = h->W[world];
     if (!in || n != D.bodyCount) return fail(h, DBX_E_INVALID_ARG, "one state per body is required");
-    const int nb = D.bodyCount, b0 = D.bodyBase;
-    std::vector<uint32_t> fl(nb);
-    std::vector<float4> xf(nb), pos(nb), pos0(nb), vel(nb), frc;
-    DBX_HIP(h, hipStreamSynchronize(h->stream));
-    DBX_HIP(h, hipMemcpy(fl.data(), h->d.bflags + b0, nb * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    const int nb = D.bodyCount;
     for (int i = 0; i < nb; ++i) {
         const dbx_body_state &s = in[i];
         const float v[] = {s.px, s.py, s.qs, s.qc, s.cx, s.cy, s.a, s.sleep_time, s.vx, s.vy, s.w, s.c0x, s.c0y, s.a0};
         for (float x : v)
             if (!std::isfinite(x)) return fail(h, DBX_E_INVALID_ARG, "body state is not finite");
-        xf[i] = make_float4(s.px, s.py, s.qs, s.qc);
-        pos[i] = make_float4(s.cx, s.cy, s.a, s.sleep_time);
-        pos0[i] = make_float4(s.c0x, s.c0y, s.a0, 0.0f);
-        vel[i] = make_float4(s.vx, s.vy, s.w, 0.0f);
-        fl[i] = (fl[i] & ~(uint32_t)kBodyAwake) | ((uint32_t)s.flags & kBodyAwake);
     }
-    if (force3) {
-        frc.resize(nb);
-        for (int i = 0; i < nb; ++i) {
-            if (!std::isfinite(force3[3 * i]) || !std::isfinite(force3[3 * i + 1]) || !std::isfinite(force3[3 * i + 2]))
-                return fail(h, DBX_E_INVALID_ARG, "force is not finite");
-            frc[i] = make_float4(force3[3 * i], force3[3 * i + 1], force3[3 * i + 2], 0.0f);
-        }
+    for (int i = 0; force3 && i < 3 * nb; ++i)
+        if (!std::isfinite(force3[i])) return fail(h, DBX_E_INVALID_ARG, "force is not finite");
+    // The records go to pinned memory and are applied by a kernel on the handle's
+    // stream, before anything launched after this call.
+    DBX_HIP(h, hipSetDevice(h->cfg.device));
+    const size_t bodyBytes = (size_t)nb * sizeof(dbx_body_state);
+    const size_t bytes = bodyBytes + (force3 ? (12 * (size_t)nb + 63) / 64 * 64 : 0);
+    if (h->writeAt + bytes > h->write.bytes) {
+        DBX_HIP(h, hipStreamSynchronize(h->stream));
+        h->writeAt = 0;
+        DBX_HIP(h, pinned_reserve(h, h->write, bytes));
     }
-    DBX_HIP(h, hipMemcpy(h->d.bflags + b0, fl.data(), nb * sizeof(uint32_t), hipMemcpyHostToDevice));
-    DBX_HIP(h, hipMemcpy(h->d.bxf + b0, xf.data(), nb * sizeof(float4), hipMemcpyHostToDevice));
-    DBX_HIP(h, hipMemcpy(h->d.bpos + b0, pos.data(), nb * sizeof(float4), hipMemcpyHostToDevice));
-    DBX_HIP(h, hipMemcpy(h->d.bpos0 + b0, pos0.data(), nb * sizeof(float4), hipMemcpyHostToDevice));
-    DBX_HIP(h, hipMemcpy(h->d.bvel + b0, vel.data(), nb * sizeof(float4), hipMemcpyHostToDevice));
-    if (force3) DBX_HIP(h, hipMemcpy(h->d.bforce + b0, frc.data(), nb * sizeof(float4), hipMemcpyHostToDevice));
-    DBX_HIP(h, launch_refit(h->d, world, h->stream));
-    DBX_HIP(h, hipStreamSynchronize(h->stream));
+    char *host = h->write.host + h->writeAt, *dev = h->write.dev + h->writeAt;
+    memcpy(host, in, bodyBytes);
+    if (force3) memcpy(host + bodyBytes, force3, 12 * (size_t)nb);
+    h->writeAt += bytes;
+    DBX_HIP(h, launch_write_bodies(h->d, world, nb, D.fixCount, dev, force3 ? (const float *)(dev + bodyBytes) : nullptr,
+                                   h->stream));
     return DBX_OK;
 }
 
@@ -1810,38 +1846,45 @@ dbx_status dbx_read_events(dbx_handle *h, int32_t world, dbx_contact_event *out,
     if (st) return st;
     if (!count) return fail(h, DBX_E_INVALID_ARG, "count is required");
     const WorldDesc &D = h->W[world];
-    WorldState S;
-    DBX_HIP(h, hipStreamSynchronize(h->stream));
-    DBX_HIP(h, hipMemcpy(&S, h->d.S + world, sizeof S, hipMemcpyDeviceToHost));
     // The last step's Collide walked the list held in the other buffer, where its
     // flags stay; the solved contacts are in the current list, in island order.
     // While a PRESOLVE step waits, Collide's walked list is still the current one
-    // and nothing has been solved yet.
-    const int walkedBuf = h->splitWaiting ? h->cur : h->cur ^ 1, nowBuf = walkedBuf ^ 1;
-    const int n0 = S.collideCount, m = S.contactCount, nc = h->splitWaiting ? 0 : S.constraints;
-    std::vector<Contact> walked(n0), now(m), pre;
-    std::vector<int32_t> ord(nc);
-    if (n0) DBX_HIP(h, hipMemcpy(walked.data(), h->d.cont[walkedBuf] + D.contactBase, n0 * sizeof(Contact),
-                                 hipMemcpyDeviceToHost));
-    if (m) DBX_HIP(h, hipMemcpy(now.data(), h->d.cont[nowBuf] + D.contactBase, m * sizeof(Contact), hipMemcpyDeviceToHost));
-    if (nc) DBX_HIP(h, hipMemcpy(ord.data(), h->d.ordC + D.contactBase, nc * sizeof(int32_t), hipMemcpyDeviceToHost));
-    const bool preSolve = h->lastSplit && h->contPre;
-    if (preSolve && n0) {
-        pre.resize(n0);
-        DBX_HIP(h, hipMemcpy(pre.data(), h->contPre + D.contactBase, n0 * sizeof(Contact), hipMemcpyDeviceToHost));
+    // and nothing has been solved yet.  With them come the continuous pass's log: its
+    // callbacks, and the discrete PostSolve data of the contacts it updated
+    // (kLogSnapshot), which their slots no longer hold.
+    EventRead er{};
+    er.walkedBuf = h->splitWaiting ? h->cur : h->cur ^ 1;
+    er.nowBuf = er.walkedBuf ^ 1;
+    er.w = world;
+    er.pre = h->lastSplit && h->contPre ? h->contPre : nullptr;
+    er.solved = h->splitWaiting ? 0 : 1;
+    er.log = h->lastCcd && !h->splitWaiting ? 1 : 0;
+    const int logCap = h->toiLogOff[world + 1] - h->toiLogOff[world];
+    WorldState S;
+    int n0 = 0, nc = 0, nlog = 0;
+    for (size_t bytes = 4096;;) {
+        st = pinned_read(h, 64 + bytes, [&](HostSignal sig) {
+            return launch_read_events(h->d, er, D.contactCap / 4, (WorldState *)h->read.dev, h->read.dev + 64,
+                                      h->read.bytes - 64, sig, h->stream);
+        });
+        if (st != DBX_OK) return st;
+        static_assert(sizeof(WorldState) == 64, "the read-back's head");
+        memcpy(&S, h->read.host, sizeof S);
+        event_sizes(er, S, logCap, n0, nc, nlog);
+        bytes = 4 * event_words(er, n0, nc, nlog);
+        if (bytes <= h->read.bytes - 64) break;
     }
-    // the continuous pass's log: its callbacks, and the discrete PostSolve data of
-    // the contacts it updated (kLogSnapshot), which their slots no longer hold
-    std::vector<ToiCallback> log;
-    if (h->lastCcd && !h->splitWaiting) {
-        const int cap = h->toiLogOff[world + 1] - h->toiLogOff[world];
-        if (S.toiCallbacks > cap)
-            return fail(h, DBX_E_CAPACITY, "the continuous pass made more listener callbacks than its log holds");
-        log.resize(S.toiCallbacks);
-        if (!log.empty())
-            DBX_HIP(h, hipMemcpy(log.data(), h->d.toiLog + h->toiLogOff[world], log.size() * sizeof(ToiCallback),
-                                 hipMemcpyDeviceToHost));
-    }
+    if (er.log && S.toiCallbacks > logCap)
+        return fail(h, DBX_E_CAPACITY, "the continuous pass made more listener callbacks than its log holds");
+    const bool preSolve = er.pre != nullptr;
+    const int m = S.contactCount;
+    const Contact *walked = (const Contact *)(h->read.host + 64), *pre = preSolve ? walked + n0 : nullptr;
+    const int *ord = (const int *)(walked + (preSolve ? 2 : 1) * (size_t)n0);
+    const char *after = (const char *)(ord + nc); // only 4-byte aligned from here on
+    std::vector<Contact> solvedList(nc);
+    if (nc) memcpy(solvedList.data(), after, nc * sizeof(Contact));
+    std::vector<ToiCallback> log(nlog);
+    if (nlog) memcpy(log.data(), after + nc * sizeof(Contact), nlog * sizeof(ToiCallback));
     std::unordered_map<int, const ToiCallback *> solvedBefore;
     for (const ToiCallback &r : log)
         if (r.type == kLogSnapshot) solvedBefore.emplace(r.fa, &r);
@@ -1881,7 +1924,7 @@ dbx_status dbx_read_events(dbx_handle *h, int32_t world, dbx_contact_event *out,
     }
     for (int k = 0; k < nc; ++k) {
         if (ord[k] < 0 || ord[k] >= m) return fail(h, DBX_E_STATE, "solve order out of range");
-        const Contact &c = now[ord[k]];
+        const Contact &c = solvedList[k];
         dbx_contact_event e{};
         e.type = DBX_EVENT_POST_SOLVE;
         e.fixture_a = c.fa;
@@ -1941,41 +1984,22 @@ dbx_status dbx_read_contacts(dbx_handle *h, int32_t world, dbx_contact *out, int
     dbx_status st = check_world(h, world);
     if (st) return st;
     const WorldDesc &D = h->W[world];
-    WorldState S;
-    DBX_HIP(h, hipStreamSynchronize(h->stream));
-    DBX_HIP(h, hipMemcpy(&S, h->d.S + world, sizeof S, hipMemcpyDeviceToHost));
-    int n = S.contactCount;
-    if (count) *count = n;
-    if (!out || cap <= 0) return DBX_OK;
-    std::vector<Contact> c(n);
+    static_assert(sizeof(dbx_contact) == 84, "k_read_contacts writes 21 words per contact");
     const int buf = h->splitWaiting ? h->cur ^ 1 : h->cur; // while a PRESOLVE step waits: the list Collide left
-    if (n) DBX_HIP(h, hipMemcpy(c.data(), h->d.cont[buf] + D.contactBase, n * sizeof(Contact), hipMemcpyDeviceToHost));
-    int m = std::min(n, cap);
-    for (int k = 0; k < m; ++k) {
-        const Contact &s = c[n - 1 - k]; // list order: newest first
-        dbx_contact &o = out[k];
-        o.fixture_a = s.fa;
-        o.fixture_b = s.fb;
-        o.flags = (int32_t)(s.flags & (kContactTouching | kContactEnabled));
-        o.type = s.meta & 0xf;
-        o.point_count = (s.meta >> 4) & 0xf;
-        o.local_normal[0] = s.man.x;
-        o.local_normal[1] = s.man.y;
-        o.local_point[0] = s.man.z;
-        o.local_point[1] = s.man.w;
-        o.point_local[0] = s.pt0.x;
-        o.point_local[1] = s.pt0.y;
-        o.point_local[2] = s.pt1.x;
-        o.point_local[3] = s.pt1.y;
-        o.normal_impulse[0] = s.pt0.z;
-        o.normal_impulse[1] = s.pt1.z;
-        o.tangent_impulse[0] = s.pt0.w;
-        o.tangent_impulse[1] = s.pt1.w;
-        o.id[0] = s.id0;
-        o.id[1] = s.id1;
-        o.friction = s.friction;
-        o.restitution = s.restitution;
+    const bool rows = out && cap > 0;
+    int n = 0;
+    for (size_t bytes = rows ? 4096 : 0;;) {
+        st = pinned_read(h, 64 + bytes, [&](HostSignal sig) {
+            return launch_read_contacts(h->d, buf, world, rows ? D.contactCap / 4 : 0, (int *)h->read.dev,
+                                        h->read.dev + 64, rows ? h->read.bytes - 64 : 0, sig, h->stream);
+        });
+        if (st != DBX_OK) return st;
+        n = *(const int *)h->read.host;
+        bytes = (size_t)n * sizeof(dbx_contact);
+        if (!rows || bytes <= h->read.bytes - 64) break;
     }
+    if (count) *count = n;
+    if (rows) memcpy(out, h->read.host + 64, (size_t)std::min(n, cap) * sizeof(dbx_contact));
     return DBX_OK;
 }
 

@@ -219,23 +219,28 @@ class StepWorlds:
         return len(self.body_counts)
 
     def bodies(self, world=0) -> np.ndarray:
-        out = np.zeros(self.body_counts[world], BODY_STATE_DTYPE)
+        out = np.empty(self.body_counts[world], BODY_STATE_DTYPE)
         self._check(self.L.dbx_read_bodies(self.h, world, _p(out), len(out)))
         return out
 
     def contacts(self, world=0) -> np.ndarray:
         n = C.c_int32()
-        self._check(self.L.dbx_read_contacts(self.h, world, None, 0, C.byref(n)))
-        out = np.zeros(max(n.value, 1), CONTACT_DTYPE)
-        self._check(self.L.dbx_read_contacts(self.h, world, _p(out), n.value, C.byref(n)))
+        out = np.empty(4 * self.fixture_counts[world] + 64, CONTACT_DTYPE)  # nearly always enough: one read
+        self._check(self.L.dbx_read_contacts(self.h, world, _p(out), len(out), C.byref(n)))
+        if n.value > len(out):
+            out = np.empty(n.value, CONTACT_DTYPE)
+            self._check(self.L.dbx_read_contacts(self.h, world, _p(out), n.value, C.byref(n)))
         return out[:n.value]
 
     def events(self, world=0) -> np.ndarray:
         """The b2ContactListener callbacks of the last step (dbx_read_events), in dbox's order."""
         n = C.c_int32()
-        self._check(self.L.dbx_read_events(self.h, world, None, 0, C.byref(n)))
-        out = np.zeros(max(n.value, 1), EVENT_DTYPE)
-        self._check(self.L.dbx_read_events(self.h, world, _p(out), n.value, C.byref(n)))
+        out = np.empty(8 * self.fixture_counts[world] + 64, EVENT_DTYPE)  # nearly always enough: one read
+        st = self.L.dbx_read_events(self.h, world, _p(out), len(out), C.byref(n))
+        if st == DBX_E_CAPACITY and n.value > len(out):
+            out = np.empty(n.value, EVENT_DTYPE)
+            st = self.L.dbx_read_events(self.h, world, _p(out), n.value, C.byref(n))
+        self._check(st)
         return out[:n.value]
 
     def fat_aabbs(self, world=0) -> np.ndarray:
