@@ -1745,6 +1745,53 @@ __device__ __forceinline__ float velocity_sweep(const int *Lbo, int nbatch, cons
     return lres;
 }
 
+// velocity_sweep with the accumulated impulses in the constraint records instead of
+// LDS, for islands whose impulses do not fit there: a slot's record comes with its
+// impulses two levels ahead, and the same lane stores them back after the solve, so
+// a lane reads in one sweep what it wrote in the sweep before.
+template <int kMode>
+__device__ __forceinline__ float velocity_sweep_far(const int *Lbo, int nbatch, VelCon *vc, float4 *Lvel, int lane) {
+    float lres = 0.0f;
+    auto one = [&](const VelCon &v, int k) {
+        float4 va = Lvel[v.indexA], vb = Lvel[v.indexB], im = make_float4(v.nImp0, v.tImp0, v.nImp1, v.tImp1);
+        asm volatile("" ::"v"(va.x), "v"(vb.x));
+        if (kMode == 0) warm_start_core(v, im, va, vb);
+        else lres = fmaxr(lres, solve_velocity_core<kMode == 2>(v, im, va, vb));
+        if (kMode != 0) *reinterpret_cast<float4 *>(&vc[k].nImp0) = im;
+        Lvel[v.indexA] = va;
+        Lvel[v.indexB] = vb;
+    };
+    auto level = [&](const VelCon &v, int k, bool have, int lo, int hi) {
+        if (have) one(v, k);
+        for (int c = lo + 64; c < hi; c += 64) { // levels wider than the wave
+            const int j2 = c + (int)(threadIdx.x & 63);
+            if (j2 < hi) {
+                const VelCon v2 = vc[j2];
+                one(v2, j2);
+            }
+        }
+    };
+    LevelWindow W{Lbo, nbatch + 1, 0, 0};
+    W.load(0);
+    int k0, k1, lo0, hi0, lo1, hi1;
+    bool h0, h1;
+    level_slot(W, 0, nbatch, lane, k0, h0, lo0, hi0);
+    VelCon v0 = vc[k0];
+    level_slot(W, 1, nbatch, lane, k1, h1, lo1, hi1);
+    VelCon v1 = vc[k1];
+    for (int bt = 0; bt < nbatch; bt += 2) {
+        W.cover(bt);
+        level(v0, k0, h0, lo0, hi0);
+        level_slot(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
+        v0 = vc[k0];
+        if (bt + 1 >= nbatch) break;
+        level(v1, k1, h1, lo1, hi1);
+        level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
+        v1 = vc[k1];
+    }
+    return lres;
+}
+
 // Overlapped sweeps on two waves.  Sweeps s = 0, 1, ... (the warm start when
 // warm starting, then the velocity iterations) run the same levels; wave s & 1
 // runs sweep s.  An update of body b in sweep s must follow every update of b in
@@ -2028,15 +2075,23 @@ __device__ __forceinline__ void position_test(int *Lver, const int *LminS, int n
 // compact order is the order of first discovery, so only storage changes; every
 // constraint sees the bodies' values it would see in global memory.
 // ---------------------------------------------------------------------------
+//
+// LDS holds one float4 per body, the velocities in the velocity phase and then the
+// positions, and the level offsets; the impulses stay in the constraint records and
+// the maps in global memory, which leaves room for an island of about 8,000 bodies.
+// (With velocities, positions, impulses and maps all in LDS an island of 3,400 bodies
+// and 6,900 constraints did not fit and was swept from global memory by four waves
+// with a barrier per level: that one's solve took 23.4 ms and takes 12.5, the one of a
+// 50,000-box pyramid, 2,800 bodies and 5,300 constraints, 38.9 and 22.8.)
 struct CompactLds {
-    float4 *Lvel, *Lpos, *Limp;
-    int *Lbo, *Lmin, *Lsol, *blist, *ilist, *Lsched, *Lcur, *Lstat;
+    float4 *Lbody; // velocities, then positions
+    int *Lbo, *Lmin, *Lsol, *ilist, *Lcur;
+    int *blist, *sched, *stat; // in global memory
     int cb, ci, nl, c0; // compact bodies, islands, levels; first constraint (island order)
 };
-__host__ __device__ inline size_t compact_lds_bytes(int cb, int ci, int nc, int nl) {
-    return 2 * isl_align(16 * (size_t)cb) + isl_align(16 * (size_t)nc) + isl_align(4 * (size_t)(nl + 1)) +
-           2 * isl_align(4 * (size_t)ci) + isl_align(4 * (size_t)cb) + isl_align(4 * (size_t)ci) +
-           2 * isl_align(4 * (size_t)nc) + isl_align(4 * (size_t)nl);
+__host__ __device__ inline size_t compact_lds_bytes(int cb, int ci, int nl) {
+    return isl_align(16 * (size_t)cb) + isl_align(4 * (size_t)(nl + 1)) + 3 * isl_align(4 * (size_t)ci) +
+           isl_align(4 * (size_t)nl);
 }
 
 // Constraint set-up, warm start, velocity iterations and StoreImpulses on the compact
@@ -2101,19 +2156,20 @@ __device__ __forceinline__ bool compact_velocity(const Dev &d, int cur, const St
     C.nl = s_nl;
     C.c0 = c0;
     if (timed) d.ktime[37] = __builtin_amdgcn_s_memtime();
-    if (compact_lds_bytes(C.cb, C.ci, nc, C.nl) > (size_t)ldsBytes) return false;
+    if (compact_lds_bytes(C.cb, C.ci, C.nl) > (size_t)ldsBytes) return false;
     char *p = lds;
-    C.Lvel = (float4 *)p; p += isl_align(16 * (size_t)C.cb);
-    C.Lpos = (float4 *)p; p += isl_align(16 * (size_t)C.cb);
-    C.Limp = (float4 *)p; p += isl_align(16 * (size_t)nc);
+    C.Lbody = (float4 *)p; p += isl_align(16 * (size_t)C.cb);
     C.Lbo = (int *)p; p += isl_align(4 * (size_t)(C.nl + 1));
     C.Lmin = (int *)p; p += isl_align(4 * (size_t)C.ci);
     C.Lsol = (int *)p; p += isl_align(4 * (size_t)C.ci);
-    C.blist = (int *)p; p += isl_align(4 * (size_t)C.cb);
     C.ilist = (int *)p; p += isl_align(4 * (size_t)C.ci);
-    C.Lsched = (int *)p; p += isl_align(4 * (size_t)nc);
-    C.Lstat = (int *)p; p += isl_align(4 * (size_t)nc);
     C.Lcur = (int *)p;
+    // four ints per constraint of the continuous pass's slots, which that pass resets
+    // before it reads them: at most two bodies, a schedule entry and a static slot
+    int *far = reinterpret_cast<int *>(d.toiC + wd.contactBase + c0);
+    C.blist = far;
+    C.sched = far + 2 * (size_t)nc;
+    C.stat = far + 3 * (size_t)nc;
     __syncthreads(); // every thread has read the counts
     if (tid == 0) {
         s_cb = 0;
@@ -2141,7 +2197,7 @@ __device__ __forceinline__ bool compact_velocity(const Dev &d, int cur, const St
             C.blist[i] = bb;
             bmap[bb] = i;
         }
-        C.Lstat[k - c0] = stat;
+        C.stat[k - c0] = stat;
         if (atomicCAS(&imap[is], -2, -3) == -2) {
             const int i = atomicAdd(&s_ci, 1);
             C.ilist[i] = is;
@@ -2153,17 +2209,16 @@ __device__ __forceinline__ bool compact_velocity(const Dev &d, int cur, const St
     block_scan_array(C.Lbo, C.nl + 1, s_scan); // level offsets, C.Lbo[nl] = nc
     for (int i = tid; i < C.nl; i += BS) C.Lcur[i] = C.Lbo[i];
     __syncthreads();
-    for (int k = c0 + tid; k < c1; k += BS) C.Lsched[atomicAdd(&C.Lcur[cbatch[k]], 1)] = k;
+    for (int k = c0 + tid; k < c1; k += BS) C.sched[atomicAdd(&C.Lcur[cbatch[k]], 1)] = k;
     if (timed) d.ktime[38] = __builtin_amdgcn_s_memtime();
     for (int i = tid; i < C.cb; i += BS) {
         const int b = C.blist[i] >= 0 ? C.blist[i] : ~C.blist[i];
-        C.Lvel[i] = bvel[b];
-        C.Lpos[i] = bpos[b];
+        C.Lbody[i] = bvel[b];
     }
     __syncthreads();
     // constraints in level order (a level is a contiguous range), renumbered
     for (int j = tid; j < nc; j += BS) {
-        const int k = C.Lsched[j], cix = ordC[k], stat = C.Lstat[k - c0];
+        const int k = C.sched[j], cix = ordC[k], stat = C.stat[k - c0];
         VelCon v;
         PosCon q;
         init_constraint(v, q, cont[cix], cix, cisl[k], fbody, fmat, bfl, bmass, bpos, bvel, sp,
@@ -2176,7 +2231,6 @@ __device__ __forceinline__ bool compact_velocity(const Dev &d, int cur, const St
         q.island = imap[q.island];
         vc[j] = v;
         pc[j] = q;
-        C.Limp[j] = make_float4(v.nImp0, v.tImp0, v.nImp1, v.tImp1);
     }
     __syncthreads();
     if (timed) d.ktime[39] = __builtin_amdgcn_s_memtime();
@@ -2184,7 +2238,7 @@ __device__ __forceinline__ bool compact_velocity(const Dev &d, int cur, const St
     const int nbatch = C.nl;
     if (tid < 64) {
         const int lane = tid;
-        if (nbatch > 0 && (sp.flags & 1u)) velocity_sweep<0>(C.Lbo, nbatch, vc, C.Lvel, C.Limp, lane);
+        if (nbatch > 0 && (sp.flags & 1u)) velocity_sweep_far<0>(C.Lbo, nbatch, vc, C.Lbody, lane);
         if (timed) d.ktime[40] = __builtin_amdgcn_s_memtime();
         const int iters = residualMode ? sp.maxIterations : sp.velocityIterations;
         int used = 0;
@@ -2192,10 +2246,10 @@ __device__ __forceinline__ bool compact_velocity(const Dev &d, int cur, const St
         for (int it = 0; it < iters && nbatch > 0; ++it) {
             ++used;
             if (!residualMode) {
-                velocity_sweep<1>(C.Lbo, nbatch, vc, C.Lvel, C.Limp, lane);
+                velocity_sweep_far<1>(C.Lbo, nbatch, vc, C.Lbody, lane);
                 continue;
             }
-            float r = velocity_sweep<2>(C.Lbo, nbatch, vc, C.Lvel, C.Limp, lane);
+            float r = velocity_sweep_far<2>(C.Lbo, nbatch, vc, C.Lbody, lane);
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) r = fmaxr(r, __shfl_xor(r, o, 64));
             lastRes = r;
@@ -2211,19 +2265,18 @@ __device__ __forceinline__ bool compact_velocity(const Dev &d, int cur, const St
     // StoreImpulses (b2contactsolver.d:774-787) and the velocities back
     for (int j = tid; j < nc; j += BS) {
         const VelCon &v = vc[j];
-        const float4 im = C.Limp[j];
         Contact *c = cont + v.contact;
-        c->pt0.z = im.x;
-        c->pt0.w = im.y;
+        c->pt0.z = v.nImp0;
+        c->pt0.w = v.tImp0;
         if (v.pointCount > 1) {
-            c->pt1.z = im.z;
-            c->pt1.w = im.w;
+            c->pt1.z = v.nImp1;
+            c->pt1.w = v.tImp1;
         } else if (man_count(c->meta) > 1) {
             c->flags |= kContactSolvedOne; // PostSolve reports vc.pointCount points (b2island.d:448-456)
         }
     }
     for (int i = tid; i < C.cb; i += BS)
-        if (C.blist[i] >= 0) bvel[C.blist[i]] = C.Lvel[i];
+        if (C.blist[i] >= 0) bvel[C.blist[i]] = C.Lbody[i];
     if (timed) {
         d.ktime[42] = __builtin_amdgcn_s_memtime();
         d.ktime[45] = C.cb;
@@ -2244,7 +2297,7 @@ __device__ __forceinline__ void compact_position(const Dev &d, const StepParams 
     int *islSolved = d.islSolved + wd.islandBase;
     const bool timed = d.ktime && tid == 0 && C.c0 == 0 && wd.contactBase == d.W[d.order[0]].contactBase;
     if (timed) d.ktime[43] = __builtin_amdgcn_s_memtime();
-    for (int i = tid; i < C.cb; i += BS) C.Lpos[i] = bpos[C.blist[i] >= 0 ? C.blist[i] : ~C.blist[i]];
+    for (int i = tid; i < C.cb; i += BS) C.Lbody[i] = bpos[C.blist[i] >= 0 ? C.blist[i] : ~C.blist[i]];
     for (int i = tid; i < C.ci; i += BS) C.Lsol[i] = 0;
     for (int i = i0 + tid; i < i1; i += BS) islSolved[i] = sp.positionIterations > 0 ? 1 : 0;
     __syncthreads();
@@ -2253,7 +2306,7 @@ __device__ __forceinline__ void compact_position(const Dev &d, const StepParams 
         for (int it = 0; it < sp.positionIterations; ++it) {
             for (int i = lane; i < C.ci; i += 64)
                 if (!C.Lsol[i]) C.Lmin[i] = f2ord(0.0f);
-            if (C.nl > 0) position_sweep(C.Lbo, C.nl, pc, C.Lpos, C.Lmin, C.Lsol, lane);
+            if (C.nl > 0) position_sweep(C.Lbo, C.nl, pc, C.Lbody, C.Lmin, C.Lsol, lane);
             bool open = false;
             for (int i = lane; i < C.ci; i += 64) {
                 if (C.Lsol[i]) continue;
@@ -2265,7 +2318,7 @@ __device__ __forceinline__ void compact_position(const Dev &d, const StepParams 
     }
     __syncthreads();
     for (int i = tid; i < C.cb; i += BS)
-        if (C.blist[i] >= 0) bpos[C.blist[i]] = C.Lpos[i];
+        if (C.blist[i] >= 0) bpos[C.blist[i]] = C.Lbody[i];
     for (int i = tid; i < C.ci; i += BS) islSolved[C.ilist[i]] = C.Lsol[i];
     __syncthreads();
     if (timed) d.ktime[44] = __builtin_amdgcn_s_memtime();
