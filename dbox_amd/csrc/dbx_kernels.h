@@ -26,8 +26,9 @@ hipError_t launch_islands(const Dev &d, int cur, int ordered, int worldOffset, i
 hipError_t launch_islands_wide(const Dev &d, int cur, const WideBp *wide, int nwide, hipStream_t s);
 hipError_t launch_solve(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, int block,
                         int ldsBytes, bool lead, hipStream_t s);
-hipError_t launch_solve_wave(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, int ldsBytes,
-                             bool lead, hipStream_t s);
+// waves: 1 to 8 per world
+hipError_t launch_solve_wave(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, int waves,
+                             int ldsBytes, bool lead, hipStream_t s);
 // exact order with kStepGrouped: the islands of the tier's big worlds (no joints)
 // solved by groups of workgroups; the solve launches above skip those worlds
 hipError_t launch_solve_groups(const Dev &d, int cur, const StepParams &sp, const WideBp *wide, int nwide,

@@ -1792,22 +1792,28 @@ __device__ __forceinline__ float velocity_sweep_far(const int *Lbo, int nbatch, 
     return lres;
 }
 
-// Overlapped sweeps on two waves.  Sweeps s = 0, 1, ... (the warm start when
-// warm starting, then the velocity iterations) run the same levels; wave s & 1
-// runs sweep s.  An update of body b in sweep s must follow every update of b in
-// sweep s - 1 and precede every one in sweep s + 1 (the other wave's sweeps); all
-// other orders are free.  So level l of sweep s waits only until the other wave
-// has finished level need(l) of sweep s - 1, where need(l) is the largest level
-// holding a constraint on a dynamic body of level l (the last level that body is
-// updated in).  Each wave publishes its progress in LDS after every level, as
-// s * nbatch + levels done in sweep s, and as (s + 2) * nbatch once sweep s is
-// done (INT_MAX after its last sweep); progress only grows.  A wave in sweep s
-// waits only on the other wave's sweep s - 1, never on its sweep s + 1, and that
-// wave is never waiting on sweep s: of two waves one can always go on.  A wave's
-// LDS operations are performed in issue order, so a publication follows the
-// level's writes, and the waiting wave issues its reads only after it has seen
-// the publication.  Each lane publishes its own copy (one conflict-free write),
+// Overlapped sweeps on several waves.  Sweeps s = 0, 1, ... (the warm start when
+// warm starting, then the velocity iterations) run the same levels; of N waves,
+// wave s mod N runs sweep s.  An update of body b in sweep s must follow every update
+// of b in sweep s - 1 and precede every one in sweep s + 1; all other orders are
+// free.  So level l of sweep s waits only until the wave before it has finished
+// level need(l) of sweep s - 1, where need(l) is the largest level holding a
+// constraint on a dynamic body of level l (the last level that body is updated in).
+// Each wave publishes its progress in LDS after every level, as s * nbatch + levels
+// done in sweep s, and as (s + N) * nbatch, the start of its next sweep, once sweep s
+// is done (INT_MAX after its last sweep); progress only grows.  A wave in sweep s waits
+// only on sweep s - 1, never on a later one, so the earliest unfinished sweep can
+// always go on.  A wave's LDS operations are performed in issue order, so a publication
+// follows the level's writes, and the waiting wave issues its reads only after it has
+// seen the publication.  Each lane publishes its own copy (one conflict-free write),
 // read back by lane; the results are the sequential sweeps' bit for bit.
+//
+// How many waves help is the schedule's: a sweep trails the one before it by lag
+// levels (the largest need(l) - l, plus one), so N = levels / lag waves keep every
+// wave busy and more would only wait.  In a pile some body's contacts spread over
+// half the levels or more (two waves); in a tall stack a body meets its two
+// neighbours in consecutive levels, and eight sweeps run at once: 128 stack worlds
+// iterated to a residual take 5.4 ms a step in one wave's sweeps and 0.9 in eight's.
 __device__ __forceinline__ void pipe_wait(const int *Lnext, int other, int need, int &seen) {
     while (seen < need)
         seen = __builtin_amdgcn_readfirstlane(__hip_atomic_load(Lnext + 64 * other + (threadIdx.x & 63),
@@ -1820,12 +1826,13 @@ __device__ __forceinline__ void pipe_publish(int *Lnext, int me, int progress) {
                        __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// One sweep s of the overlapped velocity phase; Lneed holds need(l) per level.
+// One sweep s of the overlapped velocity phase; Lneed holds need(l) per level, prev
+// is the wave of sweep s - 1.  Returns the lane's residual (kMode 2).
 template <int kMode>
-__device__ __forceinline__ void velocity_sweep_piped(const int *Lbo, const int *Lneed, int nbatch,
+__device__ __forceinline__ float velocity_sweep_piped(const int *Lbo, const int *Lneed, int nbatch,
                                                      const VelCon *__restrict__ vc, float4 *Lvel, float4 *Limp,
                                                      int lane, int s, int endProgress, int *Lnext, int me,
-                                                     int &seen) {
+                                                     int prev, int &seen) {
     float lres = 0.0f;
     LevelWindow W{Lbo, nbatch + 1, 0, 0}, N{Lneed, nbatch, 0, 0};
     W.load(0);
@@ -1842,42 +1849,47 @@ __device__ __forceinline__ void velocity_sweep_piped(const int *Lbo, const int *
     for (int bt = 0; bt < nbatch; bt += 2) {
         W.cover(bt);
         N.cover(bt);
-        pipe_wait(Lnext, me ^ 1, base + N.at(bt), seen);
+        pipe_wait(Lnext, prev, base + N.at(bt), seen);
         velocity_level<kMode>(c0, k0, h0, lo0, hi0, vc, Lvel, Limp, lres);
         pipe_publish(Lnext, me, bt + 1 < nbatch ? mine + bt + 1 : endProgress);
         level_slot(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
         c0 = vc[k0];
         if (bt + 1 >= nbatch) break;
-        pipe_wait(Lnext, me ^ 1, base + N.at(bt + 1), seen);
+        pipe_wait(Lnext, prev, base + N.at(bt + 1), seen);
         velocity_level<kMode>(c1, k1, h1, lo1, hi1, vc, Lvel, Limp, lres);
         pipe_publish(Lnext, me, bt + 2 < nbatch ? mine + bt + 2 : endProgress);
         level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
         c1 = vc[k1];
     }
+    return lres;
 }
 
-// The warm start and nvel velocity iterations, overlapped on waves 0 and 1 of the
-// workgroup.  Lnext: 128 ints of LDS that hold 0 on entry.  Stamps the warm
-// start's end (or the velocity phase's start) through prof.
+// The warm start (when warm is set) and nvel velocity iterations, overlapped on the
+// workgroup's first nact waves.  Lnext: 64 ints of LDS per wave that hold 0 on entry.
+// kMode 2: Lres[i] receives iteration i's residual.  Stamps the warm start's end (or
+// the velocity phase's start) through prof.
+template <int kMode>
 __device__ __forceinline__ void velocity_piped(const int *Lbo, const int *Lneed, int nbatch,
-                                               const VelCon *__restrict__ vc, float4 *Lvel, float4 *Limp,
-                                               int *Lnext, bool warm, int nvel, const ProfStamp &prof) {
+                                               const VelCon *__restrict__ vc, float4 *Lvel, float4 *Limp, int *Lnext,
+                                               int nact, bool warm, int nvel, float *Lres, const ProfStamp &prof) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int nsweeps = (warm ? 1 : 0) + nvel;
+    const int nsweeps = (warm ? 1 : 0) + nvel, prev = wave > 0 ? wave - 1 : nact - 1;
     int seen = 0;
     if (!warm) prof.at(kProfVel0);
-    if (wave >= 2) return;
-    if (wave >= nsweeps) {
-        pipe_publish(Lnext, wave, INT_MAX);
-        return;
-    }
-    for (int s = wave; s < nsweeps; s += 2) {
-        const int endProgress = s + 2 < nsweeps ? (s + 2) * nbatch : INT_MAX;
+    if (wave >= nact) return;
+    for (int s = wave; s < nsweeps; s += nact) {
+        const int endProgress = s + nact < nsweeps ? (s + nact) * nbatch : INT_MAX;
         if (warm && s == 0) {
-            velocity_sweep_piped<0>(Lbo, Lneed, nbatch, vc, Lvel, Limp, lane, s, endProgress, Lnext, wave, seen);
+            velocity_sweep_piped<0>(Lbo, Lneed, nbatch, vc, Lvel, Limp, lane, s, endProgress, Lnext, wave, prev, seen);
             prof.at(kProfVel0);
         } else {
-            velocity_sweep_piped<1>(Lbo, Lneed, nbatch, vc, Lvel, Limp, lane, s, endProgress, Lnext, wave, seen);
+            float r = velocity_sweep_piped<kMode>(Lbo, Lneed, nbatch, vc, Lvel, Limp, lane, s, endProgress, Lnext, wave,
+                                                  prev, seen);
+            if (kMode == 2) {
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) r = fmaxr(r, __shfl_xor(r, o, 64));
+                if (lane == 0) Lres[s - (warm ? 1 : 0)] = r;
+            }
         }
     }
 }
@@ -1980,8 +1992,8 @@ __device__ __forceinline__ void position_sweep(const int *Lbo, int nbatch, const
     }
 }
 
-// The three position iterations overlapped on two waves (sweeps 0 and 2 on wave
-// 0, sweep 1 on wave 1), with the dependency waits of velocity_piped.  A sweep
+// The three position iterations overlapped on three waves (or two: sweeps 0 and 2
+// on wave 0), with the dependency waits of velocity_piped.  A sweep
 // depends on the per-island exit test of the sweep before it, which it cannot
 // wait for, so it runs speculatively: an island already known to be solved is
 // skipped, the others are solved, and a body's value before its first update of
@@ -2032,7 +2044,7 @@ __device__ __forceinline__ void position_level_piped(const PosCon &q, int slot, 
 __device__ __forceinline__ void position_sweep_piped(const int *Lbo, const int *Lneed, int nbatch,
                                                      const PosCon *__restrict__ pc, float4 *Lpos, int *LminS,
                                                      const int *Lver, int skip, const int *Lflag, float4 *Lbak,
-                                                     int lane, int s, int *Lnext, int me, int &seen) {
+                                                     int lane, int s, int *Lnext, int me, int prev, int &seen) {
     LevelWindow W{Lbo, nbatch + 1, 0, 0}, N{Lneed, nbatch, 0, 0};
     W.load(0);
     N.load(0);
@@ -2047,13 +2059,13 @@ __device__ __forceinline__ void position_sweep_piped(const int *Lbo, const int *
     for (int bt = 0; bt < nbatch; bt += 2) {
         W.cover(bt);
         N.cover(bt);
-        pipe_wait(Lnext, me ^ 1, base + N.at(bt), seen);
+        pipe_wait(Lnext, prev, base + N.at(bt), seen);
         position_level_piped(c0, k0, h0, lo0, hi0, pc, Lpos, LminS, Lver, skip, Lflag, Lbak);
         if (bt + 1 < nbatch) pipe_publish(Lnext, me, mine + bt + 1); // the last level: after the test
         level_slot<1>(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
         c0 = pc[k0];
         if (bt + 1 >= nbatch) break;
-        pipe_wait(Lnext, me ^ 1, base + N.at(bt + 1), seen);
+        pipe_wait(Lnext, prev, base + N.at(bt + 1), seen);
         position_level_piped(c1, k1, h1, lo1, hi1, pc, Lpos, LminS, Lver, skip, Lflag, Lbak);
         if (bt + 2 < nbatch) pipe_publish(Lnext, me, mine + bt + 2);
         level_slot<1>(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
@@ -2831,12 +2843,12 @@ __global__ __launch_bounds__(256) void k_solve_grp(Dev d, int cur, StepParams sp
     solve_world_global(d, cur, sp, w, lead != 0, lds, ldsBytes, blockIdx.x, G);
 }
 
-// The lead tier runs two waves per world (128 threads): the velocity phase
-// overlaps its sweeps on them (kStepPiped, velocity_piped) and the passes over
-// bodies and constraints are shared; the position sweeps stay on wave 0.  Other
-// tiers run one wave per world.
+// One to eight waves per world (solve_waves in the runtime): the velocity and
+// position phases overlap their sweeps on them (kStepPiped) and the passes over bodies
+// and constraints are shared.
+constexpr int kMaxSolveWaves = 8;
 template <bool kLead>
-__global__ __launch_bounds__(128) void k_solve_wave(Dev d, int cur, StepParams sp, int worldOffset, int ldsBytes) {
+__global__ __launch_bounds__(64 * kMaxSolveWaves) void k_solve_wave(Dev d, int cur, StepParams sp, int worldOffset, int ldsBytes) {
     extern __shared__ __align__(16) char lds[];
     const int w = d.order[worldOffset + blockIdx.x];
     const WorldDesc wd = d.W[w];
@@ -2851,11 +2863,13 @@ __global__ __launch_bounds__(128) void k_solve_wave(Dev d, int cur, StepParams s
     }
     const int tid = threadIdx.x, BS = blockDim.x, lane = tid & 63, wave = tid >> 6;
     const bool residualMode = (sp.flags & (1u << 5)) != 0;
-    // overlapped sweeps: two waves, per body the level of its last constraint
+    // overlapped sweeps: several waves, per body the level of its last constraint
     // (Llast), per level need(l) (Lneed) and the published progress (Lnext)
-    const size_t pipeBytes = isl_align(4 * (size_t)nb) + isl_align(4 * (size_t)nbatch) + 16 + 4 * 128;
-    const bool piped = (sp.flags & kStepPiped) && BS >= 128 && !residualMode && nbatch > 0 &&
-                       (long long)(sp.velocityIterations + 3) * (nbatch + 1) < (1ll << 30) &&
+    __shared__ float s_res[kMaxSolveWaves];
+    const int iters = residualMode ? sp.maxIterations : sp.velocityIterations;
+    const size_t pipeBytes = isl_align(4 * (size_t)nb) + isl_align(4 * (size_t)nbatch) + 16 + 4 * (size_t)BS;
+    const bool piped = (sp.flags & kStepPiped) && BS >= 128 && nbatch > 0 &&
+                       (long long)(iters + kMaxSolveWaves + 1) * (nbatch + 1) < (1ll << 30) &&
                        solve_lds_bytes(nb, nc, nbatch, nisl) + pipeBytes <= (size_t)ldsBytes;
     char *p = lds;
     float4 *Lvel = (float4 *)p; p += isl_align(16 * (size_t)nb);
@@ -2867,12 +2881,12 @@ __global__ __launch_bounds__(128) void k_solve_wave(Dev d, int cur, StepParams s
     int *Llast = (int *)p; p += isl_align(4 * (size_t)nb);
     int *Lneed = (int *)p; p += isl_align(4 * (size_t)nbatch);
     int *Llag = (int *)p; p += 16;
-    int *Lnext = (int *)p; p += 4 * 128;
+    int *Lnext = (int *)p; p += 4 * BS;
     // overlapped position iterations (three of them): per body the first level of
     // its constraints, per slot its first-update bits, the two sweeps' backups, the
     // later sweeps' minimum separations, the tests' verdicts and a second progress pair
     const size_t posBytes = isl_align(4 * (size_t)nb) + isl_align(4 * (size_t)nc) + 2 * isl_align(16 * (size_t)nb) +
-                            3 * isl_align(4 * (size_t)nisl) + 4 * 128;
+                            3 * isl_align(4 * (size_t)nisl) + 4 * (size_t)BS;
     const bool pipedPos = piped && sp.positionIterations == 3 &&
                           solve_lds_bytes(nb, nc, nbatch, nisl) + pipeBytes + posBytes <= (size_t)ldsBytes;
     int *Lfirst = (int *)p; p += isl_align(4 * (size_t)nb);
@@ -2917,12 +2931,12 @@ __global__ __launch_bounds__(128) void k_solve_wave(Dev d, int cur, StepParams s
     if (piped) {
         for (int b = tid; b < nb; b += BS) Llast[b] = -1;
         for (int i = tid; i < nbatch; i += BS) Lneed[i] = 0;
-        if (tid < 128) Lnext[tid] = 0;
+        Lnext[tid] = 0;
         if (tid == 0) Llag[0] = 0;
     }
     if (pipedPos) {
         for (int b = tid; b < nb; b += BS) Lfirst[b] = INT_MAX;
-        if (tid < 128) Lnext2[tid] = 0;
+        Lnext2[tid] = 0;
     }
     // Integrate velocities with damping (b2island.d:82-116) while staging the bodies.
     for (int b = tid; b < nb; b += BS) {
@@ -2977,7 +2991,7 @@ __global__ __launch_bounds__(128) void k_solve_wave(Dev d, int cur, StepParams s
     if (sp.flags & ((1u << 4) | (1u << 6))) mlp_new_points(d, w, nc, sp.flags, vc, pc, cont, ImpRef{Limp, 1}, Lvel, Lpos);
 
     if (timed && tid == 0) d.ktime[5] = __builtin_amdgcn_s_memtime();
-    bool overlap = false, overlapPos = false;
+    int nact = 0, posWaves = 0; // waves of the overlapped velocity and position sweeps (0: one after the other)
     if (piped) {
         // need(l): the last level of the dynamic bodies of level l's constraints;
         // the lag: the most levels a sweep's level l must trail need(l) by
@@ -2992,26 +3006,70 @@ __global__ __launch_bounds__(128) void k_solve_wave(Dev d, int cur, StepParams s
             }
         }
         __syncthreads();
-        // a sweep starts at least lag + 1 levels after the one before it, and two
-        // sweeps after it on the same wave: overlapped only when that gains a tenth
+        // a sweep starts at least lag levels after the one before it and `waves`
+        // sweeps after it on the same wave: overlapped only when that gains a tenth.
+        // The residual mode overlaps one sweep per wave and keeps its start in the
+        // position phase's first backup.
         const int lag = __builtin_amdgcn_readfirstlane(Llag[0]) + 1;
+        const int waves =
+            (sp.flags & kStepPipedAlways) ? BS / 64 : max(2, min(BS / 64, (nbatch + lag - 1) / lag));
+        auto gains = [&](long long sweeps, int n) {
+            const long long stride = max(lag, (nbatch + n - 1) / n);
+            return (sp.flags & kStepPipedAlways) || 10 * ((sweeps - 1) * stride + nbatch) <= 9 * sweeps * nbatch;
+        };
         const int ns = ((sp.flags & 1u) ? 1 : 0) + sp.velocityIterations;
-        const long long stride = max(lag, (nbatch + 1) / 2);
-        overlap = ns > 1 && ((sp.flags & kStepPipedAlways) || 10 * ((ns - 1) * stride + nbatch) <= 9ll * ns * nbatch);
-        overlapPos = pipedPos && ((sp.flags & kStepPipedAlways) || 10 * (2 * stride + nbatch) <= 27ll * nbatch);
+        if (residualMode ? pipedPos && iters > 1 && gains(waves, waves) : ns > 1 && gains(ns, waves)) nact = waves;
+        posWaves = pipedPos && gains(3, min(waves, 3)) ? min(waves, 3) : 0;
     }
-    if (overlap) {
-        velocity_piped(Lbo, Lneed, nbatch, vc, Lvel, Limp, Lnext, (sp.flags & 1u) != 0, sp.velocityIterations, prof);
+    if (nact > 0 && !residualMode) {
+        velocity_piped<1>(Lbo, Lneed, nbatch, vc, Lvel, Limp, Lnext, nact, (sp.flags & 1u) != 0, sp.velocityIterations,
+                          nullptr, prof);
         if (tid == 0) {
             d.S[w].iterations = sp.velocityIterations;
             d.S[w].residual = -1.0f;
         }
-        if (timed && lane == 0) d.ktime[6 + wave] = __builtin_amdgcn_s_memtime(); // each wave's last sweep done
+        if (timed && lane == 0 && wave < 2) d.ktime[6 + wave] = __builtin_amdgcn_s_memtime(); // its last sweep done
+    } else if (nact > 0) {
+        // Residual mode, a batch of one iteration per wave at a time: the batch runs
+        // past the iteration whose residual ends the step, if it holds one, so its start
+        // is kept (velocities in Lbak1, impulses in the constraint records) and a batch
+        // that went too far is run again from there up to that iteration.
+        int used = 0;
+        float lastRes = 0.0f;
+        bool warm = (sp.flags & 1u) != 0;
+        while (used < iters) {
+            const int n = min(nact, iters - used);
+            for (int b = tid; b < nb; b += BS) Lbak1[b] = Lvel[b];
+            for (int k = tid; k < nc; k += BS) *reinterpret_cast<float4 *>(&vc[k].nImp0) = Limp[k];
+            __syncthreads();
+            velocity_piped<2>(Lbo, Lneed, nbatch, vc, Lvel, Limp, Lnext, nact, warm, n, s_res,
+                              used == 0 ? prof : ProfStamp{});
+            __syncthreads();
+            int last = 0;
+            while (last < n && !(s_res[last] <= sp.residualTol)) ++last;
+            const bool stop = last < n;
+            lastRes = s_res[stop ? last : n - 1];
+            Lnext[tid] = 0;
+            if (stop && last + 1 < n) {
+                for (int b = tid; b < nb; b += BS) Lvel[b] = Lbak1[b];
+                for (int k = tid; k < nc; k += BS) Limp[k] = *reinterpret_cast<const float4 *>(&vc[k].nImp0);
+                __syncthreads();
+                velocity_piped<1>(Lbo, Lneed, nbatch, vc, Lvel, Limp, Lnext, nact, warm, last + 1, nullptr, ProfStamp{});
+            }
+            used += stop ? last + 1 : n;
+            warm = false;
+            __syncthreads();
+            if (stop) break;
+        }
+        if (tid == 0) {
+            d.S[w].iterations = used;
+            d.S[w].residual = lastRes;
+        }
+        if (timed && tid == 0) d.ktime[6] = d.ktime[7] = __builtin_amdgcn_s_memtime();
     } else if (wave == 0) {
         if (nbatch > 0 && (sp.flags & 1u)) velocity_sweep<0>(Lbo, nbatch, vc, Lvel, Limp, lane);
         if (timed && lane == 0) d.ktime[6] = __builtin_amdgcn_s_memtime();
         prof.at(kProfVel0);
-        const int iters = residualMode ? sp.maxIterations : sp.velocityIterations;
         int used = 0;
         float lastRes = residualMode ? 0.0f : -1.0f;
         for (int it = 0; it < iters && nbatch > 0; ++it) {
@@ -3069,7 +3127,7 @@ __global__ __launch_bounds__(128) void k_solve_wave(Dev d, int cur, StepParams s
         Lvel[b] = make_float4(v.x, v.y, wv, 0.0f);
     }
     for (int i = tid; i < nisl; i += BS) Lsol[i] = 0;
-    if (overlapPos)
+    if (posWaves)
         for (int i = tid; i < nisl; i += BS) {
             Lmin[i] = f2ord(0.0f);
             Lmin1[i] = f2ord(0.0f);
@@ -3078,19 +3136,22 @@ __global__ __launch_bounds__(128) void k_solve_wave(Dev d, int cur, StepParams s
         }
     __syncthreads();
     prof.at(kProfPos0);
-    if (overlapPos) {
+    if (posWaves) {
         // the three position iterations overlapped (position_sweep_piped)
         int seen = 0;
+        const int own2 = posWaves == 3 ? 2 : 0; // sweep 2's wave; with two waves it runs after sweep 0 on wave 0
         if (wave == 0) {
-            position_sweep_piped(Lbo, Lneed, nbatch, pc, Lpos, Lmin, Lver, 0, Lflag, nullptr, lane, 0, Lnext2, 0, seen);
+            position_sweep_piped(Lbo, Lneed, nbatch, pc, Lpos, Lmin, Lver, 0, Lflag, nullptr, lane, 0, Lnext2, 0, 1, seen);
             position_test(Lver, Lmin, nisl, 0, lane);
-            pipe_publish(Lnext2, 0, 2 * nbatch);
-            position_sweep_piped(Lbo, Lneed, nbatch, pc, Lpos, Lmin2, Lver, 3, Lflag, Lbak2, lane, 2, Lnext2, 0, seen);
-            position_test(Lver, Lmin2, nisl, 2, lane);
+            pipe_publish(Lnext2, 0, own2 == 0 ? 2 * nbatch : INT_MAX);
         } else if (wave == 1) {
-            position_sweep_piped(Lbo, Lneed, nbatch, pc, Lpos, Lmin1, Lver, 1, Lflag, Lbak1, lane, 1, Lnext2, 1, seen);
+            position_sweep_piped(Lbo, Lneed, nbatch, pc, Lpos, Lmin1, Lver, 1, Lflag, Lbak1, lane, 1, Lnext2, 1, 0, seen);
             position_test(Lver, Lmin1, nisl, 1, lane);
             pipe_publish(Lnext2, 1, INT_MAX);
+        }
+        if (wave == own2) {
+            position_sweep_piped(Lbo, Lneed, nbatch, pc, Lpos, Lmin2, Lver, 3, Lflag, Lbak2, lane, 2, Lnext2, own2, 1, seen);
+            position_test(Lver, Lmin2, nisl, 2, lane);
         }
         __syncthreads();
         // islands solved by the sweep-0 test get their bodies from before sweep 1,
@@ -3105,7 +3166,7 @@ __global__ __launch_bounds__(128) void k_solve_wave(Dev d, int cur, StepParams s
         for (int i = tid; i < nisl; i += BS) Lsol[i] = Lver[i] != 0;
     }
     // Position iterations with the per-island early exit (b2island.d:206-224), on wave 0.
-    for (int it = 0; it < sp.positionIterations && wave == 0 && !overlapPos; ++it) {
+    for (int it = 0; it < sp.positionIterations && wave == 0 && !posWaves; ++it) {
         for (int i = lane; i < nisl; i += 64)
             if (!Lsol[i]) Lmin[i] = f2ord(0.0f);
         if (nbatch > 0) position_sweep(Lbo, nbatch, pc, Lpos, Lmin, Lsol, lane);
@@ -5377,11 +5438,11 @@ hipError_t launch_solve_groups(const Dev &d, int cur, const StepParams &sp, cons
     }
     return hipGetLastError();
 }
-hipError_t launch_solve_wave(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, int ldsBytes,
-                             bool lead, hipStream_t s) {
+hipError_t launch_solve_wave(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, int waves,
+                             int ldsBytes, bool lead, hipStream_t s) {
     if (nworlds <= 0) return hipSuccess;
-    DBX_LAUNCH(k_solve_wave, lead, dim3(nworlds), dim3(lead ? 128 : 64), ldsBytes, s, d, cur, sp, worldOffset,
-               ldsBytes);
+    if (waves < 1 || waves > kMaxSolveWaves) return hipErrorInvalidValue;
+    DBX_LAUNCH(k_solve_wave, lead, dim3(nworlds), dim3(64 * waves), ldsBytes, s, d, cur, sp, worldOffset, ldsBytes);
     return hipGetLastError();
 }
 size_t broadphase_scratch_bytes(int proxies) { return bp_bytes(proxies); }

@@ -635,6 +635,7 @@ bool build_world(const dbx_body_def *bodies, int nb, const dbx_fixture_def *fx, 
 struct Tier {
     int first = 0, count = 0; // range in the launch order
     int lds = 0;
+    int bodies = 0;           // of its largest world
     int block = 256;          // threads of its collide, broadphase and coloured-solve workgroups
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;
@@ -1036,6 +1037,7 @@ dbx_status dbx_finalize(dbx_handle *h) {
                 tiers.push_back(T);
             }
             tiers.back().count++;
+            tiers.back().bodies = std::max(tiers.back().bodies, h->W[order[i]].bodyCount);
         }
         // A world whose broadphase scratch does not fit in its tier's LDS has its
         // pairs found by the device-wide pass.
@@ -1292,6 +1294,19 @@ static dbx_status stage_mlp(dbx_handle *h) {
     return DBX_OK;
 }
 
+// Waves per world of the exact-order solve.  A world's sweeps overlap on its waves as
+// far as its schedule lets them, and its other passes are shared by them; a wave
+// that has nothing to do still holds registers (two such waves fit a SIMD) and joins
+// every barrier, so a world gets one per 16 bodies, and more than one only while the
+// handle's worlds leave room for it on the device.  The lead tier's few worlds, which
+// set the step time, are not held back by the others.
+static int solve_waves(const dbx_handle *h, const Tier &T, bool lead) {
+    int w = 8;
+    while (w > 1 && (16 * w > T.bodies + 15 || (!(lead && T.count <= kLeadCus) && (long long)w * h->nworlds > 8ll * h->cuCount)))
+        w >>= 1;
+    return lead ? std::max(w, 2) : w;
+}
+
 // The step chain of one tier (b2World.Step, b2world.d:367-434, for its worlds).
 // part bits: 1 = FindNewContacts (when fixtures were added), 2 = Collide, 4 = the
 // island search and everything after it.
@@ -1319,7 +1334,7 @@ static dbx_status step_tier(dbx_handle *h, int t, const StepParams &sp, uint32_t
         // worlds too big for LDS (all with the device-wide broadphase): their levels
         // (hundreds of constraints wide in a 20,000-body container) are swept from
         // global memory by a 256-thread workgroup, level batches separated by barriers.
-        if (ordered && T.wideCount < T.count) DBX_HIP(h, launch_solve_wave(d, cout, sp, T.first, T.count, lds1, lead, s));
+        if (ordered && T.wideCount < T.count) DBX_HIP(h, launch_solve_wave(d, cout, sp, T.first, T.count, solve_waves(h, T, lead), lds1, lead, s));
         else DBX_HIP(h, launch_solve(d, cout, sp, T.first, T.count, ordered ? 256 : T.block, ordered ? lds1 : 0, lead, s));
         if (ordered && T.wideCount && d.iwParent && (sp.flags & kStepGrouped))
             DBX_HIP(h, launch_solve_groups(d, cout, sp, wide, T.wideCount, lds1, lead, s));
@@ -1476,7 +1491,7 @@ dbx_status dbx_step(dbx_handle *h, float dt, int32_t vel, int32_t pos, uint32_t 
     if ((flags & DBX_STEP_ORDERED) && !(flags & (DBX_STEP_RESIDUAL | DBX_STEP_LEARNED | DBX_STEP_LOG)) &&
         !getenv("DBX_SOLVE_UNGROUPED"))
         sp.flags |= kStepGrouped;
-    if ((flags & DBX_STEP_ORDERED) && !(flags & DBX_STEP_RESIDUAL) && !getenv("DBX_SWEEPS_SEQUENTIAL"))
+    if ((flags & DBX_STEP_ORDERED) && !getenv("DBX_SWEEPS_SEQUENTIAL"))
         sp.flags |= kStepPiped | (getenv("DBX_SWEEPS_OVERLAP_ALWAYS") ? kStepPipedAlways : 0u);
     if ((flags & (DBX_STEP_LEARNED | DBX_STEP_LOG)) && !h->staged) {
         dbx_status st = stage_mlp(h);

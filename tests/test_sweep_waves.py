@@ -1,0 +1,136 @@
+"""Sweeps overlapped on up to eight waves: a CPU model of the protocol (wave s mod N
+runs sweep s and waits on the wave before it), and on the GPU the overlapped steps
+against sequential ones, bit for bit, with fixed iteration counts and in the residual
+mode, whose batches of sweeps run past the iteration that ends them and roll back."""
+import random
+
+import numpy as np
+import pytest
+
+from dbox_amd import native, scenes
+from tests.test_overlap_protocol import _levels
+
+DT = 1.0 / 60.0
+
+
+def _run(seed, waves, short=False):
+    R = random.Random(seed)
+    nb, n = R.randint(2, 30), R.randint(1, 60)
+    cons = [(R.randrange(nb), R.randrange(nb), R.choice([1, 2, 3, 3, 3])) for _ in range(n)]
+    lvl, llast = _levels(cons)
+    N = max(lvl) + 1
+    need = [0] * N
+    for (a, b, dm), l in zip(cons, lvl):
+        need[l] = max(need[l], llast[a] if dm & 1 else 0, llast[b] if dm & 2 else 0)
+    if short:
+        need = [max(x - 1, 0) for x in need]
+    ns = R.randint(1, 20)
+    levels = [[i for i in range(n) if lvl[i] == l] for l in range(N)]
+    ref, got = {x: [] for x in range(nb)}, {x: [] for x in range(nb)}
+
+    def level(s, l, out):
+        for i in levels[l]:
+            a, b, dm = cons[i]
+            if dm & 1:
+                out[a].append((s, i))
+            if dm & 2:
+                out[b].append((s, i))
+
+    for s in range(ns):
+        for l in range(N):
+            level(s, l, ref)
+    inf = 10 ** 9
+    pub, pos = [0] * waves, [0] * waves
+    plans = [[(s, l) for s in range(w, ns, waves) for l in range(N)] for w in range(waves)]
+    while True:
+        open_ = [w for w in range(waves) if pos[w] < len(plans[w])]
+        if not open_:
+            return None if got == ref else "order"
+        ready = []
+        for w in open_:
+            s, l = plans[w][pos[w]]
+            if s == 0 or pub[(w - 1) % waves] >= (s - 1) * N + need[l] + 1:
+                ready.append(w)
+        if not ready:
+            return "deadlock"
+        w = R.choice(ready)
+        s, l = plans[w][pos[w]]
+        level(s, l, got)
+        pos[w] += 1
+        pub[w] = s * N + l + 1 if l + 1 < N else ((s + waves) * N if s + waves < ns else inf)
+
+
+@pytest.mark.parametrize("waves", [2, 3, 5, 8])
+def test_protocol_keeps_every_body_in_order_and_finishes(waves):
+    bad = [(k, r) for k in range(600) if (r := _run(k, waves))]
+    assert not bad, bad[:5]
+    assert sum(_run(k, waves, short=True) == "order" for k in range(300)) > 50
+
+
+def _handles(ws):
+    out = {}
+    for m in ("default", "always", "sequential"):
+        h = native.StepWorlds()
+        for s in ws:
+            h.add_scene(s)
+        h.finalize()
+        out[m] = h
+    return out
+
+
+ENV = {"default": {}, "always": {"DBX_SWEEPS_OVERLAP_ALWAYS": "1"}, "sequential": {"DBX_SWEEPS_SEQUENTIAL": "1"}}
+
+
+def _step(hs, monkeypatch, vel, pos, flags):
+    for m, env in ENV.items():
+        for var in ("DBX_SWEEPS_OVERLAP_ALWAYS", "DBX_SWEEPS_SEQUENTIAL"):
+            monkeypatch.delenv(var, raising=False)
+        for var, val in env.items():
+            monkeypatch.setenv(var, val)
+        hs[m].step(DT, vel, pos, flags)
+
+
+def _same(hs, label):
+    for w in range(hs["sequential"].world_count):
+        for m in ("default", "always"):
+            assert hs[m].bodies(w).tobytes() == hs["sequential"].bodies(w).tobytes(), f"{label}, {m}, world {w}: bodies"
+            assert hs[m].contacts(w).tobytes() == hs["sequential"].contacts(w).tobytes(), f"{label}, {m}, world {w}"
+
+
+def _worlds():
+    return ([scenes.stacks_world(k) for k in range(6)] + [scenes.pyramid(n, seed=n) for n in (1, 2, 3, 9, 20)] +
+            [scenes.mixed_container(n, 14.0, 30.0, n) for n in (8, 60, 250)] + [scenes.hello_world()])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vel,pos,warm", [(8, 3, True), (8, 3, False), (1, 3, True), (20, 2, True), (0, 3, True)])
+def test_overlapped_sweeps_equal_sequential(vel, pos, warm, monkeypatch):
+    print(f"case: sweeps on several waves, {vel} / {pos} iterations, warm {warm}", flush=True)
+    hs = _handles(_worlds())
+    flags = native.SLEEP | native.ORDERED | (native.WARM if warm else 0)
+    for i in range(90):
+        _step(hs, monkeypatch, vel, pos, flags)
+        if i % 30 == 29:
+            _same(hs, f"step {i + 1}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tol,most", [(1e-3, 100), (1e-1, 13), (1e-3, 1), (-1.0, 8), (-1.0, 9), (-1.0, 17), (1e9, 50)])
+def test_overlapped_residual_sweeps_equal_sequential(tol, most, monkeypatch):
+    print(f"case: residual sweeps on several waves, tolerance {tol}, at most {most}", flush=True)
+    hs = _handles(_worlds())
+    for h in hs.values():
+        h.set_residual(tol, most)
+    flags = native.WARM | native.SLEEP | native.ORDERED | native.RESIDUAL
+    seen = set()
+    for i in range(40):
+        _step(hs, monkeypatch, 8, 3, flags)
+        its = {m: h.solver_stats()[0] for m, h in hs.items()}
+        res = {m: h.residuals() for m, h in hs.items()}
+        for m in ("default", "always"):
+            assert np.array_equal(its[m], its["sequential"]) and res[m].tobytes() == res["sequential"].tobytes(), (i, m)
+        seen |= set(its["sequential"].tolist())
+        if i % 20 == 19:
+            _same(hs, f"step {i + 1}")
+    if tol == 1e-3 and most == 100:
+        assert len(seen) > 8  # ends inside a batch of sweeps as well as at its end
