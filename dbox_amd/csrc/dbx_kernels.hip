@@ -3291,20 +3291,137 @@ __device__ __forceinline__ unsigned int f2key(float f) {
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
+// Positive exactly when a and f do not overlap (b2TestOverlap, overlap()): the
+// largest of the four gaps.  The constant stands for a gap that is not a number
+// (infinity minus infinity), which overlap() does not take for a separation either.
+__device__ __forceinline__ float bp1_gap(float4 a, float4 f) {
+    return __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(f.x - a.z, f.y - a.w), a.x - f.z),
+                           __builtin_fmaxf(a.y - f.w, -1.0f));
+}
+// Sorts the np pair keys of LDS (P2: the power of two above np) and writes the pairs.
+__device__ __forceinline__ void bp_sort_out(unsigned long long *skeys, int np, int P2, int2 *out) {
+    const int tid = threadIdx.x, BS = blockDim.x;
+    for (int i = np + tid; i < P2; i += BS) skeys[i] = ~0ull;
+    __syncthreads();
+    for (int k = 2; k <= P2; k <<= 1) {
+        for (int jj = k >> 1; jj > 0; jj >>= 1) {
+            for (int i = tid; i < P2; i += BS) {
+                const int ixj = i ^ jj;
+                if (ixj > i) {
+                    const unsigned long long x = skeys[i], y = skeys[ixj];
+                    if ((x > y) == ((i & k) == 0)) {
+                        skeys[i] = y;
+                        skeys[ixj] = x;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+    for (int e = tid; e < np; e += BS) {
+        const unsigned long long key = skeys[e];
+        out[e] = make_int2((int)(key >> 32), (int)(key & 0xffffffffu));
+    }
+    __syncthreads();
+}
+
+// A workgroup tests all its proxies against each moved one directly while that is at
+// most kBpDirect wave steps per wave (proxies / threads x moved proxies), and sorts and
+// sweeps beyond.  The sort is bound by its barriers, some 25 us for the smallest world:
+// a container's step took 27 us sorted and 12 direct with 60 bodies, 41 and 20 with 250,
+// 152 and 89 with 1,000 (256 threads).  With every proxy moved both cost the same from
+// about 1,000 proxies on 256 threads (210 and 213 us, 4,000 steps) and 1,500 on 1,024
+// (133 and 133 us, 3,000 steps); 2,500 on 1,024 take 241 us sorted and 272 direct.
+constexpr int kBpDirect = 4096;
+// Pairs ordered by counting the smaller ones (60 bodies: 12.4 us a step, with the
+// sorting network 14.7); the count grows with the square, the network does not.
+constexpr int kBpRank = 192;
+
 // Returns the pair count; pairs are written only when they fit in cap.
 // Pairs are emitted and sorted in `stage` (LDS, stageCap pairs) when they fit
 // there, and copied to `out` afterwards; otherwise they are sorted in `out`.
 __device__ __forceinline__ int bp_pairs(const float4 *gfat, const int *gmoved, int n, BpMem M, int2 *out, int cap,
                                         int2 *stage, int stageCap, int *s_tmp) {
-    const int tid = threadIdx.x, BS = blockDim.x;
-    __shared__ int s_ext[4];
+    const int tid = threadIdx.x, BS = blockDim.x, lane = tid & 63;
+    __shared__ int s_ext[4], s_nm, s_np;
     if (tid < 4) s_ext[tid] = (tid < 2) ? f2ord(kMaxFloat) : f2ord(-kMaxFloat);
+    if (tid == 0) s_nm = s_np = 0;
     __syncthreads();
+    for (int c0 = 0; c0 < n; c0 += BS) {
+        const int i = c0 + tid;
+        bool mv = false;
+        if (i < n) {
+            M.fat[i] = gfat[i];
+            const int m = gmoved[i];
+            M.moved[i] = m;
+            mv = m != 0;
+        }
+        // the moved proxies, in any order, in M.cur
+        const unsigned long long mm = __builtin_amdgcn_ballot_w64(mv);
+        int at = 0;
+        if (lane == 0 && mm) at = atomicAdd(&s_nm, __popcll(mm));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (mv) M.cur[at + __popcll(mm & ((1ull << lane) - 1ull))] = i;
+    }
+    __syncthreads();
+    const int nm = s_nm;
+    if (nm == 0) return 0; // every pair has a moved member
+    unsigned long long *skeys = (unsigned long long *)stage;
+    if ((long long)((n + BS - 1) / BS) * nm <= kBpDirect) {
+        // Few tests: every proxy, one per lane, against each moved one, whose AABB all
+        // lanes read at once.  A pair of two moved proxies is kept where the larger is in
+        // the lane.
+        for (int c0 = 0; c0 < n; c0 += BS) {
+            const int i = c0 + tid;
+            const float4 a = M.fat[min(i, n - 1)];
+            const bool mi = i < n && M.moved[i];
+            for (int q0 = 0; q0 < nm; q0 += 4) {
+                int j[4];
+                float4 f[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) j[u] = M.cur[min(q0 + u, nm - 1)];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) f[u] = M.fat[j[u]];
+                float gap[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) gap[u] = bp1_gap(a, f[u]);
+                if (!__builtin_amdgcn_ballot_w64(
+                        __builtin_fminf(__builtin_fminf(gap[0], gap[1]), __builtin_fminf(gap[2], gap[3])) <= 0.0f))
+                    continue;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (!(gap[u] <= 0.0f) || q0 + u >= nm || i >= n || i == j[u] || (mi && i < j[u])) continue;
+                    const int slot = atomicAdd(&s_np, 1);
+                    const unsigned int x = i < j[u] ? i : j[u], y = i < j[u] ? j[u] : i;
+                    if (slot < stageCap) skeys[slot] = ((unsigned long long)x << 32) | y;
+                }
+            }
+        }
+        __syncthreads();
+        const int np = s_np;
+        if (np > cap) return np;
+        if (np <= stageCap && np <= kBpRank) { // in order by counting the smaller keys
+            for (int e = tid; e < np; e += BS) {
+                const unsigned long long key = skeys[e];
+                int r = 0;
+                for (int q = 0; q < np; ++q) r += skeys[q] < key ? 1 : 0;
+                out[r] = make_int2((int)(key >> 32), (int)(key & 0xffffffffu));
+            }
+            __syncthreads();
+            return np;
+        }
+        const int P2 = bp_pow2(np);
+        if (P2 <= stageCap) {
+            bp_sort_out(skeys, np, P2, out);
+            return np;
+        }
+        __syncthreads();
+        if (tid == 0) s_np = 0; // too many pairs for the staging space: sort and sweep
+        __syncthreads();
+    }
     float lx = kMaxFloat, ly = kMaxFloat, hx = -kMaxFloat, hy = -kMaxFloat;
     for (int i = tid; i < n; i += BS) {
-        float4 f = gfat[i];
-        M.fat[i] = f;
-        M.moved[i] = gmoved[i];
+        const float4 f = M.fat[i];
         M.cnt[i] = 0;
         M.cur[i] = 0;
         lx = fminr(lx, f.x);
@@ -3353,8 +3470,6 @@ __device__ __forceinline__ int bp_pairs(const float4 *gfat, const int *gmoved, i
     // pairs are collected as (a << 32 | b) keys and sorted, which is the
     // b2PairLessThan order.
     {
-        __shared__ int s_np;
-        if (tid == 0) s_np = 0;
         for (int p = tid; p < n; p += BS) {
             const float4 fi = M.fat[(int)(M.keys[p] & 0xffffffffu)];
             const unsigned int hk = f2key(axis == 0 ? fi.z : fi.w);
@@ -3369,7 +3484,6 @@ __device__ __forceinline__ int bp_pairs(const float4 *gfat, const int *gmoved, i
         }
         __syncthreads();
         const int C = block_scan_array(M.cur, n, s_tmp);
-        unsigned long long *skeys = (unsigned long long *)stage;
         for (int t = tid; t < C; t += BS) {
             int lo = 0, hi = n; // last p with cur[p] <= t
             while (hi - lo > 1) {
@@ -3391,28 +3505,7 @@ __device__ __forceinline__ int bp_pairs(const float4 *gfat, const int *gmoved, i
         if (np > cap) return np;
         const int P2 = bp_pow2(np > 0 ? np : 1);
         if (P2 <= stageCap) {
-            for (int i = np + tid; i < P2; i += BS) skeys[i] = ~0ull;
-            __syncthreads();
-            for (int k = 2; k <= P2; k <<= 1) {
-                for (int jj = k >> 1; jj > 0; jj >>= 1) {
-                    for (int i = tid; i < P2; i += BS) {
-                        const int ixj = i ^ jj;
-                        if (ixj > i) {
-                            const unsigned long long x = skeys[i], y = skeys[ixj];
-                            if ((x > y) == ((i & k) == 0)) {
-                                skeys[i] = y;
-                                skeys[ixj] = x;
-                            }
-                        }
-                    }
-                    __syncthreads();
-                }
-            }
-            for (int e = tid; e < np; e += BS) {
-                const unsigned long long key = skeys[e];
-                out[e] = make_int2((int)(key >> 32), (int)(key & 0xffffffffu));
-            }
-            __syncthreads();
+            bp_sort_out(skeys, np, P2, out);
             return np;
         }
         // too many pairs for the staging space: per-proxy lists below
@@ -4916,13 +5009,6 @@ __device__ __forceinline__ void bp1_cell(const Bp1 &b, int cell, int &blk, int &
     const int end = wave_incl_scan(mine);
     seg = __popcll(__builtin_amdgcn_ballot_w64(end <= cell));
     blk = cell - (seg > 0 ? __builtin_amdgcn_readlane(end, seg - 1) : 0);
-}
-// Positive exactly when a and f do not overlap (b2TestOverlap, overlap()): the
-// largest of the four gaps.  The constant stands for a gap that is not a number
-// (infinity minus infinity), which overlap() does not take for a separation either.
-__device__ __forceinline__ float bp1_gap(float4 a, float4 f) {
-    return __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(f.x - a.z, f.y - a.w), a.x - f.z),
-                           __builtin_fmaxf(a.y - f.w, -1.0f));
 }
 __device__ __forceinline__ float lane_value(float x, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
