@@ -20,8 +20,8 @@ namespace dbx {
 enum : int { kJointRevolute = 1, kJointPrismatic = 2, kJointDistance = 3, kJointPulley = 4, kJointMouse = 5,
              kJointGear = 6, kJointWheel = 7, kJointWeld = 8, kJointFriction = 9, kJointRope = 10, kJointMotor = 11 };
 enum : int { kLimitInactive = 0, kLimitLower = 1, kLimitUpper = 2, kLimitEqual = 3 }; // b2LimitState
-// JointRec.flags: b2JointDef.collideConnected, enableLimit, enableMotor, and b2Joint.m_islandFlag
-enum : int { kJointCollide = 1, kJointLimit = 2, kJointMotorOn = 4, kJointInIsland = 8 };
+// JointRec.flags: b2JointDef.collideConnected, enableLimit, enableMotor
+enum : int { kJointCollide = 1, kJointLimit = 2, kJointMotorOn = 4 };
 constexpr float kMaxAngularCorrection = (8.0f / 180.0f * kPi); // b2settings.d:127
 
 struct JointRec {
@@ -37,7 +37,8 @@ struct JointRec {
     float ix, iy, iz, motorImpulse;
     float2 linearImpulse;
     float angularImpulse, springImpulse;
-    int limitState, indexA, indexB, pad0; // indexA / indexB: world-local body indices
+    int limitState, indexA, indexB; // indexA / indexB: world-local body indices
+    int pad0;                       // mark of the island search of a world searched in global memory
     // solver temporaries
     float2 localCenterA, localCenterB;
     float invMassA, invMassB, invIA, invIB;

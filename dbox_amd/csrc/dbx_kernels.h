@@ -33,6 +33,10 @@ hipError_t launch_solve_wave(const Dev &d, int cur, const StepParams &sp, int wo
 // solved by groups of workgroups; the solve launches above skip those worlds
 hipError_t launch_solve_groups(const Dev &d, int cur, const StepParams &sp, const WideBp *wide, int nwide,
                                int ldsBytes, bool lead, hipStream_t s);
+// the tier's worlds that have joints (the launches above skip them)
+size_t solve_joint_lds_bytes(int bodies, int constraints, int joints);
+hipError_t launch_solve_joint(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, int ldsBytes,
+                              bool lead, hipStream_t s);
 size_t broadphase_scratch_bytes(int proxies);
 
 // A world whose broadphase scratch does not fit in one workgroup's LDS: its pairs

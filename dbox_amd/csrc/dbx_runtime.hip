@@ -641,6 +641,8 @@ struct Tier {
     hipEvent_t done = nullptr;
     hipEvent_t t0 = nullptr, t1 = nullptr; // chain timing while autotuning
     bool own = false;         // stream and event created for this tier
+    int jointLds = 0;         // LDS of its joint solve (0: no world of it has joints)
+    int jointWorlds = 0;      // worlds with joints
     int wideFirst = 0, wideCount = 0; // its worlds whose broadphase runs device-wide (range in the handle's list)
 };
 
@@ -1046,6 +1048,10 @@ dbx_status dbx_finalize(dbx_handle *h) {
             T.wideFirst = (int)h->wide.size();
             for (int i = T.first; i < T.first + T.count; ++i) {
                 WorldDesc &D = h->W[order[i]];
+                T.jointWorlds += D.jointCount > 0 ? 1 : 0;
+                if (D.jointCount > 0) // room for two solved contacts per fixture
+                    T.jointLds = std::max(T.jointLds, (int)std::min<size_t>(h->ldsMax - 1024,
+                                                          solve_joint_lds_bytes(D.bodyCount, 2 * D.fixCount, D.jointCount)));
                 if (broadphase_scratch_bytes(D.fixCount) <= (size_t)lds1) continue;
                 D.pad |= 2;
                 WideBp b{};
@@ -1334,8 +1340,13 @@ static dbx_status step_tier(dbx_handle *h, int t, const StepParams &sp, uint32_t
         // worlds too big for LDS (all with the device-wide broadphase): their levels
         // (hundreds of constraints wide in a 20,000-body container) are swept from
         // global memory by a 256-thread workgroup, level batches separated by barriers.
-        if (ordered && T.wideCount < T.count) DBX_HIP(h, launch_solve_wave(d, cout, sp, T.first, T.count, solve_waves(h, T, lead), lds1, lead, s));
-        else DBX_HIP(h, launch_solve(d, cout, sp, T.first, T.count, ordered ? 256 : T.block, ordered ? lds1 : 0, lead, s));
+        if (T.jointWorlds < T.count) {
+            if (ordered && T.wideCount < T.count)
+                DBX_HIP(h, launch_solve_wave(d, cout, sp, T.first, T.count, solve_waves(h, T, lead), lds1, lead, s));
+            else
+                DBX_HIP(h, launch_solve(d, cout, sp, T.first, T.count, ordered ? 256 : T.block, ordered ? lds1 : 0, lead, s));
+        }
+        if (T.jointLds) DBX_HIP(h, launch_solve_joint(d, cout, sp, T.first, T.count, T.jointLds, lead, s));
         if (ordered && T.wideCount && d.iwParent && (sp.flags & kStepGrouped))
             DBX_HIP(h, launch_solve_groups(d, cout, sp, wide, T.wideCount, lds1, lead, s));
         if (timed) (void)hipEventRecord(ev[3], s);
