@@ -149,6 +149,8 @@ constexpr uint32_t kStepGrouped = 1u << 8;
 constexpr uint32_t kStepPiped = 1u << 9;
 // With kStepPiped: overlap the sweeps even where the schedule says it gains little.
 constexpr uint32_t kStepPipedAlways = 1u << 10;
+// StepParams.flags bit: the batches are colours, not levels of the reference's order.
+constexpr uint32_t kStepColoured = 1u << 11;
 
 struct JointRec; // dbx_joints.h
 

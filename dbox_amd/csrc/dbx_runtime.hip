@@ -1336,13 +1336,13 @@ static dbx_status step_tier(dbx_handle *h, int t, const StepParams &sp, uint32_t
         DBX_HIP(h, launch_islands(d, cout, ordered, T.first, T.count, lds1, lead, s));
         if (ordered && T.wideCount && d.iwParent) DBX_HIP(h, launch_islands_wide(d, cout, wide, T.wideCount, s));
         if (timed) (void)hipEventRecord(ev[2], s);
-        // Exact order: one wave per world with the state in LDS, except for a tier of
-        // worlds too big for LDS (all with the device-wide broadphase): their levels
-        // (hundreds of constraints wide in a 20,000-body container) are swept from
-        // global memory by a 256-thread workgroup, level batches separated by barriers.
+        // Solved with the state in LDS, except for a tier of worlds too big for that (all
+        // with the device-wide broadphase): island groups in the exact order, colour
+        // batches from global memory in the coloured mode.
         if (T.jointWorlds < T.count) {
-            if (ordered && T.wideCount < T.count)
-                DBX_HIP(h, launch_solve_wave(d, cout, sp, T.first, T.count, solve_waves(h, T, lead), lds1, lead, s));
+            if (T.wideCount < T.count)
+                DBX_HIP(h, launch_solve_wave(d, cout, sp, T.first, T.count,
+                                             ordered ? solve_waves(h, T, lead) : std::min(T.block / 64, 8), lds1, lead, s));
             else
                 DBX_HIP(h, launch_solve(d, cout, sp, T.first, T.count, ordered ? 256 : T.block, ordered ? lds1 : 0, lead, s));
         }
@@ -1504,6 +1504,7 @@ dbx_status dbx_step(dbx_handle *h, float dt, int32_t vel, int32_t pos, uint32_t 
         sp.flags |= kStepGrouped;
     if ((flags & DBX_STEP_ORDERED) && !getenv("DBX_SWEEPS_SEQUENTIAL"))
         sp.flags |= kStepPiped | (getenv("DBX_SWEEPS_OVERLAP_ALWAYS") ? kStepPipedAlways : 0u);
+    if (!(flags & DBX_STEP_ORDERED)) sp.flags |= kStepColoured;
     if ((flags & (DBX_STEP_LEARNED | DBX_STEP_LOG)) && !h->staged) {
         dbx_status st = stage_mlp(h);
         if (st != DBX_OK) return st;
