@@ -242,22 +242,31 @@ struct Dev {
     const int *toiLogOff;   // nworlds + 1 offsets into toiLog
 };
 
-constexpr int kProfSlots = 4096; // steps between two syncs whose phases are kept (256 KiB)
-constexpr int kProfStamps = 8;
+constexpr int kProfSlots = 4096; // steps between two syncs whose phases are kept (512 KiB)
+constexpr int kProfStamps = 16;
 // Stamp indices of one slot: solveInit from kProfInit0 to kProfVel0, solveVelocity to
 // kProfVel1, solvePosition from kProfPos0 to kProfPos1.
 enum : int { kProfInit0 = 0, kProfVel0 = 1, kProfVel1 = 2, kProfPos0 = 3, kProfPos1 = 4 };
+// The step's phases when it ran as one launch (k_step): Collide from kProfStart, then the
+// ends of Collide, island search, solve, broadphase and continuous pass.
+enum : int { kProfStart = 5, kProfCollided = 6, kProfSearched = 7, kProfSolved = 8, kProfPaired = 9, kProfEnd = 10 };
 
 // Phase stamps of the island solve of the largest world (the lead tier's first
-// workgroup): the first stamp takes a slot, the others write into it.
+// workgroup): start or begin takes a slot, the others write into it.
 struct ProfStamp {
     unsigned long long *slot = nullptr;
-    __device__ __forceinline__ void begin(const Dev &d, bool lead) {
-        if (lead && d.prof) {
-            const unsigned long long k = atomicAdd(d.prof, 1ull) % (unsigned long long)kProfSlots;
-            slot = d.prof + kProfStamps * (k + 1);
-            slot[kProfInit0] = wall_clock64();
-        }
+    __device__ __forceinline__ void take(const Dev &d, bool lead) {
+        if (slot || !lead || !d.prof) return;
+        const unsigned long long k = atomicAdd(d.prof, 1ull) % (unsigned long long)kProfSlots;
+        slot = d.prof + kProfStamps * (k + 1);
+    }
+    __device__ __forceinline__ void start(const Dev &d, bool lead) { // the step's, when one launch runs all of it
+        take(d, lead);
+        at(kProfStart);
+    }
+    __device__ __forceinline__ void begin(const Dev &d, bool lead) { // the island solve's
+        take(d, lead);
+        at(kProfInit0);
     }
     __device__ __forceinline__ void at(int i) const {
         if (slot) slot[i] = wall_clock64();

@@ -33,6 +33,16 @@ hipError_t launch_solve_wave(const Dev &d, int cur, const StepParams &sp, int wo
 // solved by groups of workgroups; the solve launches above skip those worlds
 hipError_t launch_solve_groups(const Dev &d, int cur, const StepParams &sp, const WideBp *wide, int nwide,
                                int ldsBytes, bool lead, hipStream_t s);
+// The phases named by `what` of a step of worlds that fit one workgroup (at most
+// kStepBodies bodies), in one launch: what the launches above do in as many.
+// ldsBytes: at least step_lds_bytes().
+// Larger worlds gain little from fewer launches (a pyramid of 121 bodies: 700 us a step in
+// a launch per phase, 690 in one) and more from the eight waves of their own solve.
+constexpr int kStepBodies = 128;
+enum : int { kStepCollide = 1, kStepSolve = 2, kStepOrdered = 4, kStepToi = 8 };
+int step_lds_bytes();
+hipError_t launch_step(const Dev &d, int cin, const StepParams &sp, int worldOffset, int nworlds, int ldsBytes, int what,
+                       bool lead, hipStream_t s);
 // the tier's worlds that have joints (the launches above skip them)
 size_t solve_joint_lds_bytes(int bodies, int constraints, int joints);
 hipError_t launch_solve_joint(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, int ldsBytes,

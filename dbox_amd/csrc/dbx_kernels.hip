@@ -174,14 +174,9 @@ __device__ void process_contact(Contact &c, int pos, const int *__restrict__ fbo
     }
 }
 
-// kLead marks the launch of the lead tier (the largest worlds, which set the
-// step time); the two instantiations differ only in name, so that profiles
-// report the lead tier on its own.
-template <bool kLead>
-__global__ void k_collide(Dev d, int cur, int worldOffset, int ldsBytes) {
-    extern __shared__ __align__(16) char lds[];
+// Collide of one world by a workgroup (first: the launch order's first world).
+__device__ __forceinline__ void collide_world(const Dev &d, int cur, int w, bool first, char *lds, int ldsBytes) {
     __shared__ int s_tmp[kMaxBlock / 64 + 1];
-    const int w = d.order[worldOffset + blockIdx.x];
     const WorldDesc wd = d.W[w];
     const int n = d.S[w].contactCount;
     Contact *src = d.cont[cur] + wd.contactBase;
@@ -197,7 +192,7 @@ __global__ void k_collide(Dev d, int cur, int worldOffset, int ldsBytes) {
     int *wake = d.wake + wd.bodyBase;
     const int nb = wd.bodyCount;
     const int tid = threadIdx.x, BS = blockDim.x;
-    const bool timed = d.ktime && worldOffset + blockIdx.x == 0 && tid == 0;
+    const bool timed = d.ktime && first && tid == 0;
     if (timed) d.ktime[16] = __builtin_amdgcn_s_memtime();
 
     // a world too big for one workgroup (pad bit 1) had its first pass done by
@@ -339,6 +334,15 @@ __global__ void k_collide(Dev d, int cur, int worldOffset, int ldsBytes) {
         d.S[w].adjContacts = m;
     }
     if (timed) d.ktime[21] = __builtin_amdgcn_s_memtime();
+}
+
+// kLead marks the launch of the lead tier (the largest worlds, which set the
+// step time); the two instantiations differ only in name, so that profiles
+// report the lead tier on its own.
+template <bool kLead>
+__global__ void k_collide(Dev d, int cur, int worldOffset, int ldsBytes) {
+    extern __shared__ __align__(16) char lds[];
+    collide_world(d, cur, d.order[worldOffset + blockIdx.x], worldOffset + blockIdx.x == 0, lds, ldsBytes);
 }
 
 // ---------------------------------------------------------------------------
@@ -1185,10 +1189,8 @@ __global__ __launch_bounds__(256) void k_iw_scatter(Dev d, int w) {
 
 // The lead tier runs four waves per world: they share the staging and output
 // passes, the search itself runs on wave 0.  Other tiers run one wave per world.
-template <bool kLead>
-__global__ __launch_bounds__(256) void k_islands(Dev d, int cur, int ordered, int worldOffset, int ldsBytes) {
-    extern __shared__ __align__(16) char lds[];
-    const int w = d.order[worldOffset + blockIdx.x];
+__device__ __forceinline__ void islands_world(const Dev &d, int cur, int ordered, int worldOffset, int w, char *lds,
+                                              int ldsBytes) {
     const WorldDesc wd = d.W[w];
     const int nb = wd.bodyCount;
     const int m = d.S[w].contactCount;
@@ -1199,6 +1201,11 @@ __global__ __launch_bounds__(256) void k_islands(Dev d, int cur, int ordered, in
         island_search(d, cur, ordered, worldOffset, w, wd, nb, m, isl_carve(lds, nb, m));
     else
         island_search(d, cur, ordered, worldOffset, w, wd, nb, m, isl_carve(d.islScratch + wd.islScratchBase, nb, m));
+}
+template <bool kLead>
+__global__ __launch_bounds__(256) void k_islands(Dev d, int cur, int ordered, int worldOffset, int ldsBytes) {
+    extern __shared__ __align__(16) char lds[];
+    islands_world(d, cur, ordered, worldOffset, d.order[worldOffset + blockIdx.x], lds, ldsBytes);
 }
 
 // ---------------------------------------------------------------------------
@@ -2517,7 +2524,7 @@ __device__ __forceinline__ int island_at(const int4 *isl, int n, int at) {
 // kJoints: the world has joints (k_solve_joint).
 template <bool kJoints>
 __device__ __forceinline__ void solve_world_global(const Dev &d, int cur, const StepParams &sp, int w, bool lead,
-                                                   char *lds, int ldsBytes, int g = 0, int G = 1) {
+                                                   char *lds, int ldsBytes, ProfStamp prof, int g = 0, int G = 1) {
     __shared__ float s_res;
     const WorldDesc wd = d.W[w];
     const int nb = wd.bodyCount, nf = wd.fixCount;
@@ -2615,9 +2622,7 @@ __device__ __forceinline__ void solve_world_global(const Dev &d, int cur, const 
         }
     }
     __syncthreads();
-    ProfStamp prof;
-    lead = lead && g == 0;
-    if (tid == 0) prof.begin(d, lead);
+    if (tid == 0) prof.begin(d, lead && g == 0);
 
     // The compact LDS path when the constrained bodies fit (no joints, no learned
     // warm start or logging, which address bodies by their world index).  With
@@ -3011,7 +3016,7 @@ __global__ __launch_bounds__(256) void k_solve(Dev d, int cur, StepParams sp, in
     extern __shared__ __align__(16) char lds[];
     const int w = d.order[worldOffset + blockIdx.x];
     if (solve_grouped(d, sp, d.W[w]) || d.W[w].jointCount > 0) return;
-    solve_world_global<false>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, ldsBytes);
+    solve_world_global<false>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, ldsBytes, ProfStamp{});
 }
 
 // The worlds of a tier that have joints, in either solver mode: one island per lane in
@@ -3025,7 +3030,7 @@ __global__ __launch_bounds__(256) void k_solve_joint(Dev d, int cur, StepParams 
     extern __shared__ __align__(16) char lds[];
     const int w = d.order[worldOffset + blockIdx.x];
     if (d.W[w].jointCount == 0) return;
-    solve_world_global<true>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, ldsBytes);
+    solve_world_global<true>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, ldsBytes, ProfStamp{});
 }
 
 // One big world's islands on G workgroups, each solving the islands that hold a
@@ -3033,7 +3038,7 @@ __global__ __launch_bounds__(256) void k_solve_joint(Dev d, int cur, StepParams 
 template <bool kLead>
 __global__ __launch_bounds__(256) void k_solve_grp(Dev d, int cur, StepParams sp, int w, int G, int ldsBytes, int lead) {
     extern __shared__ __align__(16) char lds[];
-    solve_world_global<false>(d, cur, sp, w, lead != 0, lds, ldsBytes, blockIdx.x, G);
+    solve_world_global<false>(d, cur, sp, w, lead != 0, lds, ldsBytes, ProfStamp{}, blockIdx.x, G);
 }
 
 // One to eight waves per world (solve_waves in the runtime): the passes over bodies
@@ -3042,10 +3047,8 @@ __global__ __launch_bounds__(256) void k_solve_grp(Dev d, int cur, StepParams sp
 // (kStepColoured) every thread solves a constraint of each colour from
 // LDS; from global memory 256 containers' largest world took 190 us a step, so 128.
 constexpr int kMaxSolveWaves = 8;
-template <bool kLead>
-__global__ __launch_bounds__(64 * kMaxSolveWaves) void k_solve_wave(Dev d, int cur, StepParams sp, int worldOffset, int ldsBytes) {
-    extern __shared__ __align__(16) char lds[];
-    const int w = d.order[worldOffset + blockIdx.x];
+__device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const StepParams &sp, int worldOffset, int w,
+                                                 char *lds, int ldsBytes, ProfStamp prof) {
     const WorldDesc wd = d.W[w];
     if (solve_grouped(d, sp, wd)) return;
     const int nb = wd.bodyCount, nf = wd.fixCount;
@@ -3055,7 +3058,7 @@ __global__ __launch_bounds__(64 * kMaxSolveWaves) void k_solve_wave(Dev d, int c
     if (wd.jointCount > 0) return; // k_solve_joint
     const bool coloured = (sp.flags & kStepColoured) != 0;
     if (solve_lds_bytes(nb, nc, nbatch, nisl) > (size_t)ldsBytes) {
-        solve_world_global<false>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, coloured ? 0 : ldsBytes);
+        solve_world_global<false>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, coloured ? 0 : ldsBytes, prof);
         return;
     }
     const int tid = threadIdx.x, BS = blockDim.x, lane = tid & 63, wave = tid >> 6;
@@ -3160,7 +3163,6 @@ __global__ __launch_bounds__(64 * kMaxSolveWaves) void k_solve_wave(Dev d, int c
         Lvel[b] = make_float4(vx, vy, wv, vw);
     }
     __syncthreads();
-    ProfStamp prof;
     if (tid == 0) prof.begin(d, worldOffset + blockIdx.x == 0);
     // Constraints are stored in schedule order (slot j holds constraint sched[j]),
     // so a level's constraints are a contiguous range of slots.
@@ -3488,6 +3490,11 @@ __global__ __launch_bounds__(64 * kMaxSolveWaves) void k_solve_wave(Dev d, int c
         d.ktime[9] = __builtin_amdgcn_s_memtime();
         d.ktime[13] = __builtin_amdgcn_s_memrealtime();
     }
+}
+template <bool kLead>
+__global__ __launch_bounds__(64 * kMaxSolveWaves) void k_solve_wave(Dev d, int cur, StepParams sp, int worldOffset, int ldsBytes) {
+    extern __shared__ __align__(16) char lds[];
+    solve_wave_world(d, cur, sp, worldOffset, d.order[worldOffset + blockIdx.x], lds, ldsBytes, ProfStamp{});
 }
 
 // ---------------------------------------------------------------------------
@@ -3858,11 +3865,8 @@ __device__ __forceinline__ void add_pair_create(int fa, int fb, int slot, const 
     }
 }
 
-template <bool kLead>
-__global__ void k_broadphase(Dev d, int cur, int worldOffset, int ldsBytes) {
-    extern __shared__ __align__(16) char lds[];
+__device__ __forceinline__ void broadphase_world(const Dev &d, int cur, int w, bool first, char *lds, int ldsBytes) {
     __shared__ int s_tmp[kMaxBlock / 64 + 1];
-    const int w = d.order[worldOffset + blockIdx.x];
     const WorldDesc wd = d.W[w];
     const int nf = wd.fixCount;
     const float4 *fat = d.ffat + wd.fixBase;
@@ -3880,7 +3884,7 @@ __global__ void k_broadphase(Dev d, int cur, int worldOffset, int ldsBytes) {
     const int *adjOff = d.adjOff + wd.bodyBase, *adjCnt = d.adjCnt + wd.bodyBase;
     const int2 *adj = d.adjList + 2 * wd.contactBase;
     const int tid = threadIdx.x, BS = blockDim.x;
-    const bool timed = d.ktime && worldOffset + blockIdx.x == 0 && tid == 0;
+    const bool timed = d.ktime && first && tid == 0;
     if (timed) d.ktime[22] = __builtin_amdgcn_s_memtime();
     if (wd.pad & 2) { // pairs found and added over the whole device (k_bpw_*, k_bw_*)
         if (timed) d.ktime[23] = d.ktime[24] = d.ktime[22];
@@ -3938,6 +3942,11 @@ __global__ void k_broadphase(Dev d, int cur, int worldOffset, int ldsBytes) {
         d.S[w].pairCount = total;
     }
     if (timed) d.ktime[24] = __builtin_amdgcn_s_memtime();
+}
+template <bool kLead>
+__global__ void k_broadphase(Dev d, int cur, int worldOffset, int ldsBytes) {
+    extern __shared__ __align__(16) char lds[];
+    broadphase_world(d, cur, d.order[worldOffset + blockIdx.x], worldOffset + blockIdx.x == 0, lds, ldsBytes);
 }
 
 // ---------------------------------------------------------------------------
@@ -4563,21 +4572,39 @@ __global__ __launch_bounds__(256) void k_tl_link(Dev d, int w, const int *lcnt, 
     }
 }
 
-template <bool kLead>
-__global__ __launch_bounds__(256) void k_toi(Dev d, int cur, StepParams sp, int worldOffset) {
-    __shared__ int s_ibod[2 * kMaxToiContacts], s_icon[kMaxToiContacts];
-    __shared__ VelCon s_vc[kMaxToiContacts];
-    __shared__ PosCon s_pc[kMaxToiContacts];
-    __shared__ float4 s_imp[kMaxToiContacts];
-    __shared__ unsigned long long s_pairs[kToiPairCap];
-    __shared__ SweepSnap s_snap[kToiListCap];
-    __shared__ int s_woken[kToiListCap], s_movedList[kToiListCap], s_dirty[kToiDirtyCap];
-    __shared__ ToiLists s_L;
-    __shared__ float2 s_verts[(kLead ? 256 : 64) * 2 * kMaxPolygonVertices]; // per thread: the two proxies of one TOI
-    __shared__ float s_bestA[4];
-    __shared__ int s_bestPos[4], s_err;
-    __shared__ int s_nb, s_np, s_n, s_nsnap, s_nmoved, s_ncand;
-    const int w = d.order[worldOffset + blockIdx.x];
+// What the pass keeps in LDS; kThreads: the workgroup's threads at most.
+template <int kThreads>
+struct ToiShared {
+    VelCon vc[kMaxToiContacts];
+    PosCon pc[kMaxToiContacts];
+    float4 imp[kMaxToiContacts];
+    unsigned long long pairs[kToiPairCap];
+    SweepSnap snap[kToiListCap];
+    float2 verts[kThreads * 2 * kMaxPolygonVertices]; // per thread: the two proxies of one TOI
+    int ibod[2 * kMaxToiContacts], icon[kMaxToiContacts];
+    int woken[kToiListCap], movedList[kToiListCap], dirty[kToiDirtyCap];
+    ToiLists L;
+    float bestA[4];
+    int bestPos[4], err, nb, np, n, nsnap, nmoved, ncand;
+};
+template <int kThreads>
+__device__ __forceinline__ void toi_pass(const Dev &d, int cur, const StepParams &sp, int worldOffset, int w,
+                                         ToiShared<kThreads> &T) {
+    auto &s_vc = T.vc;
+    auto &s_pc = T.pc;
+    auto &s_imp = T.imp;
+    auto &s_pairs = T.pairs;
+    auto &s_snap = T.snap;
+    auto &s_verts = T.verts;
+    auto &s_ibod = T.ibod;
+    auto &s_icon = T.icon;
+    auto &s_woken = T.woken;
+    auto &s_movedList = T.movedList;
+    auto &s_dirty = T.dirty;
+    auto &s_L = T.L;
+    auto &s_bestA = T.bestA;
+    auto &s_bestPos = T.bestPos;
+    int &s_err = T.err, &s_nb = T.nb, &s_np = T.np, &s_n = T.n, &s_nsnap = T.nsnap, &s_nmoved = T.nmoved, &s_ncand = T.ncand;
     const WorldDesc wd = d.W[w];
     // the lead tier runs four waves per world, the other tiers one; the events
     // themselves run on thread 0
@@ -4874,6 +4901,51 @@ __global__ __launch_bounds__(256) void k_toi(Dev d, int cur, StepParams sp, int 
         d.ktime[35] = __builtin_amdgcn_s_memtime();
     }
 }
+template <bool kLead>
+__global__ __launch_bounds__(256) void k_toi(Dev d, int cur, StepParams sp, int worldOffset) {
+    __shared__ ToiShared<(kLead ? 256 : 64)> T;
+    toi_pass(d, cur, sp, worldOffset, d.order[worldOffset + blockIdx.x], T);
+}
+
+// ---------------------------------------------------------------------------
+// The whole step of a small world by one workgroup in one launch (or, of a split step,
+// what follows Collide): the phases above one after the other.  For worlds of up to
+// kStepBodies bodies the launches of the separate kernels, the events between them
+// and the wait of every world for the slowest at each of them cost as much as the
+// work.  Containers with continuous physics, us a step in a launch per phase and in one:
+// 1 world of 4 bodies 83 and 57, of 125 bodies 243 and 215; 256 worlds of 40 bodies 223
+// and 177, of 125 bodies 353 and 272.  Its registers leave room for one workgroup per CU,
+// so a second round of workgroups loses what it gains: 512 worlds of 40 bodies take 302
+// and 341, of 125 bodies 477 and 541.
+// ---------------------------------------------------------------------------
+template <bool kLead>
+__global__ __launch_bounds__(256) void k_step(Dev d, int cin, StepParams sp, int worldOffset, int ldsBytes, int what) {
+    extern __shared__ __align__(16) char lds[];
+    const int w = d.order[worldOffset + blockIdx.x], cout = cin ^ 1;
+    const bool first = worldOffset + blockIdx.x == 0;
+    ProfStamp prof;
+    if (threadIdx.x == 0 && (what & kStepSolve)) prof.start(d, first);
+    if (what & kStepCollide) {
+        collide_world(d, cin, w, first, lds, ldsBytes);
+        __syncthreads();
+    }
+    if (!(what & kStepSolve)) return;
+    prof.at(kProfCollided);
+    islands_world(d, cout, (what & kStepOrdered) ? 1 : 0, worldOffset, w, lds, ldsBytes);
+    __syncthreads();
+    prof.at(kProfSearched);
+    if (d.W[w].jointCount > 0) solve_world_global<true>(d, cout, sp, w, first, lds, ldsBytes, prof);
+    else solve_wave_world(d, cout, sp, worldOffset, w, lds, ldsBytes, prof);
+    __syncthreads();
+    prof.at(kProfSolved);
+    broadphase_world(d, cout, w, first, lds, ldsBytes);
+    __syncthreads();
+    prof.at(kProfPaired);
+    if (what & kStepToi) toi_pass(d, cout, sp, worldOffset, w, *reinterpret_cast<ToiShared<256> *>(lds));
+    __syncthreads();
+    prof.at(kProfEnd);
+}
+
 
 // ---------------------------------------------------------------------------
 // Device-wide broadphase of one big world: the pair set and order of bp_pairs
@@ -5707,6 +5779,9 @@ static hipError_t configure_tier(int maxDynamicLds) {
     e = hipFuncSetAttribute((const void *)k_solve_grp<kLead>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             maxDynamicLds - 1024);
     if (e != hipSuccess) return e;
+    e = hipFuncSetAttribute((const void *)k_step<kLead>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            maxDynamicLds - 1024);
+    if (e != hipSuccess) return e;
     e = hipFuncSetAttribute((const void *)k_solve_joint<kLead>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             maxDynamicLds - 1024);
     if (e != hipSuccess) return e;
@@ -5770,6 +5845,14 @@ hipError_t launch_solve_wave(const Dev &d, int cur, const StepParams &sp, int wo
     if (nworlds <= 0) return hipSuccess;
     if (waves < 1 || waves > kMaxSolveWaves) return hipErrorInvalidValue;
     DBX_LAUNCH(k_solve_wave, lead, dim3(nworlds), dim3(64 * waves), ldsBytes, s, d, cur, sp, worldOffset, ldsBytes);
+    return hipGetLastError();
+}
+int step_lds_bytes() { return (int)isl_align(sizeof(ToiShared<256>)); }
+hipError_t launch_step(const Dev &d, int cin, const StepParams &sp, int worldOffset, int nworlds, int ldsBytes, int what,
+                       bool lead, hipStream_t s) {
+    if (nworlds <= 0) return hipSuccess;
+    if (ldsBytes < step_lds_bytes()) return hipErrorInvalidValue;
+    DBX_LAUNCH(k_step, lead, dim3(nworlds), dim3(256), ldsBytes, s, d, cin, sp, worldOffset, ldsBytes, what);
     return hipGetLastError();
 }
 size_t solve_joint_lds_bytes(int bodies, int constraints, int joints) {

@@ -642,6 +642,7 @@ struct Tier {
     hipEvent_t t0 = nullptr, t1 = nullptr; // chain timing while autotuning
     bool own = false;         // stream and event created for this tier
     int jointLds = 0;         // LDS of its joint solve (0: no world of it has joints)
+    int stepLds = 0;          // LDS of its one-launch step (0: a launch per phase)
     int jointWorlds = 0;      // worlds with joints
     int wideFirst = 0, wideCount = 0; // its worlds whose broadphase runs device-wide (range in the handle's list)
 };
@@ -697,6 +698,7 @@ struct dbx_handle {
     dbx_profile prof{};             // last step
     void *noallocScratch = nullptr; // device address of `scratch` on this handle's GPU
     std::vector<char> ringSolved;   // per ring entry: the step ran the island solve (dt > 0)
+    std::vector<char> ringOne;      // per ring entry: the lead tier's step was one launch (its phases are stamped)
     unsigned long long profSeen = 0; // phase-stamp slots of the solve kernels already read
     // pinned host memory that kernels write read-backs into (read) and take body writes
     // from (write, filled from writeAt on since the stream was last known to be idle)
@@ -1063,6 +1065,13 @@ dbx_status dbx_finalize(dbx_handle *h) {
             }
             T.wideCount = (int)h->wide.size() - T.wideFirst;
         }
+        // One launch per step for tiers of small worlds while every world has a CU of its
+        // own (both sides measured at k_step).
+        for (Tier &T : tiers) {
+            const int lds = std::max({T.lds, T.jointLds, step_lds_bytes()});
+            if (T.wideCount == 0 && T.bodies <= kStepBodies && lds <= h->ldsMax - 1024 && nw <= h->cuCount)
+                T.stepLds = lds;
+        }
         DBX_HIP(h, create_tier_streams(h, tiers));
         h->tiers = tiers;
         if (getenv("DBX_VERBOSE"))
@@ -1327,6 +1336,13 @@ static dbx_status step_tier(dbx_handle *h, int t, const StepParams &sp, uint32_t
     const WideBp *wide = T.wideCount ? &h->wide[T.wideFirst] : nullptr;
     if ((part & 1) && findNew) // FindNewContacts when fixtures were added (b2world.d:372-376)
         DBX_HIP(h, launch_broadphase(d, cin, T.first, T.count, lds1, T.block, lead, s, wide, T.wideCount));
+    if (T.stepLds) {
+        const int what = ((part & 2) ? kStepCollide : 0) | ((part & 4) && sp.dt > 0.0f ? kStepSolve : 0) |
+                         ((flags & DBX_STEP_ORDERED) ? kStepOrdered : 0) | ((flags & DBX_STEP_CCD) ? kStepToi : 0);
+        if (what & (kStepCollide | kStepSolve))
+            DBX_HIP(h, launch_step(d, cin, sp, T.first, T.count, T.stepLds, what, lead, s));
+        return DBX_OK;
+    }
     if (part & 2) DBX_HIP(h, launch_collide(d, cin, T.first, T.count, lds1, T.block, lead, s, wide, T.wideCount));
     if (!(part & 4)) return DBX_OK;
     const bool timed = lead && ev; // phase events: lead tier, eager steps only
@@ -1519,6 +1535,7 @@ dbx_status dbx_step(dbx_handle *h, float dt, int32_t vel, int32_t pos, uint32_t 
         }
         h->ringGraph.push_back(0);
         h->ringSolved.push_back(0);
+        h->ringOne.push_back(0);
     }
     hipEvent_t *ev = &h->ring[kStepEvents * h->ringUsed];
     h->d.mlp = mlp_dev(h->mlp);
@@ -1581,6 +1598,7 @@ dbx_status dbx_step(dbx_handle *h, float dt, int32_t vel, int32_t pos, uint32_t 
     }
     if (st != DBX_OK) return st;
     h->ringSolved[h->ringUsed] = dt > 0.0f;
+    h->ringOne[h->ringUsed] = h->tiers[0].stepLds != 0;
     if (timeTiers && !tuning) {
         DBX_HIP(h, hipStreamSynchronize(h->stream));
         h->tierMs.resize(h->tiers.size(), 0.0);
@@ -1701,6 +1719,8 @@ dbx_status dbx_sync(dbx_handle *h) {
         hipEvent_t *ev = &h->ring[kStepEvents * k];
         float ms[5] = {0, 0, 0, 0, 0}, total = 0.0f;
         float phase[3] = {0, 0, 0};
+        bool phases = !h->ringGraph[k]; // a replayed graph records only the step's ends
+        if (h->ringOne[k]) phases = false;
         if (h->ringSolved[k]) {
             const unsigned long long slot = nextSlot++;
             if (stampsMatch && slot >= firstKept) {
@@ -1709,11 +1729,19 @@ dbx_status dbx_sync(dbx_handle *h) {
                 phase[0] = (float)((double)(t[kProfVel0] - t[kProfInit0]) / perMs);
                 phase[1] = (float)((double)(t[kProfVel1] - t[kProfVel0]) / perMs);
                 phase[2] = (float)((double)(t[kProfPos1] - t[kProfPos0]) / perMs);
+                if (h->ringOne[k]) {
+                    phases = true;
+                    for (int i = 0; i < 5; ++i) ms[i] = (float)((double)(t[kProfStart + 1 + i] - t[kProfStart + i]) / perMs);
+                }
             }
         }
-        if (!h->ringGraph[k]) // a replayed graph records only the step's ends
+        if (phases && !h->ringOne[k])
             for (int i = 0; i < 5; ++i) (void)hipEventElapsedTime(&ms[i], ev[i], ev[i + 1]);
         (void)hipEventElapsedTime(&total, ev[0], ev[6]);
+        if (h->ringOne[k] && !h->ringSolved[k] && !h->ringGraph[k]) { // dt = 0: Collide alone
+            phases = true;
+            ms[0] = total;
+        }
         // b2World.Step's fields (b2world.d:397-431): collide; solve = all of b2World.Solve,
         // i.e. the island search, the island solves, SynchronizeFixtures and FindNewContacts
         // (whose share is also broadphase, b2world.d:1102-1123); the island-solve phases
@@ -1738,7 +1766,7 @@ dbx_status dbx_sync(dbx_handle *h) {
         h->sum.broadphase += p.broadphase;
         h->sum.solveTOI += p.solveTOI;
         h->sumSteps++;
-        if (!h->ringGraph[k]) {
+        if (phases) {
             for (int i = 0; i < 5; ++i) h->phaseSum[i] += ms[i];
             h->phaseSteps++;
         }

@@ -191,10 +191,13 @@ typedef struct {
  *              largest world run in one workgroup while the other worlds run beside it
  *   broadphase SynchronizeFixtures + FindNewContacts (b2world.d:1102-1123)
  *   solveTOI   b2World.SolveTOI
- * A step replayed from a hipGraph records step and the three island-solve phases only;
- * split (DBX_STEP_PRESOLVE) steps are not timed.  The island-solve phases of the last
- * 4,096 steps before a dbx_sync are kept; an earlier step of a longer run without a
- * sync reports them as 0. */
+ * Handles of small worlds (no more worlds than the device has compute units, 128 bodies
+ * at most in the largest tier) run a step as one kernel; its phases, collide to
+ * solveTOI, are then timed inside that kernel like the island solve's.
+ * A step replayed from a hipGraph records step and the phases timed inside kernels only;
+ * split (DBX_STEP_PRESOLVE) steps are not timed.  The phases timed inside kernels are
+ * kept for the last 4,096 steps before a dbx_sync; an earlier step of a longer run
+ * without a sync reports them as 0. */
 typedef struct {
     float step, collide, solve, solveInit, solveVelocity, solvePosition, broadphase, solveTOI;
 } dbx_profile;
@@ -306,7 +309,7 @@ dbx_status dbx_profile_read(dbx_handle *h, dbx_profile *out);
  * Test.Step does, examples/demo/framework/test.d:558-578). */
 dbx_status dbx_profile_totals(dbx_handle *h, dbx_profile *sum, int32_t *steps, int32_t reset);
 /* Launch-level timing (no counterpart in the reference): milliseconds of the lead
- * tier's kernels, from HIP events on its stream, summed over the eager steps resolved
+ * tier's phases, from HIP events on its stream (or timed inside its one-launch steps), summed over the eager steps resolved
  * by dbx_sync since the last reset, in the order Collide, island search, island
  * solve, broadphase (SynchronizeFixtures + FindNewContacts), continuous pass; *steps
  * = steps summed.  The other tiers run beside the lead tier. */
