@@ -273,6 +273,24 @@ struct ProfStamp {
     }
 };
 
+// The end of a kernel that wrote pinned host memory: it stores seq to *flag (host
+// memory) once all its data are there.  count: a zeroed device word of the handle.
+struct HostSignal {
+    unsigned *flag;
+    unsigned *count;
+    unsigned seq;
+};
+__device__ __forceinline__ void host_signal(const HostSignal &sig) {
+    __builtin_amdgcn_s_waitcnt(0); // this wave's stores are done
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    __threadfence_system();
+    if (atomicAdd(sig.count, 1u) + 1 != gridDim.x) return;
+    *sig.count = 0;
+    __threadfence_system();
+    __hip_atomic_store(sig.flag, sig.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Order-preserving int image of a float (for atomicMin on floats).
 __device__ __forceinline__ int f2ord(float f) {
     int i = __float_as_int(f);

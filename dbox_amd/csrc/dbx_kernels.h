@@ -97,13 +97,7 @@ hipError_t launch_collide_pairs(const Shape *sa, const float *xa, const Shape *s
 hipError_t launch_max_penetration(const Dev &d, int cur, float *out, hipStream_t s);
 
 // Read-backs and body writes through pinned host memory that the kernels write and
-// read themselves.  Each launch ends by storing `seq` to *flag (host memory) once all
-// its data are there; count: a zeroed device word of the handle.
-struct HostSignal {
-    unsigned *flag;
-    unsigned *count;
-    unsigned seq;
-};
+// read themselves; the last kernel of a read ends with host_signal (dbx_device.h).
 // dbx_body_state records of the bodies [base, base + n)
 hipError_t launch_read_bodies(const Dev &d, int base, int n, void *out, HostSignal sig, hipStream_t s);
 // *head = the world's contact count; its dbx_contact records, newest first, when

@@ -6008,18 +6008,6 @@ hipError_t launch_broadphase(const Dev &d, int cur, int worldOffset, int nworlds
 // before and after: dbx_sync 42 and 9 us, bodies 73 and 12, contacts 39 (count, then
 // rows) and 11, events 74 and 12, dbx_write_bodies 88 and 8 (no longer waited for).
 // ---------------------------------------------------------------------------
-// Ends a kernel that wrote host memory: after the last workgroup's data have left,
-// the sequence number goes to the host's flag.
-__device__ __forceinline__ void host_signal(const HostSignal &sig) {
-    __builtin_amdgcn_s_waitcnt(0); // this wave's stores are done
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    __threadfence_system();
-    if (atomicAdd(sig.count, 1u) + 1 != gridDim.x) return;
-    *sig.count = 0;
-    __threadfence_system();
-    __hip_atomic_store(sig.flag, sig.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
 // Workgroups of 256 threads for n threads' worth of work, at most `most`.
 static unsigned read_grid(size_t n, unsigned most) {
     const size_t g = (n + 255) / 256;

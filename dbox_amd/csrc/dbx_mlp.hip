@@ -43,26 +43,51 @@ __global__ void k_mlp_pack(const float *__restrict__ P, bf16x8 *__restrict__ fra
 }
 
 // ---------------------------------------------------------------------------
-// Batched forward pass: x rows of kMlpFeatStride raw features -> impulses.
+// Batched forward pass: rows of kMlpIn raw features -> impulses, both in pinned host
+// memory.  It is bound by the bus that these cross: 8,192 rows take 23 us, the arithmetic
+// alone 4; a call with gradients of them took 208 us with device buffers allocated, copied
+// and freed in each call, 125 with a copy kernel and a buffer kept, and takes 98.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float2 mlp_output(const MlpDev &m, const f32x4 &y) {
     return make_float2(y[0] * m.norm[kNormOutScale] + m.norm[kNormOutMean],
                        y[1] * m.norm[kNormOutScale + 1] + m.norm[kNormOutMean + 1]);
 }
 
-__global__ __launch_bounds__(64) void k_mlp_forward(MlpDev m, const float *__restrict__ X, int n, float *__restrict__ Y) {
+// Up to 32 rows of kMlpIn floats from pinned host memory to LDS by one wave: 16 rows are
+// whole 64-byte lines, and each crosses the bus once.
+__device__ __forceinline__ void stage_rows(const float *__restrict__ x, int rows, float *buf) {
+    const float4 *src = reinterpret_cast<const float4 *>(x);
+    for (int i = threadIdx.x; i < (rows * kMlpIn + 3) / 4; i += 64) reinterpret_cast<float4 *>(buf)[i] = src[i];
+}
+
+__global__ __launch_bounds__(64) void k_mlp_forward(MlpDev m, const float *__restrict__ X, int n, float *__restrict__ Y,
+                                                    HostSignal sig) {
+    __shared__ __align__(16) float rows[16 * kMlpIn];
     const int lane = threadIdx.x, g = lane >> 4, col = lane & 15;
     for (int base = 16 * blockIdx.x; base < n; base += 16 * gridDim.x) {
         const int p = base + col;
-        const bf16x8 x = mlp_input_operand(m, p < n ? X + (size_t)p * kMlpFeatStride : nullptr, g);
+        __syncthreads();
+        stage_rows(X + (size_t)base * kMlpIn, min(16, n - base), rows);
+        __syncthreads();
+        const bf16x8 x = mlp_input_operand(m, p < n ? rows + col * kMlpIn : nullptr, g);
         MlpFwd F;
         mlp_forward16(m, x, F);
         if (g == 0 && p < n) {
             float2 o = mlp_output(m, F.y);
-            Y[2 * (size_t)p] = o.x;
-            Y[2 * (size_t)p + 1] = o.y;
+            reinterpret_cast<float2 *>(Y)[p] = o;
         }
     }
+    host_signal(sig);
+}
+__global__ __launch_bounds__(256) void k_mlp_take(float *__restrict__ G, float *__restrict__ loss, float *__restrict__ out,
+                                                  HostSignal sig) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    float *p = i < kMlpParams ? G + i : loss;
+    if (i <= kMlpParams) {
+        out[i] = *p;
+        *p = 0.0f;
+    }
+    host_signal(sig);
 }
 
 // ---------------------------------------------------------------------------
@@ -92,9 +117,13 @@ __device__ __forceinline__ bf16x8 lds_row8(const __bf16 *row, int g) {
     return r;
 }
 
+// kRows: the samples are rows 0..B-1 of kMlpIn floats in pinned host memory; otherwise
+// rows of kMlpFeatStride floats in device memory, drawn by the seed.
+template <bool kRows>
 __global__ __launch_bounds__(64) void k_mlp_grad(MlpDev m, const float *__restrict__ X, const float *__restrict__ T,
-                                                 long long n, long long B, uint64_t seed, float *__restrict__ grad,
-                                                 float *__restrict__ loss) {
+                                                 long long n, long long B, float invB, uint64_t seed,
+                                                 float *__restrict__ grad, float *__restrict__ loss) {
+    __shared__ __align__(16) float rows[kRows ? 32 * kMlpIn : 4];
     __shared__ __bf16 xs[16 * kRowPad], dys[16 * kRowPad];
     __shared__ __bf16 h1s[64 * kRowPad], dz1s[64 * kRowPad], h2s[64 * kRowPad], dz2s[64 * kRowPad];
     const int lane = threadIdx.x, g = lane >> 4, col = lane & 15;
@@ -107,16 +136,19 @@ __global__ __launch_bounds__(64) void k_mlp_grad(MlpDev m, const float *__restri
         for (int u = 0; u < 4; ++u) a2[t][u] = zero;
     }
     float gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f, lossAcc = 0.0f;
-    const float invB = 1.0f / (float)B;
     for (int r = lane; r < 16 * kRowPad; r += 64) dys[r] = (__bf16)0.0f;
     const long long rounds = (B + 31) / 32;
     for (long long rd = blockIdx.x; rd < rounds; rd += gridDim.x) {
         __syncthreads();
+        if (kRows) {
+            stage_rows(X + 32 * rd * kMlpIn, (int)(B - 32 * rd < 32 ? B - 32 * rd : 32), rows);
+            __syncthreads();
+        }
         for (int q = 0; q < 2; ++q) {
             const long long b = 32 * rd + 16 * q + col;
             const bool valid = b < B;
-            const long long idx = valid ? sample_index(seed, b, n) : 0;
-            const float *xr = valid ? X + idx * kMlpFeatStride : nullptr;
+            const long long idx = !valid ? 0 : kRows ? b : sample_index(seed, b, n);
+            const float *xr = !valid ? nullptr : kRows ? rows + (16 * q + col) * kMlpIn : X + idx * kMlpFeatStride;
             const bf16x8 x = mlp_input_operand(m, xr, g);
             const int pc = 16 * q + col; // column of this point in the staged rows
 #pragma unroll
@@ -259,6 +291,7 @@ hipError_t mlp_ensure(MlpState &m, hipStream_t s) {
     hipLaunchKernelGGL(k_fill, dim3(8), dim3(256), 0, s, m.grad, (long long)kMlpParams, 0.0f);
     hipLaunchKernelGGL(k_fill, dim3(8), dim3(256), 0, s, m.adam1, (long long)kMlpParams, 0.0f);
     hipLaunchKernelGGL(k_fill, dim3(8), dim3(256), 0, s, m.adam2, (long long)kMlpParams, 0.0f);
+    hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, s, m.loss, 1LL, 0.0f);
     return hipGetLastError();
 }
 
@@ -287,23 +320,29 @@ hipError_t mlp_upload(MlpState &m, const float *params, const float *norm, hipSt
     return hipGetLastError();
 }
 
-hipError_t mlp_forward(MlpState &m, const float *dX, int n, float *dY, hipStream_t s) {
-    if (n <= 0) return hipSuccess;
+hipError_t mlp_forward(MlpState &m, const float *x, int n, float *y, HostSignal sig, hipStream_t s) {
     const int groups = (n + 15) / 16;
-    hipLaunchKernelGGL(k_mlp_forward, dim3(groups < 4096 ? groups : 4096), dim3(64), 0, s, mlp_dev(m), dX, n, dY);
+    hipLaunchKernelGGL(k_mlp_forward, dim3(groups < 4096 ? groups : 4096), dim3(64), 0, s, mlp_dev(m), x, n, y, sig);
     return hipGetLastError();
 }
 
+static dim3 grad_grid(long long batch) {
+    const long long rounds = (batch + 31) / 32;
+    return dim3((unsigned)(rounds < 2048 ? rounds : 2048));
+}
 hipError_t mlp_gradients(MlpState &m, const float *dX, const float *dT, long long n, long long batch, uint64_t seed,
                          float *dLoss, hipStream_t s) {
-    if (!dLoss) {
-        hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, s, m.loss, 1LL, 0.0f);
-        dLoss = m.loss;
-    }
-    const long long rounds = (batch + 31) / 32;
-    const long long waves = rounds < 2048 ? rounds : 2048;
-    hipLaunchKernelGGL(k_mlp_grad, dim3((unsigned)waves), dim3(64), 0, s, mlp_dev(m), dX, dT, n, batch, seed, m.grad,
-                       dLoss);
+    hipLaunchKernelGGL(k_mlp_grad<false>, grad_grid(batch), dim3(64), 0, s, mlp_dev(m), dX, dT, n, batch,
+                       1.0f / (float)batch, seed, m.grad, dLoss);
+    return hipGetLastError();
+}
+hipError_t mlp_gradients_rows(MlpState &m, const float *x, const float *t, long long n, long long total, hipStream_t s) {
+    hipLaunchKernelGGL(k_mlp_grad<true>, grad_grid(n), dim3(64), 0, s, mlp_dev(m), x, t, n, n, 1.0f / (float)total,
+                       (uint64_t)0, m.grad, m.loss);
+    return hipGetLastError();
+}
+hipError_t mlp_take(MlpState &m, float *out, HostSignal sig, hipStream_t s) {
+    hipLaunchKernelGGL(k_mlp_take, dim3(kMlpParams / 256 + 1), dim3(256), 0, s, m.grad, m.loss, out, sig);
     return hipGetLastError();
 }
 
@@ -323,6 +362,7 @@ hipError_t mlp_adam_step(MlpState &m, float lr, hipStream_t s) {
 
 hipError_t mlp_clear_grad(MlpState &m, hipStream_t s) {
     hipLaunchKernelGGL(k_fill, dim3(8), dim3(256), 0, s, m.grad, (long long)kMlpParams, 0.0f);
+    hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, s, m.loss, 1LL, 0.0f);
     return hipGetLastError();
 }
 

@@ -2372,36 +2372,38 @@ dbx_status dbx_mlp_get(dbx_handle *h, float *params, float *norm) {
     return DBX_OK;
 }
 
-// Device copy of n feature rows of DBX_MLP_FEATURES floats, padded to kMlpFeatStride.
-static dbx_status upload_rows(dbx_handle *h, const float *x, int32_t n, float **dX) {
-    std::vector<float> pad((size_t)n * kMlpFeatStride, 0.0f);
-    for (int32_t i = 0; i < n; ++i)
-        for (int j = 0; j < kMlpIn; ++j) pad[(size_t)i * kMlpFeatStride + j] = x[(size_t)i * kMlpIn + j];
-    DBX_HIP(h, hipMalloc((void **)dX, pad.size() * sizeof(float)));
-    hipError_t e = hipMemcpy(*dX, pad.data(), pad.size() * sizeof(float), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        (void)hipFree(*dX);
-        return hip_fail(h, e, "hipMemcpy");
-    }
+// The network's entry points hand their rows to the kernels through pinned memory, at most
+// kMlpChunk at a time: inputs at h->write, results at h->read.
+constexpr int kMlpChunk = 65536;
+// Puts n rows of x (and, if given, of t) into h->write; *px and *pt: where kernels see them.
+static dbx_status put_rows(dbx_handle *h, const float *x, const float *t, int n, const float **px, const float **pt) {
+    const size_t nx = ((size_t)n * kMlpIn + 3) / 4 * 4, nt = t ? 2 * (size_t)n : 0;
+    const size_t bytes = (nx + nt) * sizeof(float);
+    if (h->writeAt) DBX_HIP(h, hipStreamSynchronize(h->stream)); // body writes or the last rows are still read from there
+    DBX_HIP(h, pinned_reserve(h, h->write, bytes));
+    float *host = (float *)h->write.host;
+    memcpy(host, x, (size_t)n * kMlpIn * sizeof(float));
+    if (t) memcpy(host + nx, t, nt * sizeof(float));
+    h->writeAt = bytes;
+    *px = (const float *)h->write.dev;
+    if (t) *pt = *px + nx;
     return DBX_OK;
 }
 
 dbx_status dbx_mlp_forward(dbx_handle *h, const float *x, int32_t n, float *y) {
     if (!h || n < 0 || (n > 0 && (!x || !y))) return DBX_E_INVALID_ARG;
     if (!h->mlp.ready) return fail(h, DBX_E_STATE, "no warm-start network loaded");
-    if (n == 0) return DBX_OK;
     DBX_HIP(h, hipSetDevice(h->cfg.device));
-    DBX_HIP(h, hipStreamSynchronize(h->stream));
-    float *dX = nullptr, *dY = nullptr;
-    dbx_status st = upload_rows(h, x, n, &dX);
-    if (st != DBX_OK) return st;
-    hipError_t e = hipMalloc((void **)&dY, 2 * (size_t)n * sizeof(float));
-    if (e == hipSuccess) e = mlp_forward(h->mlp, dX, n, dY, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e == hipSuccess) e = hipMemcpy(y, dY, 2 * (size_t)n * sizeof(float), hipMemcpyDeviceToHost);
-    (void)hipFree(dX);
-    if (dY) (void)hipFree(dY);
-    if (e != hipSuccess) return hip_fail(h, e, "mlp forward");
+    for (int32_t at = 0; at < n; at += std::min(n - at, kMlpChunk)) {
+        const int m = std::min(n - at, kMlpChunk);
+        const float *px = nullptr;
+        dbx_status st = put_rows(h, x + (size_t)at * kMlpIn, nullptr, m, &px, nullptr);
+        if (st != DBX_OK) return st;
+        st = pinned_read(h, 2 * (size_t)m * sizeof(float),
+                         [&](HostSignal sig) { return mlp_forward(h->mlp, px, m, (float *)h->read.dev, sig, h->stream); });
+        if (st != DBX_OK) return st;
+        memcpy(y + 2 * (size_t)at, h->read.host, 2 * (size_t)m * sizeof(float));
+    }
     return DBX_OK;
 }
 
@@ -2409,21 +2411,24 @@ dbx_status dbx_mlp_gradients(dbx_handle *h, const float *x, const float *t, int3
     if (!h || n <= 0 || !x || !t || !grad) return DBX_E_INVALID_ARG;
     if (!h->mlp.ready) return fail(h, DBX_E_STATE, "no warm-start network loaded");
     DBX_HIP(h, hipSetDevice(h->cfg.device));
-    DBX_HIP(h, hipStreamSynchronize(h->stream));
-    float *dX = nullptr, *dT = nullptr;
-    dbx_status st = upload_rows(h, x, n, &dX);
-    if (st != DBX_OK) return st;
-    hipError_t e = hipMalloc((void **)&dT, 2 * (size_t)n * sizeof(float));
-    if (e == hipSuccess) e = hipMemcpy(dT, t, 2 * (size_t)n * sizeof(float), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = mlp_clear_grad(h->mlp, h->stream);
-    if (e == hipSuccess) e = mlp_gradients(h->mlp, dX, dT, n, n, 0, nullptr, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e == hipSuccess) e = hipMemcpy(grad, h->mlp.grad, kMlpParams * sizeof(float), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && loss) e = hipMemcpy(loss, h->mlp.loss, sizeof(float), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = mlp_clear_grad(h->mlp, h->stream);
-    (void)hipFree(dX);
-    if (dT) (void)hipFree(dT);
-    if (e != hipSuccess) return hip_fail(h, e, "mlp gradients");
+    dbx_status st = DBX_OK;
+    for (int32_t at = 0; at < n && st == DBX_OK; at += std::min(n - at, kMlpChunk)) { // the kernels add up
+        const int m = std::min(n - at, kMlpChunk);
+        const float *px = nullptr, *pt = nullptr;
+        st = put_rows(h, x + (size_t)at * kMlpIn, t + 2 * (size_t)at, m, &px, &pt);
+        if (st != DBX_OK) break;
+        const hipError_t e = mlp_gradients_rows(h->mlp, px, pt, m, n, h->stream);
+        if (e != hipSuccess) st = hip_fail(h, e, "mlp gradients");
+    }
+    if (st == DBX_OK)
+        st = pinned_read(h, (kMlpParams + 1) * sizeof(float),
+                         [&](HostSignal sig) { return mlp_take(h->mlp, (float *)h->read.dev, sig, h->stream); });
+    if (st != DBX_OK) {
+        (void)mlp_clear_grad(h->mlp, h->stream);
+        return st;
+    }
+    memcpy(grad, h->read.host, kMlpParams * sizeof(float));
+    if (loss) *loss = ((const float *)h->read.host)[kMlpParams];
     return DBX_OK;
 }
 

@@ -309,8 +309,8 @@ dbx_status dbx_profile_read(dbx_handle *h, dbx_profile *out);
  * Test.Step does, examples/demo/framework/test.d:558-578). */
 dbx_status dbx_profile_totals(dbx_handle *h, dbx_profile *sum, int32_t *steps, int32_t reset);
 /* Launch-level timing (no counterpart in the reference): milliseconds of the lead
- * tier's phases, from HIP events on its stream (or timed inside its one-launch steps), summed over the eager steps resolved
- * by dbx_sync since the last reset, in the order Collide, island search, island
+ * tier's phases, from HIP events on its stream (or timed inside its one-launch steps),
+ * summed over the eager steps resolved by dbx_sync since the last reset, in the order Collide, island search, island
  * solve, broadphase (SynchronizeFixtures + FindNewContacts), continuous pass; *steps
  * = steps summed.  The other tiers run beside the lead tier. */
 dbx_status dbx_phase_totals(dbx_handle *h, float *ms5, int32_t *steps, int32_t reset);
