@@ -186,6 +186,11 @@ __device__ __forceinline__ Xf mulT(const Xf &A, const Xf &B) {
     C.p = mulT(A.q, sub(B.p, A.p));
     return C;
 }
+// The value on the other lane of a pair (an even lane and the odd lane after it), a DPP
+// quad permutation [1,0,3,2]; both lanes have to be active.
+__device__ __forceinline__ int pair_swap(int x) { return __builtin_amdgcn_mov_dpp(x, 0xb1, 0xf, 0xf, true); }
+__device__ __forceinline__ float pair_swap(float x) { return __int_as_float(pair_swap(__float_as_int(x))); }
+__device__ __forceinline__ float2 pair_swap(float2 x) { return v2(pair_swap(x.x), pair_swap(x.y)); }
 // Transform of a body from its centre of mass c, angle a and local centre lc.
 __device__ __forceinline__ Xf xf_from(float2 c, float a, float2 lc) {
     Xf x;

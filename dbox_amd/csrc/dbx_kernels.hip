@@ -2008,12 +2008,9 @@ __device__ __forceinline__ void velocity_piped(const int *Lbo, const int *Lneed,
 // The position sweeps give each constraint two lanes (an even lane and the odd
 // lane after it), which compute the same constraint except that the even lane
 // evaluates b2Rot.Set of body A's angle and the odd lane of body B's, and the
-// two exchange the results (a DPP quad permutation [1,0,3,2]): each lane then
+// two exchange the results (pair_swap): each lane then
 // holds both rotations for the cost of one.  The two lanes of a pair always take
 // the same branches, so both are active at every exchange.
-__device__ __forceinline__ float pair_swap(float x) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xb1, 0xf, 0xf, true));
-}
 __device__ __forceinline__ void pair_xfs(float2 cA, float aA, float2 lcA, float2 cB, float aB, float2 lcB, Xf &xfA,
                                          Xf &xfB) {
     const bool odd = (threadIdx.x & 1) != 0;
@@ -2139,7 +2136,7 @@ __device__ __forceinline__ void colour_position(const int *Lbo, int nbatch, cons
 // separation; Lver: per island, bit s = first solved by the sweep-s test.
 // The even lane's value of x on both lanes of a pair.
 __device__ __forceinline__ int pair_even(int x) {
-    const int other = __builtin_amdgcn_mov_dpp(x, 0xb1, 0xf, 0xf, true);
+    const int other = pair_swap(x);
     return (threadIdx.x & 1) ? other : x;
 }
 __device__ __forceinline__ void position_level_piped(const PosCon &q, int slot, bool have, int lo, int hi,
@@ -4145,37 +4142,33 @@ __device__ __forceinline__ int toi_status(const ToiWorld &W, const Contact &c, i
     if (!collideA && !collideB) return 0;
     return 2;
 }
+// LDS entries of one thread's proxy; odd, so that the lanes' entries lie in different banks.
+constexpr int kVertStride = kMaxPolygonVertices + 1;
 // The start of each sweep (c0, a0, alpha0) that one contact's TOI sees.
 struct SweepSnap {
     int contact;
     float ax, ay, aa, aalpha, bx, by, ba, balpha;
 };
 // The contact's TOI as a fraction of the step (b2world.d:1221-1238) from the
-// given sweep starts; the sweeps' ends are the bodies' current c and a.  vbuf:
-// this lane's LDS space for the two proxies' vertices.
+// given sweep starts, by a lane pair; the sweeps' ends are the bodies' current c and a.
+// vbuf: this lane's LDS space for one proxy's vertices.
 // It takes the few arrays it reads, not the ToiWorld: a called function that
 // took the world's table by reference would keep a copy of it in scratch memory.
 __device__ __noinline__ float contact_toi(const Shape *shp, const int *fbody, const float4 *bmass, const float4 *bpos,
-                                         int fa, int fb, SweepSnap sn, float2 *vbuf) {
-    const int ba = fbody[fa], bb = fbody[fb];
-    const float4 mA = bmass[ba], mB = bmass[bb], pa = bpos[ba], pb = bpos[bb];
-    Sweep sA, sB;
-    sA.lc = v2(mA.z, mA.w);
-    sA.c0 = v2(sn.ax, sn.ay);
-    sA.a0 = sn.aa;
-    sA.c = v2(pa.x, pa.y);
-    sA.a = pa.z;
-    sA.alpha0 = sn.aalpha;
-    sB.lc = v2(mB.z, mB.w);
-    sB.c0 = v2(sn.bx, sn.by);
-    sB.a0 = sn.ba;
-    sB.c = v2(pb.x, pb.y);
-    sB.a = pb.z;
-    sB.alpha0 = sn.balpha;
-    const float alpha0 = sA.alpha0;
-    const DProxy pA = make_proxy_in(shp + fa, vbuf), pB = make_proxy_in(shp + fb, vbuf + kMaxPolygonVertices);
+                                         int fa, int fb, SweepSnap sn, LdsFloat2 *vbuf) {
+    const bool odd = (threadIdx.x & 1) != 0;
+    const int f = odd ? fb : fa, b = fbody[f];
+    const float4 m = bmass[b], p = bpos[b];
+    Sweep s;
+    s.lc = v2(m.z, m.w);
+    s.c0 = v2(odd ? sn.bx : sn.ax, odd ? sn.by : sn.ay);
+    s.a0 = odd ? sn.ba : sn.aa;
+    s.c = v2(p.x, p.y);
+    s.a = p.z;
+    s.alpha0 = odd ? sn.balpha : sn.aalpha;
+    const float alpha0 = sn.aalpha;
     float beta;
-    const int state = time_of_impact(beta, pA, pB, sA, sB, 1.0f);
+    const int state = time_of_impact(beta, make_proxy_in(shp + f, vbuf), s, 1.0f);
     return state == kToiTouching ? fminr(alpha0 + (1.0f - alpha0) * beta, 1.0f) : 1.0f;
 }
 __device__ __forceinline__ SweepSnap snap_of(const ToiWorld &W, int j) {
@@ -4506,21 +4499,30 @@ __global__ __launch_bounds__(256) void k_toi_wide_bodies(Dev d, int w, int *lcnt
     if (blockIdx.x == 0 && threadIdx.x == 0) d.S[w].toiCand = 0;
 }
 __global__ __launch_bounds__(64) void k_toi_wide_first(Dev d, int cur, int w) {
-    __shared__ float2 s_verts[64 * 2 * kMaxPolygonVertices];
+    __shared__ float2 s_verts[64 * kVertStride];
+    __shared__ int s_need[64];
     const WorldDesc wd = d.W[w];
     const ToiWorld W = toi_world(d, cur, w, wd);
     const int n = d.S[w].contactCount;
     int *cand = d.toiCand + wd.contactBase;
-    for (int i = blockIdx.x * 64 + threadIdx.x; i < n; i += gridDim.x * 64) {
-        int4 t = make_int4(__float_as_int(1.0f), 0, -1, -1);
-        if (toi_status(W, W.cont[i], 0) == 2) {
-            t.x = __float_as_int(contact_toi(W.shp, W.fbody, W.bmass, W.bpos, W.cont[i].fa, W.cont[i].fb,
-                                             snap_of(W, i), s_verts + 2 * kMaxPolygonVertices * threadIdx.x));
-            t.y = kTcToi | kTcCand;
+    const int lane = threadIdx.x;
+    for (int base = blockIdx.x * 64; base < n; base += gridDim.x * 64) {
+        const int i = base + lane;
+        const bool need = i < n && toi_status(W, W.cont[i], 0) == 2;
+        const unsigned long long mask = __builtin_amdgcn_ballot_w64(need);
+        if (i < n && !need) W.tc[i] = make_int4(__float_as_int(1.0f), 0, -1, -1);
+        if (need) s_need[__popcll(mask & ((1ull << lane) - 1ull))] = i;
+        __syncthreads();
+        for (int k = lane >> 1; k < __popcll(mask); k += 32) { // a lane pair per TOI
+            const int j = s_need[k];
+            const float a = contact_toi(W.shp, W.fbody, W.bmass, W.bpos, W.cont[j].fa, W.cont[j].fb, snap_of(W, j),
+                                        (LdsFloat2 *)(s_verts + kVertStride * lane));
+            if (lane & 1) continue;
+            W.tc[j] = make_int4(__float_as_int(a), kTcToi | kTcCand, -1, -1);
             const int slot = atomicAdd(&d.S[w].toiCand, 1);
-            if (slot < wd.contactCap) cand[slot] = i;
+            if (slot < wd.contactCap) cand[slot] = j;
         }
-        W.tc[i] = t;
+        __syncthreads();
     }
 }
 __global__ __launch_bounds__(256) void k_tl_count(Dev d, int cur, int w, int *lcnt) {
@@ -4580,7 +4582,7 @@ struct ToiShared {
     float4 imp[kMaxToiContacts];
     unsigned long long pairs[kToiPairCap];
     SweepSnap snap[kToiListCap];
-    float2 verts[kThreads * 2 * kMaxPolygonVertices]; // per thread: the two proxies of one TOI
+    float2 verts[kThreads * kVertStride]; // per thread: the proxy of one body of a TOI
     int ibod[2 * kMaxToiContacts], icon[kMaxToiContacts];
     int woken[kToiListCap], movedList[kToiListCap], dirty[kToiDirtyCap];
     ToiLists L;
@@ -4609,7 +4611,7 @@ __device__ __forceinline__ void toi_pass(const Dev &d, int cur, const StepParams
     // the lead tier runs four waves per world, the other tiers one; the events
     // themselves run on thread 0
     const int tid = threadIdx.x, BS = blockDim.x, lane = tid & 63, wave = tid >> 6;
-    float2 *verts = s_verts + 2 * kMaxPolygonVertices * tid;
+    LdsFloat2 *verts = (LdsFloat2 *)(s_verts + kVertStride * tid);
     const ToiWorld W = toi_world(d, cur, w, wd);
     const int nb = wd.bodyCount, nf = wd.fixCount;
     int n = d.S[w].contactCount;
@@ -4664,10 +4666,11 @@ __device__ __forceinline__ void toi_pass(const Dev &d, int cur, const StepParams
         __syncthreads();
         const int ne = s_nsnap;
         if (ne > kToiDirtyCap - 256 || (base + 256 >= n && ne > 0)) {
-            for (int k = tid; k < ne; k += BS) {
+            for (int k = tid >> 1; k < ne; k += BS >> 1) { // a lane pair per TOI
                 const int i = s_dirty[k];
                 const float a = contact_toi(W.shp, W.fbody, W.bmass, W.bpos, W.cont[i].fa, W.cont[i].fb,
                                             snap_of(W, i), verts);
+                if (tid & 1) continue;
                 W.tc[i].x = __float_as_int(a);
                 W.tc[i].y = kTcToi | kTcCand;
                 cand[atomicAdd(&s_ncand, 1)] = i;
@@ -4724,11 +4727,12 @@ __device__ __forceinline__ void toi_pass(const Dev &d, int cur, const StepParams
                 }
                 __syncthreads();
                 const int ns = s_nsnap;
-                for (int k = tid; k < ns; k += BS) {
+                for (int k = tid >> 1; k < ns; k += BS >> 1) {
                     const int j = s_snap[k].contact;
                     const float a =
                         contact_toi(W.shp, W.fbody, W.bmass, W.bpos, W.cont[j].fa, W.cont[j].fb, s_snap[k],
                                     verts);
+                    if (tid & 1) continue;
                     const int y = W.tc[j].y;
                     W.tc[j].x = __float_as_int(a);
                     W.tc[j].y = y | kTcToi | kTcCand;

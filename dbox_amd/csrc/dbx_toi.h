@@ -1,7 +1,7 @@
 // dbx_toi.h -- continuous collision for the step kernels: b2Distance (GJK with a
 // simplex cache, src/dbox/collision/b2distance.d:30-707) and b2TimeOfImpact
 // (conservative advancement on separating axes, b2timeofimpact.d:67-530), one
-// shape pair per lane.
+// shape pair per lane pair (b2Distance for the overlap test: per lane).
 //
 // The simplex keeps its three vertices as named members and every access by a
 // run-time index goes through a select, so the whole state stays in registers.
@@ -29,15 +29,28 @@ __device__ __forceinline__ DProxy make_proxy(const Shape *s) {
     p.radius = s->radius;
     return p;
 }
-// The same proxy with its vertices copied to buf (kMaxPolygonVertices entries,
-// LDS), so that the many support and evaluate calls of one TOI read them from
-// LDS instead of global memory; the copies are independent loads.
-__device__ __forceinline__ DProxy make_proxy_in(const Shape *s, float2 *buf) {
-    DProxy p = make_proxy(s);
+// A proxy with its vertices in LDS (kMaxPolygonVertices entries), for the many support
+// and evaluate calls of one TOI.
+typedef float Float2Vec __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) Float2Vec LdsFloat2;
+struct LdsProxy {
+    const LdsFloat2 *v;
+    int count;
+    float radius;
+    __device__ __forceinline__ float2 at(int i) const {
+        const Float2Vec x = v[i];
+        return v2(x.x, x.y);
+    }
+};
+__device__ __forceinline__ LdsProxy make_proxy_in(const Shape *s, LdsFloat2 *buf) {
+    const DProxy g = make_proxy(s);
 #pragma unroll
     for (int i = 0; i < kMaxPolygonVertices; ++i)
-        if (i < p.count) buf[i] = p.v[i];
+        if (i < g.count) buf[i] = Float2Vec{g.v[i].x, g.v[i].y};
+    LdsProxy p;
     p.v = buf;
+    p.count = g.count;
+    p.radius = g.radius;
     return p;
 }
 // GetSupport (b2distance.d:94-111): first vertex of largest dot product.
@@ -47,6 +60,24 @@ __device__ __forceinline__ int support(const DProxy &p, float2 d) {
     for (int i = 1; i < p.count; ++i) {
         const float value = dot(p.v[i], d);
         if (value > bestValue) {
+            best = i;
+            bestValue = value;
+        }
+    }
+    return best;
+}
+// From LDS all entries are read at once, those past the count to no effect: one
+// latency for the whole search instead of one per vertex.
+__device__ __forceinline__ int support(const LdsProxy &p, float2 d) {
+    Float2Vec x[kMaxPolygonVertices];
+#pragma unroll
+    for (int i = 0; i < kMaxPolygonVertices; ++i) x[i] = p.v[i];
+    int best = 0;
+    float bestValue = dot(v2(x[0].x, x[0].y), d);
+#pragma unroll
+    for (int i = 1; i < kMaxPolygonVertices; ++i) {
+        const float value = dot(v2(x[i].x, x[i].y), d);
+        if (i < p.count && value > bestValue) {
             best = i;
             bestValue = value;
         }
@@ -98,17 +129,52 @@ struct Simplex {
     int count;
 };
 
-__device__ __forceinline__ SVert make_svert(const DProxy &pA, const Xf &xfA, int iA, const DProxy &pB, const Xf &xfB,
-                                            int iB) {
-    SVert s;
-    s.iA = iA;
-    s.iB = iB;
-    s.wA = mul(xfA, pA.v[iA]);
-    s.wB = mul(xfB, pB.v[iB]);
-    s.w = sub(s.wB, s.wA);
-    s.a = 0.0f;
-    return s;
-}
+// Two proxies and their transforms on one lane.
+struct LaneShapes {
+    DProxy pA, pB;
+    Xf xfA, xfB;
+    __device__ __forceinline__ SVert vertex(int iA, int iB) const {
+        SVert s;
+        s.iA = iA;
+        s.iB = iB;
+        s.wA = mul(xfA, pA.v[iA]);
+        s.wB = mul(xfB, pB.v[iB]);
+        s.w = sub(s.wB, s.wA);
+        s.a = 0.0f;
+        return s;
+    }
+    __device__ __forceinline__ void supports(float2 d, int &iA, int &iB) const {
+        iA = support(pA, mulT(xfA.q, neg(d)));
+        iB = support(pB, mulT(xfB.q, d));
+    }
+};
+// The same on a lane pair, which takes every branch together: the even lane holds and
+// evaluates body A's side, the odd lane body B's, and the two exchange the results.  A
+// TOI is one long chain of instructions whose transforms (a sine and a cosine in double
+// precision for each body at each time looked at) are most of it; this way it does
+// each body's half only.  64 rooms of 40 projectiles: 586 us a step with a TOI per lane,
+// 560 so.
+struct PairShapes {
+    LdsProxy own;
+    Xf xf;
+    bool odd;
+    __device__ __forceinline__ SVert vertex(int iA, int iB) const {
+        SVert s;
+        s.iA = iA;
+        s.iB = iB;
+        const float2 w = mul(xf, own.at(odd ? iB : iA)), o = pair_swap(w);
+        s.wA = v2(odd ? o.x : w.x, odd ? o.y : w.y);
+        s.wB = v2(odd ? w.x : o.x, odd ? w.y : o.y);
+        s.w = sub(s.wB, s.wA);
+        s.a = 0.0f;
+        return s;
+    }
+    __device__ __forceinline__ void supports(float2 d, int &iA, int &iB) const {
+        const int i = support(own, mulT(xf.q, odd ? d : neg(d))), o = pair_swap(i);
+        iA = odd ? o : i;
+        iB = odd ? i : o;
+    }
+};
 // GetMetric (b2distance.d:710-728)
 __device__ __forceinline__ float simplex_metric(const Simplex &s) {
     if (s.count == 1) return 0.0f;
@@ -119,19 +185,19 @@ __device__ __forceinline__ float simplex_metric(const Simplex &s) {
     return crs(sub(s.v2.w, s.v1.w), sub(s.v3.w, s.v1.w));
 }
 // ReadCache (b2distance.d:574-624)
-__device__ __forceinline__ void read_cache(Simplex &s, const SimplexCache &c, const DProxy &pA, const Xf &xfA,
-                                           const DProxy &pB, const Xf &xfB) {
+template <class P>
+__device__ __forceinline__ void read_cache(Simplex &s, const SimplexCache &c, const P &p) {
     s.count = c.count;
-    if (c.count > 0) s.v1 = make_svert(pA, xfA, c.iA0, pB, xfB, c.iB0);
-    if (c.count > 1) s.v2 = make_svert(pA, xfA, c.iA1, pB, xfB, c.iB1);
-    if (c.count > 2) s.v3 = make_svert(pA, xfA, c.iA2, pB, xfB, c.iB2);
+    if (c.count > 0) s.v1 = p.vertex(c.iA0, c.iB0);
+    if (c.count > 1) s.v2 = p.vertex(c.iA1, c.iB1);
+    if (c.count > 2) s.v3 = p.vertex(c.iA2, c.iB2);
     if (s.count > 1) {
         const float metric1 = c.metric;
         const float metric2 = simplex_metric(s);
         if (metric2 < 0.5f * metric1 || 2.0f * metric1 < metric2 || metric2 < kEps) s.count = 0;
     }
     if (s.count == 0) {
-        s.v1 = make_svert(pA, xfA, 0, pB, xfB, 0);
+        s.v1 = p.vertex(0, 0);
         s.v1.a = 1.0f;
         s.count = 1;
     }
@@ -234,9 +300,10 @@ __device__ __forceinline__ void solve3(Simplex &s) {
 
 // b2Distance (b2distance.d:185-345) without radii: the distance of the two
 // shapes' cores and the simplex left in the cache.
-__device__ float gjk_distance(SimplexCache &cache, const DProxy &pA, const Xf &xfA, const DProxy &pB, const Xf &xfB) {
+template <class P>
+__device__ __forceinline__ float gjk_distance(SimplexCache &cache, const P &p) {
     Simplex s;
-    read_cache(s, cache, pA, xfA, pB, xfB);
+    read_cache(s, cache, p);
     int sA0 = 0, sA1 = 0, sA2 = 0, sB0 = 0, sB1 = 0, sB2 = 0;
     for (int iter = 0; iter < 20;) {
         const int saveCount = s.count;
@@ -259,9 +326,9 @@ __device__ float gjk_distance(SimplexCache &cache, const DProxy &pA, const Xf &x
             d = sgn > 0.0f ? crs(1.0f, e12) : crs(e12, 1.0f);
         }
         if (lensq(d) < kEps * kEps) break;
-        const int iA = support(pA, mulT(xfA.q, neg(d)));
-        const int iB = support(pB, mulT(xfB.q, d));
-        const SVert nv = make_svert(pA, xfA, iA, pB, xfB, iB);
+        int iA, iB;
+        p.supports(d, iA, iB);
+        const SVert nv = p.vertex(iA, iB);
         ++iter;
         const bool dup = (saveCount > 0 && iA == sA0 && iB == sB0) || (saveCount > 1 && iA == sA1 && iB == sB1) ||
                          (saveCount > 2 && iA == sA2 && iB == sB2);
@@ -292,110 +359,87 @@ __device__ float gjk_distance(SimplexCache &cache, const DProxy &pA, const Xf &x
 __device__ __noinline__ bool test_overlap(const Shape *a, const Xf &xfA, const Shape *b, const Xf &xfB) {
     SimplexCache cache;
     cache.count = 0;
-    const DProxy pA = make_proxy(a), pB = make_proxy(b);
-    const float d = gjk_distance(cache, pA, xfA, pB, xfB);
-    const float r = pA.radius + pB.radius;
+    const LaneShapes p{make_proxy(a), make_proxy(b), xfA, xfB};
+    const float d = gjk_distance(cache, p);
+    const float r = p.pA.radius + p.pB.radius;
     const float dist = (d > r && d > kEps) ? d - r : 0.0f;
     return dist < 10.0f * kEps;
 }
 
-// b2SeparationFunction (b2timeofimpact.d:297-530)
+// b2SeparationFunction (b2timeofimpact.d:297-530) on a lane pair: the lane's own sweep
+// and proxy.
 struct SepFn {
-    Sweep sA, sB;
+    Sweep s;
     int type; // 0 points, 1 faceA, 2 faceB
+    bool face; // the face (lp, axis) is on this lane's body
     float2 lp, axis;
 };
+// A lane's own value where `own`, else the other lane's.
+__device__ __forceinline__ float2 pair_pick(bool own, float2 x) {
+    const float2 o = pair_swap(x);
+    return v2(own ? x.x : o.x, own ? x.y : o.y);
+}
+// dot(pB - pA, n) of the lanes' points (types 0 and 1), dot(pA - pB, n) for type 2.
+__device__ __forceinline__ float pair_separation(bool minuend, float2 p, float2 n) {
+    const float2 o = pair_swap(p);
+    return dot(v2(minuend ? p.x - o.x : o.x - p.x, minuend ? p.y - o.y : o.y - p.y), n);
+}
 // Initialize (b2timeofimpact.d:331-410)
-__device__ void sep_init(SepFn &f, const SimplexCache &cache, const DProxy &pA, const Sweep &sA, const DProxy &pB,
-                         const Sweep &sB, float t1) {
-    f.sA = sA;
-    f.sB = sB;
-    const Xf xfA = sweep_xf(sA, t1), xfB = sweep_xf(sB, t1);
+__device__ __forceinline__ void sep_init(SepFn &f, const SimplexCache &cache, const LdsProxy &own, bool odd,
+                                         const Sweep &s, float t1) {
+    f.s = s;
+    const Xf xf = sweep_xf(s, t1);
+    const float2 e0 = own.at(odd ? cache.iB0 : cache.iA0);
     if (cache.count == 1) {
         f.type = 0;
-        const float2 pointA = mul(xfA, pA.v[cache.iA0]);
-        const float2 pointB = mul(xfB, pB.v[cache.iB0]);
-        f.axis = sub(pointB, pointA);
+        f.face = false;
+        const float2 w = mul(xf, e0), o = pair_swap(w);
+        f.axis = odd ? sub(w, o) : sub(o, w);
         normalize(f.axis);
         f.lp = v2(0.0f, 0.0f);
-    } else if (cache.iA0 == cache.iA1) {
-        f.type = 2;
-        const float2 b1 = pB.v[cache.iB0], b2 = pB.v[cache.iB1];
-        f.axis = crs(sub(b2, b1), 1.0f);
-        normalize(f.axis);
-        const float2 normal = mul(xfB.q, f.axis);
-        f.lp = scl(0.5f, add(b1, b2));
-        const float2 pointB = mul(xfB, f.lp);
-        const float2 pointA = mul(xfA, pA.v[cache.iA0]);
-        const float s = dot(sub(pointA, pointB), normal);
-        if (s < 0.0f) f.axis = neg(f.axis);
-    } else {
-        f.type = 1;
-        const float2 a1 = pA.v[cache.iA0], a2 = pA.v[cache.iA1];
-        f.axis = crs(sub(a2, a1), 1.0f);
-        normalize(f.axis);
-        const float2 normal = mul(xfA.q, f.axis);
-        f.lp = scl(0.5f, add(a1, a2));
-        const float2 pointA = mul(xfA, f.lp);
-        const float2 pointB = mul(xfB, pB.v[cache.iB0]);
-        const float s = dot(sub(pointB, pointA), normal);
-        if (s < 0.0f) f.axis = neg(f.axis);
+        return;
     }
+    const float2 e1 = own.at(odd ? cache.iB1 : cache.iA1);
+    f.type = cache.iA0 == cache.iA1 ? 2 : 1;
+    f.face = odd == (f.type == 2);
+    const float2 f0 = pair_pick(f.face, e0), f1 = pair_pick(f.face, e1);
+    f.axis = crs(sub(f1, f0), 1.0f);
+    normalize(f.axis);
+    const float2 normal = pair_pick(f.face, mul(xf.q, f.axis));
+    f.lp = scl(0.5f, add(f0, f1));
+    const float sep = pair_separation(!f.face, mul(xf, f.face ? f.lp : e0), normal);
+    if (sep < 0.0f) f.axis = neg(f.axis);
 }
-// FindMinSeparation (b2timeofimpact.d:413-470)
-__device__ float sep_find_min(const SepFn &f, const DProxy &pA, const DProxy &pB, int &iA, int &iB, float t) {
-    const Xf xfA = sweep_xf(f.sA, t), xfB = sweep_xf(f.sB, t);
+// FindMinSeparation (b2timeofimpact.d:413-470); v: this lane's vertex.
+__device__ __forceinline__ float sep_find_min(const SepFn &f, const LdsProxy &own, bool odd, float2 &v, float t) {
+    const Xf xf = sweep_xf(f.s, t);
     if (f.type == 0) {
-        iA = support(pA, mulT(xfA.q, f.axis));
-        iB = support(pB, mulT(xfB.q, neg(f.axis)));
-        const float2 pointA = mul(xfA, pA.v[iA]);
-        const float2 pointB = mul(xfB, pB.v[iB]);
-        return dot(sub(pointB, pointA), f.axis);
+        v = own.at(support(own, mulT(xf.q, odd ? neg(f.axis) : f.axis)));
+        return pair_separation(odd, mul(xf, v), f.axis);
     }
-    if (f.type == 1) {
-        const float2 normal = mul(xfA.q, f.axis);
-        const float2 pointA = mul(xfA, f.lp);
-        iA = -1;
-        iB = support(pB, mulT(xfB.q, neg(normal)));
-        const float2 pointB = mul(xfB, pB.v[iB]);
-        return dot(sub(pointB, pointA), normal);
-    }
-    const float2 normal = mul(xfB.q, f.axis);
-    const float2 pointB = mul(xfB, f.lp);
-    iB = -1;
-    iA = support(pA, mulT(xfA.q, neg(normal)));
-    const float2 pointA = mul(xfA, pA.v[iA]);
-    return dot(sub(pointA, pointB), normal);
+    const float2 normal = pair_pick(f.face, mul(xf.q, f.axis));
+    v = own.at(support(own, mulT(xf.q, neg(normal))));
+    return pair_separation(!f.face, mul(xf, f.face ? f.lp : v), normal);
 }
 // Evaluate (b2timeofimpact.d:473-518)
-__device__ float sep_eval(const SepFn &f, const DProxy &pA, const DProxy &pB, int iA, int iB, float t) {
-    const Xf xfA = sweep_xf(f.sA, t), xfB = sweep_xf(f.sB, t);
-    if (f.type == 0) {
-        const float2 pointA = mul(xfA, pA.v[iA]);
-        const float2 pointB = mul(xfB, pB.v[iB]);
-        return dot(sub(pointB, pointA), f.axis);
-    }
-    if (f.type == 1) {
-        const float2 normal = mul(xfA.q, f.axis);
-        const float2 pointA = mul(xfA, f.lp);
-        const float2 pointB = mul(xfB, pB.v[iB]);
-        return dot(sub(pointB, pointA), normal);
-    }
-    const float2 normal = mul(xfB.q, f.axis);
-    const float2 pointB = mul(xfB, f.lp);
-    const float2 pointA = mul(xfA, pA.v[iA]);
-    return dot(sub(pointA, pointB), normal);
+__device__ __forceinline__ float sep_eval(const SepFn &f, bool odd, float2 v, float t) {
+    const Xf xf = sweep_xf(f.s, t);
+    if (f.type == 0) return pair_separation(odd, mul(xf, v), f.axis);
+    const float2 normal = pair_pick(f.face, mul(xf.q, f.axis));
+    return pair_separation(!f.face, mul(xf, f.face ? f.lp : v), normal);
 }
 
 // b2TimeOfImpact (b2timeofimpact.d:67-295) over [0, tMax]; returns the output
 // state and writes the time.  Every loop is bounded as in the reference (20
-// outer iterations, b2_maxPolygonVertices push-backs, 50 root-finder steps).
-__device__ int time_of_impact(float &tOut, const DProxy &pA, const DProxy &pB, Sweep sA, Sweep sB, float tMax) {
+// outer iterations, b2_maxPolygonVertices push-backs, 50 root-finder steps).  On a lane
+// pair: own and s are body A's on the even lane and body B's on the odd one; both
+// lanes return the same.
+__device__ __forceinline__ int time_of_impact(float &tOut, const LdsProxy &own, Sweep s, float tMax) {
+    const bool odd = (threadIdx.x & 1) != 0;
     int state = kToiUnknown;
     tOut = tMax;
-    sweep_normalize(sA);
-    sweep_normalize(sB);
-    const float totalRadius = pA.radius + pB.radius;
+    sweep_normalize(s);
+    const float totalRadius = own.radius + pair_swap(own.radius);
     const float target = fmaxr(kLinearSlop, totalRadius - 3.0f * kLinearSlop);
     const float tolerance = 0.25f * kLinearSlop;
     float t1 = 0.0f;
@@ -404,8 +448,8 @@ __device__ int time_of_impact(float &tOut, const DProxy &pA, const DProxy &pB, S
     cache.metric = 0.0f;
     cache.iA0 = cache.iA1 = cache.iA2 = cache.iB0 = cache.iB1 = cache.iB2 = 0;
     for (int iter = 0;;) {
-        const Xf xfA = sweep_xf(sA, t1), xfB = sweep_xf(sB, t1);
-        const float distance = gjk_distance(cache, pA, xfA, pB, xfB);
+        const PairShapes p{own, sweep_xf(s, t1), odd};
+        const float distance = gjk_distance(cache, p);
         if (distance <= 0.0f) {
             state = kToiOverlapped;
             tOut = 0.0f;
@@ -417,12 +461,12 @@ __device__ int time_of_impact(float &tOut, const DProxy &pA, const DProxy &pB, S
             break;
         }
         SepFn fcn;
-        sep_init(fcn, cache, pA, sA, pB, sB, t1);
+        sep_init(fcn, cache, own, odd, s, t1);
         bool done = false;
         float t2 = tMax;
         for (int pushBackIter = 0;;) {
-            int iA, iB;
-            float s2 = sep_find_min(fcn, pA, pB, iA, iB, t2);
+            float2 v;
+            float s2 = sep_find_min(fcn, own, odd, v, t2);
             if (s2 > target + tolerance) {
                 state = kToiSeparated;
                 tOut = tMax;
@@ -433,7 +477,7 @@ __device__ int time_of_impact(float &tOut, const DProxy &pA, const DProxy &pB, S
                 t1 = t2;
                 break;
             }
-            float s1 = sep_eval(fcn, pA, pB, iA, iB, t1);
+            float s1 = sep_eval(fcn, odd, v, t1);
             if (s1 < target - tolerance) {
                 state = kToiFailed;
                 tOut = t1;
@@ -452,17 +496,17 @@ __device__ int time_of_impact(float &tOut, const DProxy &pA, const DProxy &pB, S
                 if (rootIterCount & 1) t = a1 + (target - s1) * (a2 - a1) / (s2 - s1);
                 else t = 0.5f * (a1 + a2);
                 ++rootIterCount;
-                const float s = sep_eval(fcn, pA, pB, iA, iB, t);
-                if (fabsr(s - target) < tolerance) {
+                const float sep = sep_eval(fcn, odd, v, t);
+                if (fabsr(sep - target) < tolerance) {
                     t2 = t;
                     break;
                 }
-                if (s > target) {
+                if (sep > target) {
                     a1 = t;
-                    s1 = s;
+                    s1 = sep;
                 } else {
                     a2 = t;
-                    s2 = s;
+                    s2 = sep;
                 }
                 if (rootIterCount == 50) break;
             }
