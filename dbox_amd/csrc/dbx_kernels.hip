@@ -2024,15 +2024,15 @@ __device__ __forceinline__ void pair_xfs(float2 cA, float aA, float2 lcA, float2
     xfB.p = sub(cB, mul(xfB.q, lcB));
 }
 // solve_position_core with the transforms built by a lane pair.
-__device__ __forceinline__ float solve_position_pair(const PosCon &p, float4 &pa, float4 &pb) {
+__device__ __forceinline__ float solve_position_pair(const PosCon &p, float4 &pa, float4 &pb, float beta = kBaumgarte) {
     float2 cA = v2(pa.x, pa.y), cB = v2(pb.x, pb.y);
     float aA = pa.z, aB = pb.z;
     Xf xfA, xfB;
     pair_xfs(cA, aA, p.lcA, cB, aB, p.lcB, xfA, xfB);
-    float minSep = fminr(0.0f, position_point(p, p.lp0, xfA, xfB, cA, aA, cB, aB));
+    float minSep = fminr(0.0f, position_point(p, p.lp0, xfA, xfB, cA, aA, cB, aB, beta));
     if (p.pointCount > 1) {
         pair_xfs(cA, aA, p.lcA, cB, aB, p.lcB, xfA, xfB);
-        minSep = fminr(minSep, position_point(p, p.lp1, xfA, xfB, cA, aA, cB, aB));
+        minSep = fminr(minSep, position_point(p, p.lp1, xfA, xfB, cA, aA, cB, aB, beta));
     }
     pa = make_float4(cA.x, cA.y, aA, pa.w);
     pb = make_float4(cB.x, cB.y, aB, pb.w);
@@ -4032,6 +4032,39 @@ __device__ __forceinline__ void mark_dirty(const ToiWorld &W, ToiLists &L, int j
     W.tc[j].y = (y & ~clear) | kTcDirty;
 }
 
+// Orders the wave's memory accesses: what its lanes wrote before is read after.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+}
+// mark_dirty for every contact of body b, by one wave, an edge per lane.
+__device__ __forceinline__ void mark_body(const ToiWorld &W, ToiLists &L, int b, int clear) {
+    const int lane = threadIdx.x & 63;
+    for (int e = W.tb[b].z; e >= 0;) { // contacts made since the Collide
+        const int4 t = W.tc[e >> 1];
+        if (lane == 0) mark_dirty(W, L, e >> 1, clear);
+        e = (e & 1) ? t.w : t.z;
+    }
+    const int o = W.adjOff[b], cnt = W.adjCnt[b];
+    for (int k0 = 0; k0 < cnt; k0 += 64) {
+        const bool have = k0 + lane < cnt;
+        const int j = have ? W.adj[o + k0 + lane].x >> 1 : 0;
+        const int y = have ? W.tc[j].y : kTcDirty;
+        wave_sync();
+        const unsigned long long fresh = __builtin_amdgcn_ballot_w64(!(y & kTcDirty));
+        const int nd = L.ndirty, at = nd + __popcll(fresh & ((1ull << lane) - 1ull));
+        if (!(y & kTcDirty) && at < kToiDirtyCap) L.dirty[at] = j;
+        if (have) W.tc[j].y = (y & ~clear) | kTcDirty;
+        wave_sync(); // all lanes have read ndirty
+        if (lane == 0) {
+            L.ndirty = min(nd + __popcll(fresh), kToiDirtyCap);
+            if (nd + __popcll(fresh) > kToiDirtyCap) L.overflow |= 1;
+        }
+        wave_sync();
+    }
+    wave_sync();
+}
+
 __device__ __forceinline__ Sweep load_sweep(const ToiWorld &W, int b) {
     Sweep s;
     const float4 m = W.bmass[b], p0 = W.bpos0[b], p = W.bpos[b];
@@ -4188,69 +4221,114 @@ __device__ __forceinline__ SweepSnap snap_of(const ToiWorld &W, int j) {
     return sn;
 }
 
-// One TOI event (b2world.d:1270-1405) on one lane: advance both bodies to the
+// One TOI event (b2world.d:1270-1405) by one wave: advance both bodies to the
 // TOI, update the contact, build the island and solve it (b2island.d:282-416).
 // Returns the island body count, 0 when the contact was not touching at the TOI.
 // ibod, icon, vcs, pcs, imp: the island's bodies, contacts and solver state in LDS.
+//
+// An event is one chain, bound by its instructions and by the latency of its loads.
+// Lanes 0 and 1 run its serial part together, doing and writing the same, except that
+// the even lane has body A's sweep and rotations and the odd lane body B's; what is
+// independent per contact or body (which edges of a body matter, set-up,
+// integration, fixtures, marks) is spread over the wave.  64 rooms of 40 projectiles: 548
+// us a step with all of it on one lane, 487 so.
 __device__ __forceinline__ int toi_event(const ToiWorld &W, ToiLists &L, int ci, float minAlpha, const StepParams &sp,
                                          int *ibod, int *icon, VelCon *vcs, PosCon *pcs, float4 *imp) {
     Contact *cont = W.cont;
-    const int ia = W.fbody[cont[ci].fa], ib = W.fbody[cont[ci].fb];
-    const Sweep backup1 = load_sweep(W, ia), backup2 = load_sweep(W, ib);
-    body_advance(W, ia, minAlpha);
-    body_advance(W, ib, minAlpha);
-    Contact mc = cont[ci];
-    toi_update(W, L, mc, ci);
-    cont[ci] = mc;
-    const int t0 = W.tc[ci].y;
-    W.tc[ci].y = (((t0 & kTcCount) + 1) & kTcCount) | (t0 & (kTcIsland | kTcDirty | kTcSnap | kTcCand));
-    if (!(mc.flags & kContactEnabled) || !(mc.flags & kContactTouching)) {
-        cont[ci].flags = mc.flags & ~kContactEnabled;
-        store_sweep(W, ia, backup1);
-        store_sweep(W, ib, backup2);
-        sync_transform(W, ia);
-        sync_transform(W, ib);
-        return 0;
+    const int lane = threadIdx.x & 63;
+    const bool serial = lane < 2;
+    const int ia = W.fbody[cont[ci].fa], ib = W.fbody[cont[ci].fb], own = lane == 1 ? ib : ia;
+    int go = 0;
+    Sweep backup{};
+    if (serial) {
+        backup = load_sweep(W, own);
+        body_advance(W, own, minAlpha);
+        wave_sync();
+        Contact mc = cont[ci];
+        toi_update(W, L, mc, ci);
+        cont[ci] = mc;
+        const int t0 = W.tc[ci].y;
+        W.tc[ci].y = (((t0 & kTcCount) + 1) & kTcCount) | (t0 & (kTcIsland | kTcDirty | kTcSnap | kTcCand));
+        go = (mc.flags & kContactEnabled) && (mc.flags & kContactTouching);
+        if (!go) {
+            cont[ci].flags = mc.flags & ~kContactEnabled;
+            store_sweep(W, own, backup);
+            sync_transform(W, own);
+        }
     }
-    toi_wake(W, L, ia);
-    toi_wake(W, L, ib);
-    int nbod = 0, ncon = 0;
-    ibod[nbod++] = ia;
-    ibod[nbod++] = ib;
-    icon[ncon++] = ci;
-    W.tb[ia].y = 1;
-    W.tb[ib].y = 1;
-    W.tc[ci].y |= kTcIsland;
+    wave_sync();
+    if (!__builtin_amdgcn_readfirstlane(go)) return 0;
+    int nbod = 2, ncon = 1;
+    if (serial) {
+        toi_wake(W, L, ia);
+        toi_wake(W, L, ib);
+        ibod[0] = ia;
+        ibod[1] = ib;
+        icon[0] = ci;
+        W.tb[ia].y = 1;
+        W.tb[ib].y = 1;
+        W.tc[ci].y |= kTcIsland;
+    }
     // contacts of the two bodies with static, kinematic or bullet bodies that
     // touch at the TOI
     for (int side = 0; side < 2; ++side) {
         const int body = side ? ib : ia;
         const uint32_t bf = W.bfl[body];
         if (body_type(bf) != kDynamic) continue;
-        body_contacts(W, body, [&](int j, int other) {
-            if (nbod == 2 * kMaxToiContacts || ncon == kMaxToiContacts) return false;
-            if (W.tc[j].y & kTcIsland) return true;
-            if (W.cont[j].flags & kContactSensor) return true;
+        const auto takes_part = [&](int j, int other) {
+            if (W.cont[j].flags & kContactSensor) return false;
             const uint32_t of = W.bfl[other];
-            if (body_type(of) == kDynamic && !(bf & kBodyBullet) && !(of & kBodyBullet)) return true;
-            const Sweep backup = load_sweep(W, other);
+            return body_type(of) != kDynamic || (bf & kBodyBullet) || (of & kBodyBullet);
+        };
+        const auto visit = [&](int j, int other) { // on the serial lanes
+            if (W.tc[j].y & kTcIsland) return;
+            const Sweep back = load_sweep(W, other);
             if (W.tb[other].y == 0) body_advance(W, other, minAlpha);
             Contact cu = cont[j];
             toi_update(W, L, cu, j);
             cont[j] = cu;
             if (!(cu.flags & kContactEnabled) || !(cu.flags & kContactTouching)) {
-                store_sweep(W, other, backup);
+                store_sweep(W, other, back);
                 sync_transform(W, other);
-                return true;
+                return;
             }
             W.tc[j].y |= kTcIsland;
             icon[ncon++] = j;
-            if (W.tb[other].y) return true;
+            if (W.tb[other].y) return;
             W.tb[other].y = 1;
             if (body_type(W.bfl[other]) != kStatic) toi_wake(W, L, other);
             ibod[nbod++] = other;
-            return true;
-        });
+        };
+        wave_sync();
+        bool full = nbod == 2 * kMaxToiContacts || ncon == kMaxToiContacts;
+        for (int e = W.tb[body].z; e >= 0 && !full;) { // contacts made since the Collide
+            const int j = e >> 1;
+            const int4 t = W.tc[j];
+            const int other = W.fbody[(e & 1) ? W.cont[j].fa : W.cont[j].fb];
+            if (takes_part(j, other)) {
+                if (serial) visit(j, other);
+                wave_sync();
+                nbod = __builtin_amdgcn_readfirstlane(nbod);
+                ncon = __builtin_amdgcn_readfirstlane(ncon);
+                full = nbod == 2 * kMaxToiContacts || ncon == kMaxToiContacts;
+            }
+            e = (e & 1) ? t.w : t.z;
+        }
+        const int o = W.adjOff[body], cnt = W.adjCnt[body];
+        for (int k0 = 0; k0 < cnt && !full; k0 += 64) {
+            const bool have = k0 + lane < cnt;
+            const int2 a = have ? W.adj[o + k0 + lane] : make_int2(0, 0);
+            unsigned long long todo = __builtin_amdgcn_ballot_w64(have && takes_part(a.x >> 1, a.y));
+            for (; todo && !full; todo &= todo - 1) {
+                const int l = __builtin_ctzll(todo);
+                const int j = __builtin_amdgcn_readlane(a.x, l) >> 1, other = __builtin_amdgcn_readlane(a.y, l);
+                if (serial) visit(j, other);
+                wave_sync();
+                nbod = __builtin_amdgcn_readfirstlane(nbod);
+                ncon = __builtin_amdgcn_readfirstlane(ncon);
+                full = nbod == 2 * kMaxToiContacts || ncon == kMaxToiContacts;
+            }
+        }
     }
     // the sub-step: the rest of the step, no warm starting (b2world.d:1391-1398)
     StepParams ss = sp;
@@ -4258,79 +4336,88 @@ __device__ __forceinline__ int toi_event(const ToiWorld &W, ToiLists &L, int ci,
     ss.inv_dt = 1.0f / ss.dt;
     ss.dtRatio = 1.0f;
     ss.flags = sp.flags & ~1u; // no warm starting
+    wave_sync();
     // The solver works on the bodies' own sweep positions, which the island's
     // position array starts from and which nothing else reads until the end.
-    for (int k = 0; k < ncon; ++k)
-        init_constraint(vcs[k], pcs[k], cont[icon[k]], icon[k], 0, W.fbody, W.fmat, W.bfl, W.bmass, W.bpos, W.bvel, ss,
-                        W.ctan[icon[k]]);
+    if (lane < ncon)
+        init_constraint(vcs[lane], pcs[lane], cont[icon[lane]], icon[lane], 0, W.fbody, W.fmat, W.bfl, W.bmass, W.bpos,
+                        W.bvel, ss, W.ctan[icon[lane]]);
+    wave_sync();
     // SolveTOIPositionConstraints (b2contactsolver.d:152-242): only the two TOI
     // bodies move.  An island of the TOI contact alone (the usual event) keeps its
     // two bodies in registers over the iterations.
-    if (ncon == 1) {
-        const PosCon p = pcs[0]; // its bodies are the two TOI bodies
-        float4 pa = W.bpos[p.indexA], pb = W.bpos[p.indexB];
-        for (int it = 0; it < 20; ++it)
-            if (fminr(0.0f, solve_position_core(p, pa, pb, kToiBaumgarte)) >= -1.5f * kLinearSlop) break;
-        W.bpos[p.indexA] = pa;
-        W.bpos[p.indexB] = pb;
-    } else {
-        for (int it = 0; it < 20; ++it) {
-            float minSep = 0.0f;
-            for (int k = 0; k < ncon; ++k) {
-                PosCon p = pcs[k];
-                if (p.indexA != ia && p.indexA != ib) {
-                    p.invMassA = 0.0f;
-                    p.invIA = 0.0f;
+    if (serial) {
+        if (ncon == 1) {
+            const PosCon p = pcs[0]; // its bodies are the two TOI bodies
+            float4 pa = W.bpos[p.indexA], pb = W.bpos[p.indexB];
+            for (int it = 0; it < 20; ++it)
+                if (fminr(0.0f, solve_position_pair(p, pa, pb, kToiBaumgarte)) >= -1.5f * kLinearSlop) break;
+            W.bpos[p.indexA] = pa;
+            W.bpos[p.indexB] = pb;
+        } else {
+            for (int it = 0; it < 20; ++it) {
+                float minSep = 0.0f;
+                for (int k = 0; k < ncon; ++k) {
+                    PosCon p = pcs[k];
+                    if (p.indexA != ia && p.indexA != ib) {
+                        p.invMassA = 0.0f;
+                        p.invIA = 0.0f;
+                    }
+                    if (p.indexB != ia && p.indexB != ib) {
+                        p.invMassB = 0.0f;
+                        p.invIB = 0.0f;
+                    }
+                    float4 pa = W.bpos[p.indexA], pb = W.bpos[p.indexB];
+                    minSep = fminr(minSep, solve_position_pair(p, pa, pb, kToiBaumgarte));
+                    W.bpos[p.indexA] = pa;
+                    W.bpos[p.indexB] = pb;
                 }
-                if (p.indexB != ia && p.indexB != ib) {
-                    p.invMassB = 0.0f;
-                    p.invIB = 0.0f;
-                }
-                float4 pa = W.bpos[p.indexA], pb = W.bpos[p.indexB];
-                minSep = fminr(minSep, solve_position_core(p, pa, pb, kToiBaumgarte));
-                W.bpos[p.indexA] = pa;
-                W.bpos[p.indexB] = pb;
+                if (minSep >= -1.5f * kLinearSlop) break;
             }
-            if (minSep >= -1.5f * kLinearSlop) break;
         }
+        // leap of faith to the new safe state
+        const float4 p = W.bpos[own];
+        W.bpos0[own] = make_float4(p.x, p.y, p.z, W.bpos0[own].w);
     }
-    // leap of faith to the new safe state
-    {
-        const float4 pa = W.bpos[ia], pb = W.bpos[ib];
-        W.bpos0[ia] = make_float4(pa.x, pa.y, pa.z, W.bpos0[ia].w);
-        W.bpos0[ib] = make_float4(pb.x, pb.y, pb.z, W.bpos0[ib].w);
+    wave_sync();
+    if (lane < ncon) {
+        init_constraint(vcs[lane], pcs[lane], cont[icon[lane]], icon[lane], 0, W.fbody, W.fmat, W.bfl, W.bmass, W.bpos,
+                        W.bvel, ss, W.ctan[icon[lane]]);
+        imp[lane] = make_float4(vcs[lane].nImp0, vcs[lane].tImp0, vcs[lane].nImp1, vcs[lane].tImp1);
     }
-    for (int k = 0; k < ncon; ++k) {
-        init_constraint(vcs[k], pcs[k], cont[icon[k]], icon[k], 0, W.fbody, W.fmat, W.bfl, W.bmass, W.bpos, W.bvel, ss,
-                        W.ctan[icon[k]]);
-        imp[k] = make_float4(vcs[k].nImp0, vcs[k].tImp0, vcs[k].nImp1, vcs[k].tImp1);
+    wave_sync();
+    if (serial) {
+        if (ncon == 1) { // the two bodies and the impulses stay in registers
+            const VelCon v = vcs[0];
+            float4 va = W.bvel[v.indexA], vb = W.bvel[v.indexB], im = imp[0];
+            for (int it = 0; it < sp.velocityIterations; ++it) solve_velocity_core<false>(v, im, va, vb);
+            imp[0] = im;
+            W.bvel[v.indexA] = va;
+            W.bvel[v.indexB] = vb;
+        } else {
+            for (int it = 0; it < sp.velocityIterations; ++it)
+                for (int k = 0; k < ncon; ++k) {
+                    const VelCon &v = vcs[k];
+                    float4 va = W.bvel[v.indexA], vb = W.bvel[v.indexB];
+                    float4 im = imp[k];
+                    solve_velocity_core<false>(v, im, va, vb);
+                    imp[k] = im;
+                    W.bvel[v.indexA] = va;
+                    W.bvel[v.indexB] = vb;
+                }
+        }
+        // b2Island.Report of the sub-step island (b2island.d:415,438-461): the
+        // solver's impulses, which are not stored into the manifolds
+        for (int k = 0; k < ncon; ++k) toi_log(W, L, 3, cont[icon[k]], vcs[k].pointCount, imp[k]);
     }
-    if (ncon == 1) { // the two bodies and the impulses stay in registers
-        const VelCon v = vcs[0];
-        float4 va = W.bvel[v.indexA], vb = W.bvel[v.indexB], im = imp[0];
-        for (int it = 0; it < sp.velocityIterations; ++it) solve_velocity_core<false>(v, im, va, vb);
-        imp[0] = im;
-        W.bvel[v.indexA] = va;
-        W.bvel[v.indexB] = vb;
-    } else {
-        for (int it = 0; it < sp.velocityIterations; ++it)
-            for (int k = 0; k < ncon; ++k) {
-                const VelCon &v = vcs[k];
-                float4 va = W.bvel[v.indexA], vb = W.bvel[v.indexB];
-                float4 im = imp[k];
-                solve_velocity_core<false>(v, im, va, vb);
-                imp[k] = im;
-                W.bvel[v.indexA] = va;
-                W.bvel[v.indexB] = vb;
-            }
-    }
-    // b2Island.Report of the sub-step island (b2island.d:415,438-461): the
-    // solver's impulses, which are not stored into the manifolds
-    for (int k = 0; k < ncon; ++k) toi_log(W, L, 3, cont[icon[k]], vcs[k].pointCount, imp[k]);
-    // integrate positions (b2island.d:370-413)
+    wave_sync();
+    // a body per lane: integrate positions (b2island.d:370-413), then island flags reset
+    // and fixtures of the dynamic bodies synchronised (the moved ones enter the move
+    // buffer, in any order)
     const float h = ss.dt;
-    for (int i = 0; i < nbod; ++i) {
-        const int b = ibod[i];
+    int type = kStatic;
+    if (lane < nbod) {
+        const int b = ibod[lane];
         const float4 p = W.bpos[b], vel = W.bvel[b];
         float2 c = v2(p.x, p.y), v = v2(vel.x, vel.y);
         float a = p.z, wv = vel.z;
@@ -4346,23 +4433,16 @@ __device__ __forceinline__ int toi_event(const ToiWorld &W, ToiLists &L, int ci,
         }
         c = add(c, scl(h, v));
         a += h * wv;
+        const float4 ms = W.bmass[b];
+        const Xf x2 = xf_from(c, a, v2(ms.z, ms.w)); // SynchronizeTransform
         W.bpos[b] = make_float4(c.x, c.y, a, p.w);
         W.bvel[b] = make_float4(v.x, v.y, wv, 0.0f);
-        sync_transform(W, b);
-    }
-    // island flags reset; fixtures of the dynamic bodies synchronised (the
-    // moved ones enter the move buffer); their contacts' TOIs dropped
-    // (b2world.d:1401-1429).  Every contact whose bodies changed is looked at
-    // again by the next search.
-    for (int i = 0; i < nbod; ++i) {
-        const int b = ibod[i];
+        W.bxf[b] = make_float4(x2.p.x, x2.p.y, x2.q.s, x2.q.c);
         W.tb[b].y = 0;
-        const int type = body_type(W.bfl[b]);
-        if (type == kStatic) continue;
+        type = body_type(W.bfl[b]);
         if (type == kDynamic) {
-            const float4 p0 = W.bpos0[b], ms = W.bmass[b];
+            const float4 p0 = W.bpos0[b];
             const Xf x1 = xf_from(v2(p0.x, p0.y), p0.z, v2(ms.z, ms.w));
-            const Xf x2 = load_xf(W.bxf, b);
             const float2 disp = sub(x2.p, x1.p);
             for (int k = 0; k < W.bfixCnt[b]; ++k) {
                 const int f = W.bfixList[W.bfixOff[b] + k];
@@ -4381,16 +4461,20 @@ __device__ __forceinline__ int toi_event(const ToiWorld &W, ToiLists &L, int ci,
                 W.fat[f] = nbx;
                 if (!W.moved[f]) {
                     W.moved[f] = 1;
-                    if (L.nmoved < kToiListCap) L.moved[L.nmoved++] = f;
-                    else L.overflow |= 2;
+                    const int at = atomicAdd(&L.nmoved, 1);
+                    if (at < kToiListCap) L.moved[at] = f;
+                    else atomicOr(&L.overflow, 2);
                 }
             }
         }
-        const int clear = type == kDynamic ? (kTcToi | kTcIsland) : 0;
-        body_contacts(W, b, [&](int j, int) {
-            mark_dirty(W, L, j, clear);
-            return true;
-        });
+    }
+    wave_sync();
+    if (lane == 0) L.nmoved = min(L.nmoved, kToiListCap);
+    // the dynamic bodies' contacts' TOIs dropped (b2world.d:1401-1429); every contact whose
+    // bodies changed is looked at again by the next search
+    for (unsigned long long todo = __builtin_amdgcn_ballot_w64(type != kStatic); todo; todo &= todo - 1) {
+        const int l = __builtin_ctzll(todo);
+        mark_body(W, L, ibod[l], __builtin_amdgcn_readlane(type, l) == kDynamic ? (kTcToi | kTcIsland) : 0);
     }
     return nbod;
 }
@@ -4693,7 +4777,7 @@ __device__ __forceinline__ void toi_pass(const Dev &d, int cur, const StepParams
             // other's time, then the TOI is computed from the sweeps as they stand
             const bool all = (s_L.overflow & 1) != 0;
             const int nd = all ? n : s_L.ndirty;
-            if (tid == 0 && !all) // list order is descending slot order
+            if (!all && nd > 64 && tid == 0) // list order is descending slot order
                 for (int i = 1; i < nd; ++i) {
                     const int v = s_dirty[i];
                     int j = i - 1;
@@ -4704,26 +4788,43 @@ __device__ __forceinline__ void toi_pass(const Dev &d, int cur, const StepParams
                     s_dirty[j + 1] = v;
                 }
             for (int c0 = 0; c0 < nd; c0 += 64) {
-                if (tid == 0) {
-                    int k = 0;
-                    const int c1 = c0 + 64 < nd ? c0 + 64 : nd;
-                    for (int q = c0; q < c1; ++q) {
-                        const int j = all ? n - 1 - q : s_dirty[q];
+                if (wave == 0) {
+                    // a contact per lane: which need a TOI; these in list order
+                    wave_sync();
+                    const int q = c0 + lane;
+                    const bool have = q < nd;
+                    int j = !have ? -1 : all ? n - 1 - q : s_dirty[q];
+                    if (!all && nd <= 64) {
+                        int rank = 0;
+                        for (int u = 0; u < nd; ++u) rank += __builtin_amdgcn_readlane(j, u) > j ? 1 : 0;
+                        if (have) s_dirty[rank] = j;
+                        wave_sync();
+                        if (have) j = s_dirty[lane];
+                    }
+                    bool need = false;
+                    if (have) {
                         const int y = W.tc[j].y & ~kTcDirty;
                         W.tc[j].y = y;
-                        const Contact &c = W.cont[j];
-                        if (toi_status(W, c, y) != 2) continue;
-                        const int ba = W.fbody[c.fa], bb = W.fbody[c.fb];
-                        const float xa = __int_as_float(W.tb[ba].x), xb = __int_as_float(W.tb[bb].x);
-                        if (xa < xb || xb < xa) { // b2Sweep.Advance of the body at the earlier time
-                            const int b = xa < xb ? ba : bb;
-                            Sweep sw = load_sweep(W, b);
-                            sweep_advance(sw, xa < xb ? xb : xa);
-                            store_sweep(W, b, sw);
-                        }
-                        s_snap[k++] = snap_of(W, j);
+                        need = toi_status(W, W.cont[j], y) == 2;
                     }
-                    s_nsnap = k;
+                    unsigned long long todo = __builtin_amdgcn_ballot_w64(need);
+                    const int k = __popcll(todo);
+                    for (int at = 0; todo; todo &= todo - 1, ++at) {
+                        const int jc = __builtin_amdgcn_readlane(j, __builtin_ctzll(todo));
+                        if (lane == 0) {
+                            const Contact &c = W.cont[jc];
+                            const int ba = W.fbody[c.fa], bb = W.fbody[c.fb];
+                            const float xa = __int_as_float(W.tb[ba].x), xb = __int_as_float(W.tb[bb].x);
+                            if (xa < xb || xb < xa) { // b2Sweep.Advance of the body at the earlier time
+                                const int b = xa < xb ? ba : bb;
+                                Sweep sw = load_sweep(W, b);
+                                sweep_advance(sw, xa < xb ? xb : xa);
+                                store_sweep(W, b, sw);
+                            }
+                            s_snap[at] = snap_of(W, jc);
+                        }
+                    }
+                    if (lane == 0) s_nsnap = k;
                 }
                 __syncthreads();
                 const int ns = s_nsnap;
@@ -4803,20 +4904,21 @@ __device__ __forceinline__ void toi_pass(const Dev &d, int cur, const StepParams
         if (bestPos == INT_MAX || 1.0f - 10.0f * kEps < bestA) break;
         const int ci = n - 1 - bestPos;
         if (timed) tMark = __builtin_amdgcn_s_memtime();
-        if (tid == 0) {
+        if (wave == 0) {
             ToiLists &L = s_L;
-            L.nwoken = L.nmoved = 0;
-            s_nb = toi_event(W, L, ci, bestA, sp, s_ibod, s_icon, s_vc, s_pc, s_imp);
+            if (lane == 0) L.nwoken = L.nmoved = 0;
+            wave_sync();
+            const int nbod = toi_event(W, L, ci, bestA, sp, s_ibod, s_icon, s_vc, s_pc, s_imp);
             // contacts of bodies the event woke take part again
-            for (int k = 0; k < L.nwoken; ++k)
-                body_contacts(W, L.woken[k], [&](int j, int) {
-                    mark_dirty(W, L, j, 0);
-                    return true;
-                });
-            s_nmoved = L.nmoved;
-            if (L.overflow & 2) error |= 4;
-            L.overflow &= ~2;
-            s_np = 0;
+            const int nwoken = L.nwoken;
+            for (int k = 0; k < nwoken; ++k) mark_body(W, L, L.woken[k], 0);
+            if (lane == 0) {
+                s_nb = nbod;
+                s_nmoved = L.nmoved;
+                if (L.overflow & 2) error |= 4;
+                L.overflow &= ~2;
+                s_np = 0;
+            }
         }
         __syncthreads();
         if (s_nb == 0) {
