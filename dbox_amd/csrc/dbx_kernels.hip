@@ -1833,53 +1833,6 @@ __device__ __forceinline__ float velocity_sweep(const int *Lbo, int nbatch, cons
     return lres;
 }
 
-// velocity_sweep with the accumulated impulses in the constraint records instead of
-// LDS, for islands whose impulses do not fit there: a slot's record comes with its
-// impulses two levels ahead, and the same lane stores them back after the solve, so
-// a lane reads in one sweep what it wrote in the sweep before.
-template <int kMode>
-__device__ __forceinline__ float velocity_sweep_far(const int *Lbo, int nbatch, VelCon *vc, float4 *Lvel, int lane) {
-    float lres = 0.0f;
-    auto one = [&](const VelCon &v, int k) {
-        float4 va = Lvel[v.indexA], vb = Lvel[v.indexB], im = make_float4(v.nImp0, v.tImp0, v.nImp1, v.tImp1);
-        asm volatile("" ::"v"(va.x), "v"(vb.x));
-        if (kMode == 0) warm_start_core(v, im, va, vb);
-        else lres = fmaxr(lres, solve_velocity_core<kMode == 2>(v, im, va, vb));
-        if (kMode != 0) *reinterpret_cast<float4 *>(&vc[k].nImp0) = im;
-        Lvel[v.indexA] = va;
-        Lvel[v.indexB] = vb;
-    };
-    auto level = [&](const VelCon &v, int k, bool have, int lo, int hi) {
-        if (have) one(v, k);
-        for (int c = lo + 64; c < hi; c += 64) { // levels wider than the wave
-            const int j2 = c + (int)(threadIdx.x & 63);
-            if (j2 < hi) {
-                const VelCon v2 = vc[j2];
-                one(v2, j2);
-            }
-        }
-    };
-    LevelWindow W{Lbo, nbatch + 1, 0, 0};
-    W.load(0);
-    int k0, k1, lo0, hi0, lo1, hi1;
-    bool h0, h1;
-    level_slot(W, 0, nbatch, lane, k0, h0, lo0, hi0);
-    VelCon v0 = vc[k0];
-    level_slot(W, 1, nbatch, lane, k1, h1, lo1, hi1);
-    VelCon v1 = vc[k1];
-    for (int bt = 0; bt < nbatch; bt += 2) {
-        W.cover(bt);
-        level(v0, k0, h0, lo0, hi0);
-        level_slot(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
-        v0 = vc[k0];
-        if (bt + 1 >= nbatch) break;
-        level(v1, k1, h1, lo1, hi1);
-        level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
-        v1 = vc[k1];
-    }
-    return lres;
-}
-
 // One sweep over the colours on every thread of the workgroup, a constraint per
 // thread, with the next colour's constraint loading while this one's is solved: a
 // barrier between colours.  (Constraints of one colour share no dynamic body.)
@@ -1935,6 +1888,79 @@ __device__ __forceinline__ void pipe_publish(int *Lnext, int me, int progress) {
     asm volatile("" ::: "memory");
     __hip_atomic_store(Lnext + 64 * me + (threadIdx.x & 63), progress, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// velocity_sweep with the accumulated impulses in the constraint records instead of
+// LDS, for islands whose impulses do not fit there: a slot's record comes with its
+// impulses two levels ahead, and the same lane stores them back after the solve, so
+// a lane reads in one sweep what it wrote in the sweep before.
+// With kPiped sweep s runs overlapped as in velocity_sweep_piped.  The next sweep also
+// reads the impulses that this one stores, so a level is published only once its store is
+// done: one level later, when the stores up to then are (vmcnt 1: all but the level's
+// own), and a record is loaded once the sweep before has published its level.
+struct FarPipe {
+    const int *Lneed;
+    int *Lnext;
+    int s, endProgress, me, prev;
+};
+template <int kMode, bool kPiped = false>
+__device__ __forceinline__ float velocity_sweep_far(const int *Lbo, int nbatch, VelCon *vc, float4 *Lvel, int lane,
+                                                    const FarPipe P = FarPipe{}, int *seen = nullptr) {
+    float lres = 0.0f;
+    auto one = [&](const VelCon &v, int k) {
+        float4 va = Lvel[v.indexA], vb = Lvel[v.indexB], im = make_float4(v.nImp0, v.tImp0, v.nImp1, v.tImp1);
+        asm volatile("" ::"v"(va.x), "v"(vb.x));
+        if (kMode == 0) warm_start_core(v, im, va, vb);
+        else lres = fmaxr(lres, solve_velocity_core<kMode == 2>(v, im, va, vb));
+        if (kMode != 0) *reinterpret_cast<float4 *>(&vc[k].nImp0) = im;
+        Lvel[v.indexA] = va;
+        Lvel[v.indexB] = vb;
+    };
+    LevelWindow W{Lbo, nbatch + 1, 0, 0}, N{P.Lneed, kPiped ? nbatch : 0, 0, 0};
+    const int base = kPiped && P.s > 0 ? (P.s - 1) * nbatch + 1 : INT_MIN / 2;
+    auto level = [&](int bt, const VelCon &v, int k, bool have, int lo, int hi) {
+        if (kPiped) pipe_wait(P.Lnext, P.prev, base + N.at(bt), *seen);
+        if (have) one(v, k);
+        for (int c = lo + 64; c < hi; c += 64) { // levels wider than the wave
+            const int j2 = c + (int)(threadIdx.x & 63);
+            if (j2 < hi) {
+                const VelCon v2 = vc[j2];
+                one(v2, j2);
+            }
+        }
+        if (kPiped) {
+            asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
+            pipe_publish(P.Lnext, P.me, P.s * nbatch + bt);
+            pipe_wait(P.Lnext, P.prev, base + min(bt + 2, nbatch - 1), *seen);
+        }
+    };
+    W.load(0);
+    if (kPiped) {
+        N.load(0);
+        pipe_wait(P.Lnext, P.prev, base + min(1, nbatch - 1), *seen);
+    }
+    int k0, k1, lo0, hi0, lo1, hi1;
+    bool h0, h1;
+    level_slot(W, 0, nbatch, lane, k0, h0, lo0, hi0);
+    VelCon v0 = vc[k0];
+    level_slot(W, 1, nbatch, lane, k1, h1, lo1, hi1);
+    VelCon v1 = vc[k1];
+    for (int bt = 0; bt < nbatch; bt += 2) {
+        W.cover(bt);
+        if (kPiped) N.cover(bt);
+        level(bt, v0, k0, h0, lo0, hi0);
+        level_slot(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
+        v0 = vc[k0];
+        if (bt + 1 >= nbatch) break;
+        level(bt + 1, v1, k1, h1, lo1, hi1);
+        level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
+        v1 = vc[k1];
+    }
+    if (kPiped) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        pipe_publish(P.Lnext, P.me, P.endProgress);
+    }
+    return lres;
 }
 
 // One sweep s of the overlapped velocity phase; Lneed holds need(l) per level, prev
@@ -2377,7 +2403,57 @@ __device__ __forceinline__ bool compact_velocity(const Dev &d, int cur, const St
     if (timed) d.ktime[39] = __builtin_amdgcn_s_memtime();
     const bool residualMode = (sp.flags & (1u << 5)) != 0;
     const int nbatch = C.nl;
-    if (tid < 64) {
+    // The sweeps overlap on up to four waves (as in solve_wave_world) where the schedule
+    // gains by it and LDS holds what it needs: an island of 3,400 bodies, 6,900
+    // constraints and 2,371 levels, whose sweeps trail each other by 1,516, takes 21.1
+    // million cycles of velocity iterations on one wave and 16.2 so.
+    int nact = 0;
+    const int ns = ((sp.flags & 1u) ? 1 : 0) + sp.velocityIterations;
+    int *Lneed = C.Lcur, *Llast = C.Lcur + isl_align(4 * (size_t)C.nl) / 4;
+    int *Lnext = Llast + isl_align(4 * (size_t)C.cb) / 4, *Llag = Lnext + 4 * 64;
+    if ((sp.flags & kStepPiped) && !residualMode && ns > 1 && nbatch > 1 && BS >= 128 &&
+        (size_t)((char *)(Llag + 1) - lds) <= (size_t)ldsBytes) {
+        for (int i = tid; i < C.cb; i += BS) Llast[i] = -1;
+        for (int i = tid; i < nbatch; i += BS) Lneed[i] = 0;
+        for (int i = tid; i < 4 * 64; i += BS) Lnext[i] = 0;
+        if (tid == 0) *Llag = 0;
+        __syncthreads();
+        for (int j = tid; j < nc; j += BS) {
+            const int dm = vc[j].dynMask, l = cbatch[C.sched[j]];
+            if (dm & 1) atomicMax(&Llast[vc[j].indexA], l);
+            if (dm & 2) atomicMax(&Llast[vc[j].indexB], l);
+        }
+        __syncthreads();
+        for (int j = tid; j < nc; j += BS) {
+            const int dm = vc[j].dynMask, l = cbatch[C.sched[j]];
+            const int e = max((dm & 1) ? Llast[vc[j].indexA] : 0, (dm & 2) ? Llast[vc[j].indexB] : 0);
+            atomicMax(&Lneed[l], e);
+            atomicMax(Llag, e - l);
+        }
+        __syncthreads();
+        const int lag = __builtin_amdgcn_readfirstlane(*Llag) + 2; // published a level late
+        const int waves = min(min(BS / 64, 4), (sp.flags & kStepPipedAlways) ? 4 : (nbatch + lag - 1) / lag);
+        const long long stride = max(lag, (nbatch + max(waves, 1) - 1) / max(waves, 1));
+        if (waves > 1 && ((sp.flags & kStepPipedAlways) || 10 * ((ns - 1) * stride + nbatch) <= 9ll * ns * nbatch))
+            nact = waves;
+    }
+    if (nact > 0) {
+        const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        int seen = 0;
+        for (int s = wave; s < ns && wave < nact; s += nact) {
+            const FarPipe P{Lneed, Lnext, s, s + nact < ns ? (s + nact) * nbatch : INT_MAX, wave,
+                            wave > 0 ? wave - 1 : nact - 1};
+            if ((sp.flags & 1u) && s == 0) velocity_sweep_far<0, true>(C.Lbo, nbatch, vc, C.Lbody, lane, P, &seen);
+            else velocity_sweep_far<1, true>(C.Lbo, nbatch, vc, C.Lbody, lane, P, &seen);
+            if (timed && s == 0) d.ktime[40] = __builtin_amdgcn_s_memtime();
+        }
+        if (tid == 0 && report) {
+            d.S[w].iterations = sp.velocityIterations;
+            d.S[w].residual = -1.0f;
+        }
+        __syncthreads();
+        if (timed) d.ktime[41] = __builtin_amdgcn_s_memtime();
+    } else if (tid < 64) {
         const int lane = tid;
         if (nbatch > 0 && (sp.flags & 1u)) velocity_sweep_far<0>(C.Lbo, nbatch, vc, C.Lbody, lane);
         if (timed) d.ktime[40] = __builtin_amdgcn_s_memtime();
