@@ -1065,6 +1065,15 @@ dbx_status dbx_finalize(dbx_handle *h) {
             }
             T.wideCount = (int)h->wide.size() - T.wideFirst;
         }
+        // Collide and broadphase take a contact or proxy per thread and pass, so a tier of
+        // bigger worlds that leaves CUs idle takes the widest workgroup: 64 worlds of 400
+        // bodies step in 775 us on 256 threads and 722 on 1,024, 4,096 containers of up to
+        // 1,100 bodies, whose lead tier this is, in 1,791 and 1,556.  With 160 bodies the
+        // two are alike, and 1,024 worlds of 160 lose (545 and 750 us, coloured).  A world
+        // with the device-wide broadphase has next to nothing left to do here.
+        if (h->cfg.block_size <= 0)
+            for (Tier &T : tiers)
+                if (T.wideCount == 0 && T.count <= h->cuCount && T.bodies > 128) T.block = kMaxBlock;
         // One launch per step for tiers of small worlds while every world has a CU of its
         // own (both sides measured at k_step).
         for (Tier &T : tiers) {
