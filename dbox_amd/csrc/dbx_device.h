@@ -102,23 +102,25 @@ struct alignas(16) Contact {
 };
 static_assert(sizeof(Contact) == 80, "contact layout");
 
-// b2ContactVelocityConstraint (b2contactsolver.d:43-58), 160 bytes.
+// b2ContactVelocityConstraint (b2contactsolver.d:43-58), 160 bytes.  What belongs to one
+// body is one run of 32 bytes, for the lane that solves that body's side (VelPair).
 struct alignas(16) VelCon {
-    float2 rA0, rB0;
-    float2 rA1, rB1;
+    float2 rA0, rA1;
+    float invMassA, invIA;
+    int indexA, contact;    // indices: world-local bodies
+    float2 rB0, rB1;
+    float invMassB, invIB;
+    int indexB, island;
     float nImp0, tImp0, nImp1, tImp1;
     float nMass0, tMass0, bias0, nMass1;
     float tMass1, bias1, friction, tangentSpeed;
-    float2 normal;
-    float invMassA, invMassB;
-    float invIA, invIB;
-    int indexA, indexB;     // world-local bodies
     float4 K;               // ex.x, ex.y, ey.x, ey.y
     float4 normalMass;      // ex.x, ex.y, ey.x, ey.y
-    int pointCount, contact, island, dynMask; // dynMask bit0/1: body A/B is dynamic
+    float2 normal;
+    int pointCount, dynMask; // dynMask bit0/1: body A/B is dynamic
 };
 static_assert(sizeof(VelCon) == 160, "velocity constraint layout");
-static_assert(offsetof(VelCon, nImp0) == 32, "impulses form one float4");
+static_assert(offsetof(VelCon, rB0) == 32 && offsetof(VelCon, nImp0) == 64, "body runs, impulses one float4");
 
 // b2ContactPositionConstraint (b2contactsolver.d:801-814) plus body indices, 96 bytes.
 struct alignas(16) PosCon {

@@ -191,6 +191,12 @@ __device__ __forceinline__ Xf mulT(const Xf &A, const Xf &B) {
 __device__ __forceinline__ int pair_swap(int x) { return __builtin_amdgcn_mov_dpp(x, 0xb1, 0xf, 0xf, true); }
 __device__ __forceinline__ float pair_swap(float x) { return __int_as_float(pair_swap(__float_as_int(x))); }
 __device__ __forceinline__ float2 pair_swap(float2 x) { return v2(pair_swap(x.x), pair_swap(x.y)); }
+// The even, and the odd, lane's value on both lanes of a pair.
+__device__ __forceinline__ int pair_even(int x) { return __builtin_amdgcn_mov_dpp(x, 0xa0, 0xf, 0xf, true); }
+__device__ __forceinline__ float pair_even(float x) { return __int_as_float(pair_even(__float_as_int(x))); }
+__device__ __forceinline__ float pair_odd(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xf5, 0xf, 0xf, true));
+}
 // Transform of a body from its centre of mass c, angle a and local centre lc.
 __device__ __forceinline__ Xf xf_from(float2 c, float a, float2 lc) {
     Xf x;
