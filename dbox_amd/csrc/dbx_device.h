@@ -122,15 +122,21 @@ struct alignas(16) VelCon {
 static_assert(sizeof(VelCon) == 160, "velocity constraint layout");
 static_assert(offsetof(VelCon, rB0) == 32 && offsetof(VelCon, nImp0) == 64, "body runs, impulses one float4");
 
-// b2ContactPositionConstraint (b2contactsolver.d:801-814) plus body indices, 96 bytes.
+// b2ContactPositionConstraint (b2contactsolver.d:801-814) plus body indices, 96 bytes; a
+// run of 32 bytes per body, as in VelCon.
 struct alignas(16) PosCon {
-    float2 lp0, lp1;
-    float2 localNormal, localPoint;
-    float2 lcA, lcB;
-    float invMassA, invMassB, invIA, invIB;
-    float radiusA, radiusB;
-    int type, pointCount;
-    int indexA, indexB, dynMask, island;
+    float2 lcA;
+    float invMassA, invIA;
+    float2 localPoint;
+    int indexA;
+    float radiusA;
+    float2 lcB;
+    float invMassB, invIB;
+    float2 lp0;
+    int indexB;
+    float radiusB;
+    float2 localNormal, lp1;
+    int type, pointCount, dynMask, island;
 };
 static_assert(sizeof(PosCon) == 96, "position constraint layout");
 
