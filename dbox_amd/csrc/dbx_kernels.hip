@@ -1858,9 +1858,9 @@ __device__ __forceinline__ float solve_position(const PosCon &p, int indexA, int
 }
 
 // ---------------------------------------------------------------------------
-// Exact-order solver: one wave per world.  Body positions, velocities and the
-// accumulated impulses live in LDS; the batches (dependency levels) are swept
-// one after another by the wave with no workgroup barrier: constraints of one
+// Exact-order solver: a wave per sweep.  Body positions, velocities and the
+// accumulated impulses live in LDS; the batches (dependency levels) of a sweep are
+// taken one after another by its wave with no workgroup barrier: constraints of one
 // level share no dynamic body, and the wave's LDS accesses complete in program
 // order, so level l+1 reads what level l wrote.  The static part of the next
 // level's constraint is loaded from global memory while the current level is
@@ -2186,9 +2186,9 @@ __device__ __forceinline__ void velocity_piped(const int *Lbo, const int *Lneed,
 // A position constraint of a TOI event gets two lanes (an even lane and the odd
 // lane after it), which compute the same constraint except that the even lane
 // evaluates b2Rot.Set of body A's angle and the odd lane of body B's, and the
-// two exchange the results (pair_swap): each lane then
-// holds both rotations for the cost of one.  The two lanes of a pair always take
-// the same branches, so both are active at every exchange.
+// two exchange the results (pair_swap): each lane then holds both rotations for the
+// cost of one.  The two lanes of a pair always take the same branches, so both are
+// active at every exchange.
 __device__ __forceinline__ void pair_xfs(float2 cA, float aA, float2 lcA, float2 cB, float aB, float2 lcB, Xf &xfA,
                                          Xf &xfB) {
     const bool odd = (threadIdx.x & 1) != 0;
