@@ -707,7 +707,7 @@ struct dbx_handle {
         size_t bytes = 0;
     } read, write;
     size_t writeAt = 0;
-    unsigned *signalHost = nullptr, *signalDev = nullptr, *signalCount = nullptr; // HostSignal's words
+    unsigned *signalCount = nullptr; // HostSignal's count; its flag lies behind read's bytes
     unsigned signalSeq = 0;
     double wallKHz = 100000.0;      // rate of the kernels' wall_clock64 stamps
     int cuCount = 0;                // compute units of the device
@@ -769,8 +769,10 @@ hipError_t pinned_reserve(dbx_handle *h, dbx_handle::Pinned &p, size_t bytes) {
     if (p.host) (void)hipHostFree(p.host);
     p = dbx_handle::Pinned{};
     const size_t n = std::max<size_t>((bytes + bytes / 2 + 4095) & ~(size_t)4095, 1u << 18);
-    e = pinned_alloc((void **)&p.host, (void **)&p.dev, n);
-    if (e == hipSuccess) p.bytes = n;
+    e = pinned_alloc((void **)&p.host, (void **)&p.dev, n + 64);
+    if (e != hipSuccess) return e;
+    p.bytes = n;
+    *(unsigned *)(p.host + n) = 0; // the flag of HostSignal
     return e;
 }
 // Runs launch(signal), a kernel that fills h->read (reserved to `bytes`) and signals,
@@ -781,19 +783,14 @@ hipError_t pinned_reserve(dbx_handle *h, dbx_handle::Pinned &p, size_t bytes) {
 template <class F>
 dbx_status pinned_read(dbx_handle *h, size_t bytes, F &&launch) {
     DBX_HIP(h, hipSetDevice(h->cfg.device));
-    if (!h->signalCount) {
-        if (!h->signalHost) {
-            DBX_HIP(h, pinned_alloc((void **)&h->signalHost, (void **)&h->signalDev, 64));
-            *h->signalHost = 0;
-        }
-        DBX_HIP(h, dalloc(h, &h->signalCount, 1));
-    }
-    DBX_HIP(h, pinned_reserve(h, h->read, bytes));
+    if (!h->signalCount) DBX_HIP(h, dalloc(h, &h->signalCount, 1));
+    DBX_HIP(h, pinned_reserve(h, h->read, std::max<size_t>(bytes, 1)));
+    const unsigned *flag = (const unsigned *)(h->read.host + h->read.bytes);
     const unsigned seq = ++h->signalSeq;
-    DBX_HIP(h, launch(HostSignal{h->signalDev, h->signalCount, seq}));
+    DBX_HIP(h, launch(HostSignal{(unsigned *)(h->read.dev + h->read.bytes), h->signalCount, seq}));
     constexpr int kSpins = 4000; // about 0.2 ms
     for (int i = 0; i < kSpins; ++i) {
-        if (__atomic_load_n(h->signalHost, __ATOMIC_ACQUIRE) == seq) {
+        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq) {
             h->writeAt = 0;
             return DBX_OK;
         }
@@ -801,7 +798,7 @@ dbx_status pinned_read(dbx_handle *h, size_t bytes, F &&launch) {
     }
     DBX_HIP(h, hipStreamSynchronize(h->stream));
     h->writeAt = 0;
-    if (__atomic_load_n(h->signalHost, __ATOMIC_ACQUIRE) != seq) return fail(h, DBX_E_HIP, "a read-back kernel did not finish");
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != seq) return fail(h, DBX_E_HIP, "a read-back kernel did not finish");
     return DBX_OK;
 }
 
@@ -865,7 +862,7 @@ void dbx_destroy(dbx_handle *h) {
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     mlp_release(h->mlp);
     for (void *p : h->allocs) (void)hipFree(p);
-    for (void *p : {(void *)h->read.host, (void *)h->write.host, (void *)h->signalHost})
+    for (void *p : {(void *)h->read.host, (void *)h->write.host})
         if (p) (void)hipHostFree(p);
     for (auto &e : h->ev)
         if (e) (void)hipEventDestroy(e);
