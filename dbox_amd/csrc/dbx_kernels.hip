@@ -5819,6 +5819,10 @@ __global__ __launch_bounds__(256) void k_bp1_scan(Bp1 b) {
 // Pairs are written only when all of them fit in cap; *total is the count either way.
 __global__ __launch_bounds__(128) void k_bp1_write(const float4 *__restrict__ fat, const int *__restrict__ moved, int n,
                                                    Bp1 b, int2 *__restrict__ out, int cap, int *__restrict__ total) {
+    if (n == 0) { // no cell to decode; the one workgroup launched reports the count
+        if (threadIdx.x == 0) *total = 0;
+        return;
+    }
     const int lane = threadIdx.x & 63;
     int blk, seg;
     bp1_cell(b, blockIdx.x, blk, seg);
@@ -5834,7 +5838,7 @@ __global__ __launch_bounds__(128) void k_bp1_write(const float4 *__restrict__ fa
         before += __shfl_xor(before, o, 64);
     }
     if (blk == 0 && seg == 0 && threadIdx.x == 0) *total = all < INT_MAX ? (int)all : INT_MAX;
-    if (all > cap || b.nblk == 0) return;
+    if (all > cap) return;
     const int tile = 2 * blk + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r0 = 128 * tile;
     const size_t t = (size_t)seg * 2 * b.nblk + tile;
     const int nh = __builtin_amdgcn_readfirstlane(b.nhit[t]);
