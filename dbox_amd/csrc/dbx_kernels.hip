@@ -13,6 +13,7 @@
 #include "dbx_device.h"
 #include "dbx_joints.h"
 #include "dbx_kernels.h"
+#include "dbx_sweeps.h"
 #include "dbx_toi.h"
 
 namespace dbx {
@@ -2628,11 +2629,12 @@ __device__ __forceinline__ bool compact_velocity(const Dev &d, int cur, const St
     // constraints and 2,371 levels, whose sweeps trail each other by 1,516, takes 21.1
     // million cycles of velocity iterations on one wave and 16.2 so.
     int nact = 0;
-    const int ns = ((sp.flags & 1u) ? 1 : 0) + sp.velocityIterations;
+    const long long ns = ((sp.flags & 1u) ? 1ll : 0ll) + sp.velocityIterations;
+    const int most = min(BS / 64, 4);
     int *Lneed = C.Lcur, *Llast = C.Lcur + isl_align(4 * (size_t)C.nl) / 4;
     int *Lnext = Llast + isl_align(4 * (size_t)C.cb) / 4, *Llag = Lnext + 4 * 64;
-    if ((sp.flags & kStepPiped) && !residualMode && ns > 1 && nbatch > 1 && BS >= 128 &&
-        (size_t)((char *)(Llag + 1) - lds) <= (size_t)ldsBytes) {
+    if ((sp.flags & kStepPiped) && !residualMode && ns > 1 && nbatch > 1 && most > 1 &&
+        sweeps_countable(ns, most, nbatch) && (size_t)((char *)(Llag + 1) - lds) <= (size_t)ldsBytes) {
         for (int i = tid; i < C.cb; i += BS) Llast[i] = -1;
         for (int i = tid; i < nbatch; i += BS) Lneed[i] = 0;
         for (int i = tid; i < 4 * 64; i += BS) Lnext[i] = 0;
@@ -2652,10 +2654,7 @@ __device__ __forceinline__ bool compact_velocity(const Dev &d, int cur, const St
         }
         __syncthreads();
         const int lag = __builtin_amdgcn_readfirstlane(*Llag) + 2; // published a level late
-        const int waves = min(min(BS / 64, 4), (sp.flags & kStepPipedAlways) ? 4 : (nbatch + lag - 1) / lag);
-        const long long stride = max(lag, (nbatch + max(waves, 1) - 1) / max(waves, 1));
-        if (waves > 1 && ((sp.flags & kStepPipedAlways) || 10 * ((ns - 1) * stride + nbatch) <= 9ll * ns * nbatch))
-            nact = waves;
+        nact = far_waves(ns, most, lag, nbatch, (sp.flags & kStepPipedAlways) != 0);
     }
     if (nact > 0) {
         const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -3363,7 +3362,7 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
     const int iters = residualMode ? sp.maxIterations : sp.velocityIterations;
     const size_t pipeBytes = isl_align(4 * (size_t)nb) + isl_align(4 * (size_t)nbatch) + 16 + 4 * (size_t)BS;
     const bool piped = !coloured && (sp.flags & kStepPiped) && BS >= 128 && nbatch > 0 &&
-                       (long long)(iters + kMaxSolveWaves + 1) * (nbatch + 1) < (1ll << 30) &&
+                       sweeps_countable(iters, kMaxSolveWaves, nbatch) &&
                        solve_lds_bytes(nb, nc, nbatch, nisl) + pipeBytes <= (size_t)ldsBytes;
     char *p = lds;
     float4 *Lvel = (float4 *)p; p += isl_align(16 * (size_t)nb);
@@ -3507,8 +3506,7 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
         const int waves =
             (sp.flags & kStepPipedAlways) ? BS / 64 : max(2, min(BS / 64, (nbatch + lag - 1) / lag));
         auto gains = [&](long long sweeps, int n) {
-            const long long stride = max(lag, (nbatch + n - 1) / n);
-            return (sp.flags & kStepPipedAlways) || 10 * ((sweeps - 1) * stride + nbatch) <= 9 * sweeps * nbatch;
+            return (sp.flags & kStepPipedAlways) || overlap_gains(sweeps, n, lag, nbatch);
         };
         const int ns = ((sp.flags & 1u) ? 1 : 0) + sp.velocityIterations;
         if (residualMode ? pipedPos && iters > 1 && gains(waves, waves) : ns > 1 && gains(ns, waves)) nact = waves;

@@ -2,7 +2,9 @@
 runs sweep s and waits on the wave before it), and on the GPU the overlapped steps
 against sequential ones, bit for bit, with fixed iteration counts and in the residual
 mode, whose batches of sweeps run past the iteration that ends them and roll back."""
+import os
 import random
+import subprocess
 
 import numpy as np
 import pytest
@@ -65,6 +67,42 @@ def test_protocol_keeps_every_body_in_order_and_finishes(waves):
     bad = [(k, r) for k in range(600) if (r := _run(k, waves))]
     assert not bad, bad[:5]
     assert sum(_run(k, waves, short=True) == "order" for k in range(300)) > 50
+
+
+RULES = """#include <cstdio>
+#include <cstdlib>
+#include "%s"
+int main(int, char **v) {
+    const int levels = atoi(v[1]), lag = atoi(v[2]);
+    for (int most = 2; most <= 8; ++most)
+        for (int always = 0; always < 2; ++always) {
+            // the largest sweep count that still overlaps, by bisection over dbx_step's range
+            long long lo = 1, hi = (1ll << 31) + 1;
+            while (hi - lo > 1) {
+                const long long mid = (lo + hi) / 2;
+                (dbx::far_waves(mid, most, lag, levels, always) > 0 ? lo : hi) = mid;
+            }
+            printf("%%d %%lld %%d %%d\\n", most, lo, dbx::far_waves(lo, most, lag, levels, always),
+                   dbx::far_waves((1ll << 31) - 1, most, lag, levels, always));
+        }
+}
+"""
+
+
+@pytest.mark.parametrize("levels,lag", [(2, 2), (59, 4), (2371, 1518), (3017, 900), (60000, 2), (1 << 22, 5)])
+def test_overlap_rule_keeps_the_progress_count_in_an_int(levels, lag, tmp_path):
+    header = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "dbox_amd", "csrc", "dbx_sweeps.h")
+    src, exe = tmp_path / "rules.cpp", tmp_path / "rules"
+    src.write_text(RULES % header)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-o", str(exe), str(src)], check=True)
+    out = subprocess.run([str(exe), str(levels), str(lag)], capture_output=True, text=True, check=True).stdout
+    overlapped = 0
+    for most, sweeps, waves, at_limit in (map(int, ln.split()) for ln in out.splitlines()):
+        assert at_limit == 0 and waves <= most
+        # the largest value published, the start of a sweep past the last, and the largest waited for
+        assert (sweeps + waves) * levels + levels < 2 ** 31
+        overlapped += waves > 0
+    assert overlapped or lag >= levels
 
 
 def _handles(ws):
