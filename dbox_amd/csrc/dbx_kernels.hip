@@ -3561,7 +3561,8 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
         if (sp.flags & 1u) colour_sweep<0>(Lbo, nbatch, vc, Lvel, Limp);
         if (timed && tid == 0) d.ktime[6] = __builtin_amdgcn_s_memtime();
         prof.at(kProfVel0);
-        int used = 0;
+        // without a constraint an iteration has nothing to do and a residual of 0
+        int used = nbatch > 0 ? 0 : (residualMode && sp.residualTol >= 0.0f ? min(iters, 1) : iters);
         float lastRes = residualMode ? 0.0f : -1.0f;
         for (int it = 0; it < iters && nbatch > 0; ++it) {
             ++used;

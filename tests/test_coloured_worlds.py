@@ -38,3 +38,22 @@ def test_coloured_worlds_equal_the_colour_order_oracle(dense, warm, residual):
                 m = body_mismatch(h.bodies(w), o.bodies(), o.bodies_def["type"]) or contact_mismatch(h.contacts(w),
                                                                                                        o.contacts())
                 assert m is None, f"step {i + 1}, world {w}: {m}"
+
+
+@pytest.mark.parametrize("fill", [0, 1100])  # in one launch, and a launch per phase
+def test_iterations_reported_without_a_constraint(fill):
+    print(f"case: iteration counts of coloured worlds in free fall, {fill} more worlds", flush=True)
+    h = native.StepWorlds()
+    for s in [scenes.hello_world(), scenes.pyramid(3)] + [scenes.hello_world()] * fill:
+        h.add_scene(s)
+    h.finalize()
+    h.step(DT, 5, 3, native.WARM, n=1)
+    it, _ = h.solver_stats()
+    assert len(h.contacts(0)) == 0 and it[0] == 5 and it[1] == 5 and h.residuals()[0] == -1.0
+    for tol, most, want in ((-1.0, 7, 7), (0.0, 7, 1), (1e-3, 1, 1), (1e-3, 30, 1)):
+        h.set_residual(tol, most)
+        h.step(DT, 8, 3, native.WARM | native.RESIDUAL, n=1)
+        it, _ = h.solver_stats()
+        assert it[0] == want and h.residuals()[0] == 0.0, (tol, most, it[0])
+        assert tol >= 0.0 or it[1] == most
+    h.close()
