@@ -1487,6 +1487,7 @@ static dbx_status tune_account(dbx_handle *h) {
     }
     if (++h->tuneDone < h->tuneSteps) return DBX_OK;
     for (size_t t = 0; t < h->tiers.size(); ++t) {
+        if (h->tiers[t].stepLds) continue; // its one-launch step has no width to tune
         int best = 0;
         for (int k = 1; k < kTuneCandidates; ++k)
             if (h->tuneMs[t * kTuneCandidates + k] < h->tuneMs[t * kTuneCandidates + best]) best = k;
@@ -1583,7 +1584,8 @@ dbx_status dbx_step(dbx_handle *h, float dt, int32_t vel, int32_t pos, uint32_t 
     const bool tuning = h->tuneDone < h->tuneSteps;
     if (tuning) {
         const int c = h->tuneDone / h->tunePer;
-        for (Tier &T : h->tiers) T.block = kTuneBlocks[c];
+        for (Tier &T : h->tiers)
+            if (!T.stepLds) T.block = kTuneBlocks[c];
     }
     // DBX_TIER_TIMES (diagnostics): time every tier's chain; each step then waits
     // for its own end, so the steps no longer overlap the host
@@ -2569,8 +2571,9 @@ dbx_status dbx_autotune(dbx_handle *h, int32_t steps_per_candidate) {
         if (!T.t0) DBX_HIP(h, hipEventCreate(&T.t0));
         if (!T.t1) DBX_HIP(h, hipEventCreate(&T.t1));
     }
+    const bool any = std::any_of(h->tiers.begin(), h->tiers.end(), [](const Tier &T) { return T.stepLds == 0; });
     h->tunePer = steps_per_candidate;
-    h->tuneSteps = steps_per_candidate * kTuneCandidates;
+    h->tuneSteps = any ? steps_per_candidate * kTuneCandidates : 0;
     h->tuneDone = 0;
     h->tuneMs.assign(h->tiers.size() * kTuneCandidates, 0.0);
     return DBX_OK;

@@ -205,7 +205,9 @@ typedef struct {
 typedef struct {
     int32_t device;                 /* HIP device ordinal */
     int32_t contacts_per_fixture;   /* contact capacity per fixture (0 = 8) */
-    int32_t block_size;             /* threads per world workgroup (0 = autotuned default) */
+    int32_t block_size;             /* threads per world workgroup (0 = a default per tier, which
+                                       dbx_autotune can improve); of no effect on tiers that step
+                                       as one kernel (see dbx_read_tiers) */
     int32_t use_graph;              /* replay each step as a captured hipGraph (one per distinct
                                        step parameters and buffer parity) */
 } dbx_config;
@@ -336,7 +338,11 @@ dbx_status dbx_read_toi_events(dbx_handle *h, int32_t *events, int32_t nworlds);
  * their step chain on a stream of their own.  Writes (first launch slot, world
  * count, LDS bytes, workgroup size) per tier into tiers[4 * i .. 4 * i + 3] for
  * up to cap tiers, the launch order (world index per slot) into order when it
- * is not null (nworlds entries), and the tier count into count. */
+ * is not null (nworlds entries), and the tier count into count.  A tier whose
+ * largest world has at most 128 bodies, in a handle with no more worlds than the
+ * device has compute units, steps as one kernel of 256 threads per world unless a
+ * world needs more LDS than that kernel has; the workgroup size kept for it is
+ * then used by the broadphase of a handle's first step alone. */
 dbx_status dbx_read_tiers(dbx_handle *h, int32_t *tiers, int32_t cap, int32_t *order, int32_t *count);
 
 /* Launch-shape autotuner (no counterpart in the reference).  The next
@@ -345,13 +351,15 @@ dbx_status dbx_read_tiers(dbx_handle *h, int32_t *tiers, int32_t cap, int32_t *o
  * and 1024 threads in turn, timing each tier's step chain on its own stream;
  * after the last of them each tier keeps its fastest size (dbx_read_tiers shows
  * it).  Results never depend on the workgroup size, so tuning steps are
- * ordinary steps.  Those steps are not captured as graphs. */
+ * ordinary steps.  Those steps are not captured as graphs.  A tier that steps as
+ * one kernel has no size to tune and keeps the one it has; where every tier does,
+ * no step is timed. */
 dbx_status dbx_autotune(dbx_handle *h, int32_t steps_per_candidate);
 /* Turns the hipGraph replay of dbx_config.use_graph on or off for later steps.
  * Replayed steps record only the step's total time in dbx_profile. */
 dbx_status dbx_set_graph(dbx_handle *h, int32_t enabled);
 /* Sets the workgroup size of each tier (n = tier count), e.g. from a cache of
- * earlier autotuning. */
+ * earlier autotuning; of no effect on the steps of a tier that steps as one kernel. */
 dbx_status dbx_set_tier_blocks(dbx_handle *h, const int32_t *blocks, int32_t n);
 
 /* The island solve order of the last step for one world: for each constraint in

@@ -29,3 +29,28 @@ def test_default_width_keeps_results(name, ordered):
     for w in range(0, len(ws), 17 if name == "many" else 1):
         for read in ("bodies", "contacts", "pairs"):
             assert getattr(hs[0], read)(w).tobytes() == getattr(hs[1], read)(w).tobytes(), (w, read)
+
+
+def test_autotuner_leaves_one_launch_tiers_alone():
+    box = lambda n, k: scenes.mixed_container(n, 3.0 + n ** 0.5, 6.0 + 2.0 * n ** 0.5, k)
+    flags = native.WARM | native.SLEEP | native.CCD | native.ORDERED
+    # only one-launch tiers, and one beside a tier with a width to tune
+    for ws, tuned in (([box(100, 1), box(20, 2)], 0), ([box(700, 3), box(20, 4)], 1)):
+        print(f"case: autotuner over {[len(s.bodies) for s in ws]} bodies", flush=True)
+        hs = [native.StepWorlds(), native.StepWorlds()]
+        for h in hs:
+            for s in ws:
+                h.add_scene(s)
+            h.finalize()
+        rows, _ = hs[0].tiers()
+        for width in (64, 512, 1024, 128, 64, 1024):
+            hs[0].set_tier_blocks([width] * len(rows))
+            hs[0].autotune(1)
+            for h in hs:
+                h.step(1.0 / 60.0, 8, 3, flags, n=5)
+                h.sync()
+            assert set(hs[0].tiers()[0][tuned:, 3]) == {width}
+        for w in range(len(ws)):
+            assert hs[0].bodies(w).tobytes() == hs[1].bodies(w).tobytes()
+        for h in hs:
+            h.close()
