@@ -261,7 +261,10 @@ dbx_status dbx_read_bodies(dbx_handle *h, int32_t world, dbx_body_state *out, in
  * order), and, when force3 is not null, its force and torque (3 floats per body,
  * the accumulators the next step integrates and then clears).  Fixtures whose
  * fat AABB no longer contains the new pose are re-fattened and moved, as
- * b2Fixture.Synchronize(xf, xf) does after SetTransform. */
+ * b2Fixture.Synchronize(xf, xf) does after SetTransform.  `in` and force3 are copied
+ * before the call returns and applied in order on the handle's stream: the call does
+ * not wait for that, so a failure on the device is reported by a later call that
+ * waits (dbx_sync or a read). */
 dbx_status dbx_write_bodies(dbx_handle *h, int32_t world, const dbx_body_state *in, const float *force3, int32_t n);
 /* For each proxy of one world (see "Proxy indices" above): its fixture's creation
  * index and its child index.  *count = proxies; nothing is written when cap is smaller. */
@@ -312,9 +315,9 @@ dbx_status dbx_profile_read(dbx_handle *h, dbx_profile *out);
 dbx_status dbx_profile_totals(dbx_handle *h, dbx_profile *sum, int32_t *steps, int32_t reset);
 /* Launch-level timing (no counterpart in the reference): milliseconds of the lead
  * tier's phases, from HIP events on its stream (or timed inside its one-launch steps),
- * summed over the eager steps resolved by dbx_sync since the last reset, in the order Collide, island search, island
- * solve, broadphase (SynchronizeFixtures + FindNewContacts), continuous pass; *steps
- * = steps summed.  The other tiers run beside the lead tier. */
+ * summed over the eager steps resolved by dbx_sync since the last reset, in the order
+ * Collide, island search, island solve, broadphase (SynchronizeFixtures +
+ * FindNewContacts), continuous pass; *steps = steps summed.  The other tiers run beside the lead tier. */
 dbx_status dbx_phase_totals(dbx_handle *h, float *ms5, int32_t *steps, int32_t reset);
 /* Totals over all worlds: dynamic bodies, contacts, touching contacts, awake bodies. */
 dbx_status dbx_totals(dbx_handle *h, int64_t out[4]);
@@ -356,7 +359,8 @@ dbx_status dbx_read_tiers(dbx_handle *h, int32_t *tiers, int32_t cap, int32_t *o
  * no step is timed. */
 dbx_status dbx_autotune(dbx_handle *h, int32_t steps_per_candidate);
 /* Turns the hipGraph replay of dbx_config.use_graph on or off for later steps.
- * Replayed steps record only the step's total time in dbx_profile. */
+ * Replayed steps record the step's total time and the phases timed inside kernels
+ * only (dbx_profile). */
 dbx_status dbx_set_graph(dbx_handle *h, int32_t enabled);
 /* Sets the workgroup size of each tier (n = tier count), e.g. from a cache of
  * earlier autotuning; of no effect on the steps of a tier that steps as one kernel. */
@@ -368,7 +372,9 @@ dbx_status dbx_set_tier_blocks(dbx_handle *h, const int32_t *blocks, int32_t n);
 dbx_status dbx_read_schedule(dbx_handle *h, int32_t world, int32_t *out, int32_t cap, int32_t *count);
 
 /* Stand-alone broadphase (b2BroadPhase.UpdatePairs semantics) on given fat
- * AABBs and moved flags of n proxies; pairs are written sorted as (i, j), i < j. */
+ * AABBs and moved flags of n proxies; pairs are written sorted as (i, j), i < j.
+ * Allocates its device buffers for the call: up to about 540 bytes per proxy and 8 per
+ * pair of cap. */
 dbx_status dbx_broadphase_pairs(dbx_handle *h, const float *fat_aabbs, const uint8_t *moved, int32_t n,
                                 int32_t *out, int32_t cap, int32_t *count);
 /* Stand-alone broadphase that allocates nothing.  No counterpart in the reference:
@@ -379,7 +385,7 @@ dbx_status dbx_broadphase_pairs(dbx_handle *h, const float *fat_aabbs, const uin
  * pairs (cap pairs of 2 int32, (i, j) with i < j, in b2PairLessThan order) is
  * written only when the pair count fits in cap; *count (device int32) receives the
  * pair count.  Asynchronous on the handle's stream (dbx_sync waits).  The working
- * memory is a fixed array of the library on each GPU, sized for at most
+ * memory is a fixed array of the library on each GPU (8.25 MiB), sized for at most
  * DBX_NOALLOC_MAX_PROXIES proxies (DBX_E_CAPACITY above that); it holds the last
  * call's data, and calls that overlap on one GPU (from other streams, handles or
  * threads) race on it. */
