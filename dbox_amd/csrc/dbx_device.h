@@ -166,6 +166,7 @@ struct JointRec; // dbx_joints.h
 struct Dev {
     int nworlds;
     const int *order;       // launch order of worlds (largest first)
+    const int *jointOrder;  // the worlds with joints in that order
     const WorldDesc *W;
     WorldState *S;
     // bodies

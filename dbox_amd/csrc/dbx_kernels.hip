@@ -3311,18 +3311,17 @@ __global__ __launch_bounds__(256) void k_solve(Dev d, int cur, StepParams sp, in
     solve_world_global<false>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, ldsBytes, ProfStamp{});
 }
 
-// The worlds of a tier that have joints, in either solver mode: one island per lane in
-// the reference's sequence.  An island is a serial chain, so what bounds it is the latency
-// of each load of a body, constraint or joint: they lie in LDS where they fit, and the
-// islands are dealt over the waves, since the lanes of one wave wait for each other's
-// joint kinds.  64 worlds of some 44 bodies and 25 joints: 312 us a step from global
-// memory with the islands on one wave, 197 so.
+// Worlds that have joints, in either solver mode: one island per lane in the reference's
+// sequence.  An island is a serial chain, so what bounds it is the latency of each load of
+// a body, constraint or joint: they lie in LDS where they fit, and the islands are dealt
+// over the waves, since the lanes of one wave wait for each other's joint kinds.  64
+// worlds of some 44 bodies and 25 joints: 312 us a step from global memory with the
+// islands on one wave, 197 so.
 template <bool kLead>
-__global__ __launch_bounds__(256) void k_solve_joint(Dev d, int cur, StepParams sp, int worldOffset, int ldsBytes) {
+__global__ __launch_bounds__(256) void k_solve_joint(Dev d, int cur, StepParams sp, int first, int ldsBytes) {
     extern __shared__ __align__(16) char lds[];
-    const int w = d.order[worldOffset + blockIdx.x];
-    if (d.W[w].jointCount == 0) return;
-    solve_world_global<true>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, ldsBytes, ProfStamp{});
+    const int w = d.jointOrder[first + blockIdx.x];
+    solve_world_global<true>(d, cur, sp, w, w == d.order[0], lds, ldsBytes, ProfStamp{});
 }
 
 // One big world's islands on G workgroups, each solving the islands that hold a
@@ -3342,12 +3341,11 @@ constexpr int kMaxSolveWaves = 8;
 __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const StepParams &sp, int worldOffset, int w,
                                                  char *lds, int ldsBytes, ProfStamp prof) {
     const WorldDesc wd = d.W[w];
-    if (solve_grouped(d, sp, wd)) return;
+    if (solve_grouped(d, sp, wd) || wd.jointCount > 0) return;
     const int nb = wd.bodyCount, nf = wd.fixCount;
     const int nc = d.S[w].constraints;
     const int nbatch = d.S[w].batchCount;
     const int nisl = d.S[w].islandCount;
-    if (wd.jointCount > 0) return; // k_solve_joint
     const bool coloured = (sp.flags & kStepColoured) != 0;
     if (solve_lds_bytes(nb, nc, nbatch, nisl) > (size_t)ldsBytes) {
         solve_world_global<false>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, coloured ? 0 : ldsBytes, prof);
@@ -3787,6 +3785,22 @@ template <bool kLead>
 __global__ __launch_bounds__(64 * kMaxSolveWaves) void k_solve_wave(Dev d, int cur, StepParams sp, int worldOffset, int ldsBytes) {
     extern __shared__ __align__(16) char lds[];
     solve_wave_world(d, cur, sp, worldOffset, d.order[worldOffset + blockIdx.x], lds, ldsBytes, ProfStamp{});
+}
+
+// A tier in which some worlds have joints: both solves in one launch, so that the long
+// chains of the joint worlds run beside the other worlds' sweeps.  300 worlds of 90 bodies
+// and one of joints: 574 us a step with the joints in k_solve_wave's own kernel, from global
+// memory, 660 with k_solve_joint after k_solve_wave, 428 so; 1,500 of 320 bodies and one of
+// 400 pieces: 14.7, 20.7 and 14.2 ms.
+template <bool kLead>
+__global__ __launch_bounds__(64 * kMaxSolveWaves) void k_solve_mixed(Dev d, int cur, StepParams sp, int worldOffset,
+                                                                     int ldsBytes) {
+    extern __shared__ __align__(16) char lds[];
+    const int w = d.order[worldOffset + blockIdx.x];
+    if (d.W[w].jointCount > 0)
+        solve_world_global<true>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, ldsBytes, ProfStamp{});
+    else
+        solve_wave_world(d, cur, sp, worldOffset, w, lds, ldsBytes, ProfStamp{});
 }
 
 // ---------------------------------------------------------------------------
@@ -6187,6 +6201,9 @@ static hipError_t configure_tier(int maxDynamicLds) {
     e = hipFuncSetAttribute((const void *)k_step<kLead>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             maxDynamicLds - 1024);
     if (e != hipSuccess) return e;
+    e = hipFuncSetAttribute((const void *)k_solve_mixed<kLead>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            maxDynamicLds - 1024);
+    if (e != hipSuccess) return e;
     e = hipFuncSetAttribute((const void *)k_solve_joint<kLead>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             maxDynamicLds - 1024);
     if (e != hipSuccess) return e;
@@ -6260,13 +6277,20 @@ hipError_t launch_step(const Dev &d, int cin, const StepParams &sp, int worldOff
     DBX_LAUNCH(k_step, lead, dim3(nworlds), dim3(256), ldsBytes, s, d, cin, sp, worldOffset, ldsBytes, what);
     return hipGetLastError();
 }
+hipError_t launch_solve_mixed(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, int waves,
+                              int ldsBytes, bool lead, hipStream_t s) {
+    if (nworlds <= 0) return hipSuccess;
+    if (waves < 1 || waves > kMaxSolveWaves) return hipErrorInvalidValue;
+    DBX_LAUNCH(k_solve_mixed, lead, dim3(nworlds), dim3(64 * waves), ldsBytes, s, d, cur, sp, worldOffset, ldsBytes);
+    return hipGetLastError();
+}
 size_t solve_joint_lds_bytes(int bodies, int constraints, int joints) {
     return joint_lds_bytes(bodies, constraints, joints);
 }
-hipError_t launch_solve_joint(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, int ldsBytes,
-                              bool lead, hipStream_t s) {
+hipError_t launch_solve_joint(const Dev &d, int cur, const StepParams &sp, int first, int nworlds, int ldsBytes, bool lead,
+                              hipStream_t s) {
     if (nworlds <= 0) return hipSuccess;
-    DBX_LAUNCH(k_solve_joint, lead, dim3(nworlds), dim3(256), ldsBytes, s, d, cur, sp, worldOffset, ldsBytes);
+    DBX_LAUNCH(k_solve_joint, lead, dim3(nworlds), dim3(256), ldsBytes, s, d, cur, sp, first, ldsBytes);
     return hipGetLastError();
 }
 size_t broadphase_scratch_bytes(int proxies) { return bp_bytes(proxies); }

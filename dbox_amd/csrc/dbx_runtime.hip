@@ -642,8 +642,9 @@ struct Tier {
     hipEvent_t t0 = nullptr, t1 = nullptr; // chain timing while autotuning
     bool own = false;         // stream and event created for this tier
     int jointLds = 0;         // LDS of its joint solve (0: no world of it has joints)
+    int mixedLds = 0;         // LDS of the launch that solves its worlds with and without joints (0: all or none have joints)
     int stepLds = 0;          // LDS of its one-launch step (0: a launch per phase)
-    int jointWorlds = 0;      // worlds with joints
+    int jointFirst = 0, jointWorlds = 0; // its worlds with joints (range in Dev.jointOrder)
     int wideFirst = 0, wideCount = 0; // its worlds whose broadphase runs device-wide (range in the handle's list)
 };
 
@@ -1021,6 +1022,7 @@ dbx_status dbx_finalize(dbx_handle *h) {
     std::vector<int> order(nw);
     for (int w = 0; w < nw; ++w) order[w] = w;
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return need[a] > need[b]; });
+    std::vector<int> jointOrder;
     {
         std::vector<int> sizes = {h->ldsMax};
         for (int l : {81920, 40960, 20480})
@@ -1045,9 +1047,13 @@ dbx_status dbx_finalize(dbx_handle *h) {
         for (Tier &T : tiers) {
             const int lds1 = std::min(T.lds, h->ldsMax - 1024);
             T.wideFirst = (int)h->wide.size();
+            T.jointFirst = (int)jointOrder.size();
+            int jointBodies = 0, otherBodies = 0; // of its largest world with and without joints
             for (int i = T.first; i < T.first + T.count; ++i) {
                 WorldDesc &D = h->W[order[i]];
-                T.jointWorlds += D.jointCount > 0 ? 1 : 0;
+                if (D.jointCount > 0) jointOrder.push_back(order[i]);
+                int &most = D.jointCount > 0 ? jointBodies : otherBodies;
+                most = std::max(most, D.bodyCount);
                 if (D.jointCount > 0) // room for two solved contacts per fixture
                     T.jointLds = std::max(T.jointLds, (int)std::min<size_t>(h->ldsMax - 1024,
                                                           solve_joint_lds_bytes(D.bodyCount, 2 * D.fixCount, D.jointCount)));
@@ -1061,6 +1067,21 @@ dbx_status dbx_finalize(dbx_handle *h) {
                 h->wide.push_back(b);
             }
             T.wideCount = (int)h->wide.size() - T.wideFirst;
+            T.jointWorlds = (int)jointOrder.size() - T.jointFirst;
+            // Joint worlds beside the others in one launch (both sides measured at k_solve_mixed),
+            // with LDS for the joint worlds' state where the extra rounds of workgroups that it
+            // means cost the others less than it saves the joint worlds, some 3 to 5 us a body and
+            // round against 10 to 15 us a body: 1,500 worlds of 60 bodies and 60 of joints, two
+            // rounds more, step in 884 us with it and 1,181 without; 1,500 of 200 bodies and one of
+            // 184 with joints, three more, in 5.25 ms and 4.83.
+            if (T.jointWorlds > 0 && T.jointWorlds < T.count) {
+                const int lds = std::max(lds1, T.jointLds);
+                const auto rounds = [&](int bytes) {
+                    const int atOnce = std::max(h->cuCount, 1) * (h->ldsMax / bytes);
+                    return (T.count + atOnce - 1) / atOnce;
+                };
+                T.mixedLds = (long long)(rounds(lds) - rounds(lds1)) * otherBodies <= 3ll * jointBodies ? lds : lds1;
+            }
         }
         // Collide and broadphase take a contact or proxy per thread and pass, so a tier of
         // bigger worlds that leaves CUs idle takes the widest workgroup: 64 worlds of 400
@@ -1088,14 +1109,17 @@ dbx_status dbx_finalize(dbx_handle *h) {
 
     Dev &d = h->d;
     d.nworlds = nw;
-    int *dOrder;
+    int *dOrder, *dJointOrder;
     WorldDesc *dW;
     DBX_HIP(h, dalloc(h, &dOrder, nw));
+    DBX_HIP(h, dalloc(h, &dJointOrder, jointOrder.size()));
+    DBX_HIP(h, upload(h, dJointOrder, jointOrder));
     DBX_HIP(h, dalloc(h, &dW, nw));
     DBX_HIP(h, dalloc(h, &d.S, nw));
     DBX_HIP(h, hipMemcpyAsync(dOrder, order.data(), nw * sizeof(int), hipMemcpyHostToDevice, h->stream));
     DBX_HIP(h, hipMemcpyAsync(dW, h->W.data(), nw * sizeof(WorldDesc), hipMemcpyHostToDevice, h->stream));
     d.order = dOrder;
+    d.jointOrder = dJointOrder;
     d.W = dW;
     // bodies
     std::vector<uint32_t> bflags;
@@ -1361,14 +1385,21 @@ static dbx_status step_tier(dbx_handle *h, int t, const StepParams &sp, uint32_t
         // Solved with the state in LDS, except for a tier of worlds too big for that (all
         // with the device-wide broadphase): island groups in the exact order, colour
         // batches from global memory in the coloured mode.
-        if (T.jointWorlds < T.count) {
-            if (T.wideCount < T.count)
-                DBX_HIP(h, launch_solve_wave(d, cout, sp, T.first, T.count,
-                                             ordered ? solve_waves(h, T, lead) : std::min(T.block / 64, 8), lds1, lead, s));
-            else
-                DBX_HIP(h, launch_solve(d, cout, sp, T.first, T.count, ordered ? 256 : T.block, ordered ? lds1 : 0, lead, s));
+        const int waves = ordered ? solve_waves(h, T, lead) : std::min(T.block / 64, 8);
+        // Without that LDS the coloured mode, whose other worlds take little time, solves the
+        // joint worlds in a launch of their own: 3.4 ms for the 1,500 worlds of 200 bodies, 4.4 in one.
+        if (T.mixedLds && (ordered || T.mixedLds >= T.jointLds)) {
+            DBX_HIP(h, launch_solve_mixed(d, cout, sp, T.first, T.count, waves, T.mixedLds, lead, s));
+        } else {
+            if (T.jointWorlds < T.count) {
+                if (T.wideCount < T.count)
+                    DBX_HIP(h, launch_solve_wave(d, cout, sp, T.first, T.count, waves, lds1, lead, s));
+                else
+                    DBX_HIP(h, launch_solve(d, cout, sp, T.first, T.count, ordered ? 256 : T.block, ordered ? lds1 : 0,
+                                            lead, s));
+            }
+            DBX_HIP(h, launch_solve_joint(d, cout, sp, T.jointFirst, T.jointWorlds, T.jointLds, lead, s));
         }
-        if (T.jointLds) DBX_HIP(h, launch_solve_joint(d, cout, sp, T.first, T.count, T.jointLds, lead, s));
         if (ordered && T.wideCount && d.iwParent && (sp.flags & kStepGrouped))
             DBX_HIP(h, launch_solve_groups(d, cout, sp, wide, T.wideCount, lds1, lead, s));
         if (timed) (void)hipEventRecord(ev[3], s);

@@ -41,3 +41,41 @@ def test_joint_worlds_equal_the_oracle(sizes, warm):
             assert h.joints(w).tobytes() == o.joints().tobytes(), f"{label}: joints"
             m = contact_mismatch(h.contacts(w), o.contacts())
             assert m is None, f"{label}: {m}"
+
+
+# joint worlds beside others in the same tier: (other worlds, their bodies, debris of the joint worlds)
+MIXES = {
+    "few": (300, 20, [0, 12, 40]),
+    "larger LDS for all": (280, 200, [150, 170]),
+    "too many rounds for that": (2000, 200, [150, 170]),  # joints from global memory, or (coloured) a launch of their own
+}
+
+
+@pytest.mark.parametrize("mode", ["exact", "coloured", "residual"])
+@pytest.mark.parametrize("mix", list(MIXES))
+def test_joint_worlds_among_others_equal_them_alone(mix, mode):
+    print(f"case: joint worlds in a mixed tier, {mix}, {mode}", flush=True)
+    others, size, debris = MIXES[mix]
+    box = [scenes.mixed_container(size, 3.0 + size ** 0.5, 6.0 + 2.0 * size ** 0.5, k) for k in range(4)]
+    ws = [_scattered(n) for n in debris] + [box[k % 4] for k in range(others)]
+    flags = native.WARM | native.SLEEP | {"exact": native.ORDERED, "coloured": 0,
+                                          "residual": native.ORDERED | native.RESIDUAL}[mode]
+
+    def run(ws):
+        h = native.StepWorlds(contacts_per_fixture=16)
+        for s in ws:
+            h.add_scene(s)
+        h.finalize()
+        h.set_residual(1e-2, 20)
+        h.step(DT, 8, 3, flags, n=15)
+        h.sync()
+        return h
+
+    mixed = run(ws)
+    for w in range(len(debris) + 4):
+        alone = run([ws[w]])
+        for read in ("bodies", "contacts", "joints"):
+            assert getattr(mixed, read)(w).tobytes() == getattr(alone, read)(0).tobytes(), f"world {w}: {read}"
+        assert mixed.solver_stats()[0][w] == alone.solver_stats()[0][0] and mixed.residuals()[w] == alone.residuals()[0]
+        alone.close()
+    mixed.close()
