@@ -218,6 +218,10 @@ class StepWorlds:
     def world_count(self):
         return len(self.body_counts)
 
+    def _proxies(self, world):
+        """Proxies of a world; 0 for a world that is not there, which the library's own check then refuses."""
+        return self.fixture_counts[world] if 0 <= world < len(self.fixture_counts) else 0
+
     def bodies(self, world=0) -> np.ndarray:
         out = np.empty(self.body_counts[world], BODY_STATE_DTYPE)
         self._check(self.L.dbx_read_bodies(self.h, world, _p(out), len(out)))
@@ -225,7 +229,7 @@ class StepWorlds:
 
     def contacts(self, world=0) -> np.ndarray:
         n = C.c_int32()
-        out = np.empty(4 * self.fixture_counts[world] + 64, CONTACT_DTYPE)  # nearly always enough: one read
+        out = np.empty(4 * self._proxies(world) + 64, CONTACT_DTYPE)  # nearly always enough: one read
         self._check(self.L.dbx_read_contacts(self.h, world, _p(out), len(out), C.byref(n)))
         if n.value > len(out):
             out = np.empty(n.value, CONTACT_DTYPE)
@@ -235,7 +239,7 @@ class StepWorlds:
     def events(self, world=0) -> np.ndarray:
         """The b2ContactListener callbacks of the last step (dbx_read_events), in dbox's order."""
         n = C.c_int32()
-        out = np.empty(8 * self.fixture_counts[world] + 64, EVENT_DTYPE)  # nearly always enough: one read
+        out = np.empty(8 * self._proxies(world) + 64, EVENT_DTYPE)  # nearly always enough: one read
         st = self.L.dbx_read_events(self.h, world, _p(out), len(out), C.byref(n))
         if st == DBX_E_CAPACITY and n.value > len(out):
             out = np.empty(n.value, EVENT_DTYPE)

@@ -81,3 +81,13 @@ def test_reads_that_outgrow_the_pinned_memory():
     assert st == native.DBX_E_CAPACITY and n.value == len(ev) and not short.view(np.uint8).any()
     assert len(h.bodies(0)) == 4001
     h.close()
+
+
+def test_reads_of_a_world_that_is_not_there_are_refused_by_the_library():
+    h = _handle([scenes.pyramid(3)])
+    for world in (1, 7, -1):
+        for read in (h.contacts, h.events):
+            with pytest.raises(native.DbxError):
+                read(world)
+    assert len(h.contacts(0)) == 0 and len(h.events(0)) == 0
+    h.close()
