@@ -1,14 +1,18 @@
 """A small world's step in one launch against the same step in a launch per phase, bit for
 bit: the same worlds in a handle of their own and in one with more worlds than the
-one-launch step takes.  Every mode, split steps, steps of no time and sizes on both
+one-launch step takes.  Every solver mode, split steps, steps of no time and sizes on both
 sides of the body limit; the phase times of the profile."""
+import os
+
 import numpy as np
 import pytest
 
-from dbox_amd import native, scenes
+import dbox_amd
+from dbox_amd import native, scenes, warmstart
 
 pytestmark = pytest.mark.gpu
 DT = 1.0 / 60.0
+NETWORK = os.path.join(os.path.dirname(os.path.abspath(dbox_amd.__file__)), "learned", "warmstart_c12.npz")
 BASE = native.WARM | native.SLEEP
 MODES = {
     "default": BASE | native.CCD | native.ORDERED,
@@ -16,6 +20,8 @@ MODES = {
     "coloured": BASE | native.CCD,
     "cold": native.CCD | native.ORDERED,
     "residual": BASE | native.ORDERED | native.RESIDUAL,
+    "learned": BASE | native.ORDERED | native.RESIDUAL | native.LEARNED,
+    "learned, fixed iterations": BASE | native.CCD | native.ORDERED | native.LEARNED,
     "split": BASE | native.CCD | native.ORDERED | native.PRESOLVE,
 }
 
@@ -45,6 +51,8 @@ def test_one_launch_equals_separate_launches(mode, graph):
     flags = MODES[mode]
     for h in hs:
         h.set_residual(1e-3, 30)
+        if flags & native.LEARNED:
+            h.mlp_set(*warmstart.load_network(NETWORK)[:2])
     events = 0
     for i in range(40):
         for h in hs:
