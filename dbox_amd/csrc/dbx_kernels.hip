@@ -824,7 +824,7 @@ __device__ void island_search_joints(const Dev &d, int cur, int w, const WorldDe
         const int g = wd.bodyBase + b;
         M.fl[b] = (int)f;
         M.isl[b] = -1;
-        // a static body's edges are not followed
+        // (a static body's ranges are staged too, but it is never reached)
         M.ao[b] = make_int2(d.adjOff[g], d.adjCnt[g]);
         M.jo[b] = make_int2(d.jadjOff[g], d.jadjCnt[g]);
     }
@@ -1909,10 +1909,9 @@ struct LevelWindow {
     __device__ __forceinline__ int at(int i) const { return __builtin_amdgcn_readlane(reg, i - base); }
 };
 
-// This lane's slot in level bt: constraints are stored in schedule order, so
-// the slot is the constraint; a lane without one reads slot 0 so that the loads
-// issued for it stay in bounds.  kPair: two lanes per constraint.
-template <int kPair = 0>
+// This lane pair's slot in level bt: constraints are stored in schedule order, so
+// the slot is the constraint; a pair without one reads slot 0 so that the loads
+// issued for it stay in bounds.
 __device__ __forceinline__ void level_slot(const LevelWindow &W, int bt, int nbatch, int lane, int &k, bool &have,
                                            int &lo, int &hi) {
     lo = 0;
@@ -1921,7 +1920,7 @@ __device__ __forceinline__ void level_slot(const LevelWindow &W, int bt, int nba
         lo = W.at(bt);
         hi = W.at(bt + 1);
     }
-    const int j = lo + (lane >> kPair);
+    const int j = lo + (lane >> 1);
     have = j < hi;
     k = have ? j : 0;
 }
@@ -1962,18 +1961,18 @@ __device__ __forceinline__ float velocity_sweep(const int *Lbo, int nbatch, cons
     W.load(0);
     int k0, k1, lo0, hi0, lo1, hi1;
     bool h0, h1;
-    level_slot<1>(W, 0, nbatch, lane, k0, h0, lo0, hi0);
+    level_slot(W, 0, nbatch, lane, k0, h0, lo0, hi0);
     VelPair c0 = load_pair(vc, k0);
-    level_slot<1>(W, 1, nbatch, lane, k1, h1, lo1, hi1);
+    level_slot(W, 1, nbatch, lane, k1, h1, lo1, hi1);
     VelPair c1 = load_pair(vc, k1);
     for (int bt = 0; bt < nbatch; bt += 2) {
         W.cover(bt);
         velocity_level<kMode>(c0, k0, h0, lo0, hi0, vc, Lvel, Limp, lres);
-        level_slot<1>(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
+        level_slot(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
         c0 = load_pair(vc, k0);
         if (bt + 1 >= nbatch) break;
         velocity_level<kMode>(c1, k1, h1, lo1, hi1, vc, Lvel, Limp, lres);
-        level_slot<1>(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
+        level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
         c1 = load_pair(vc, k1);
     }
     return lres;
@@ -2094,19 +2093,19 @@ __device__ __forceinline__ float velocity_sweep_far(const int *Lbo, int nbatch, 
     }
     int k0, k1, lo0, hi0, lo1, hi1;
     bool h0, h1;
-    level_slot<1>(W, 0, nbatch, lane, k0, h0, lo0, hi0);
+    level_slot(W, 0, nbatch, lane, k0, h0, lo0, hi0);
     VelPair v0 = load_pair(vc, k0);
-    level_slot<1>(W, 1, nbatch, lane, k1, h1, lo1, hi1);
+    level_slot(W, 1, nbatch, lane, k1, h1, lo1, hi1);
     VelPair v1 = load_pair(vc, k1);
     for (int bt = 0; bt < nbatch; bt += 2) {
         W.cover(bt);
         if (kPiped) N.cover(bt);
         level(bt, v0, k0, h0, lo0, hi0);
-        level_slot<1>(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
+        level_slot(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
         v0 = load_pair(vc, k0);
         if (bt + 1 >= nbatch) break;
         level(bt + 1, v1, k1, h1, lo1, hi1);
-        level_slot<1>(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
+        level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
         v1 = load_pair(vc, k1);
     }
     if (kPiped) {
@@ -2132,9 +2131,9 @@ __device__ __forceinline__ float velocity_sweep_piped(const int *Lbo, const int 
     const int mine = s * nbatch;
     int k0, k1, lo0, hi0, lo1, hi1;
     bool h0, h1;
-    level_slot<1>(W, 0, nbatch, lane, k0, h0, lo0, hi0);
+    level_slot(W, 0, nbatch, lane, k0, h0, lo0, hi0);
     VelPair c0 = load_pair(vc, k0);
-    level_slot<1>(W, 1, nbatch, lane, k1, h1, lo1, hi1);
+    level_slot(W, 1, nbatch, lane, k1, h1, lo1, hi1);
     VelPair c1 = load_pair(vc, k1);
     for (int bt = 0; bt < nbatch; bt += 2) {
         W.cover(bt);
@@ -2142,13 +2141,13 @@ __device__ __forceinline__ float velocity_sweep_piped(const int *Lbo, const int 
         pipe_wait(Lnext, prev, base + N.at(bt), seen);
         velocity_level<kMode>(c0, k0, h0, lo0, hi0, vc, Lvel, Limp, lres);
         pipe_publish(Lnext, me, bt + 1 < nbatch ? mine + bt + 1 : endProgress);
-        level_slot<1>(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
+        level_slot(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
         c0 = load_pair(vc, k0);
         if (bt + 1 >= nbatch) break;
         pipe_wait(Lnext, prev, base + N.at(bt + 1), seen);
         velocity_level<kMode>(c1, k1, h1, lo1, hi1, vc, Lvel, Limp, lres);
         pipe_publish(Lnext, me, bt + 2 < nbatch ? mine + bt + 2 : endProgress);
-        level_slot<1>(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
+        level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
         c1 = load_pair(vc, k1);
     }
     return lres;
@@ -2342,18 +2341,18 @@ __device__ __forceinline__ void position_sweep(const int *Lbo, int nbatch, const
     W.load(0);
     int k0, k1, lo0, hi0, lo1, hi1;
     bool h0, h1;
-    level_slot<1>(W, 0, nbatch, lane, k0, h0, lo0, hi0);
+    level_slot(W, 0, nbatch, lane, k0, h0, lo0, hi0);
     PosPair c0 = load_pair(pc, k0);
-    level_slot<1>(W, 1, nbatch, lane, k1, h1, lo1, hi1);
+    level_slot(W, 1, nbatch, lane, k1, h1, lo1, hi1);
     PosPair c1 = load_pair(pc, k1);
     for (int bt = 0; bt < nbatch; bt += 2) {
         W.cover(bt);
         position_level(c0, h0, lo0, hi0, pc, Lpos, Lmin, Lsol);
-        level_slot<1>(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
+        level_slot(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
         c0 = load_pair(pc, k0);
         if (bt + 1 >= nbatch) break;
         position_level(c1, h1, lo1, hi1, pc, Lpos, Lmin, Lsol);
-        level_slot<1>(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
+        level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
         c1 = load_pair(pc, k1);
     }
 }
@@ -2428,9 +2427,9 @@ __device__ __forceinline__ void position_sweep_piped(const int *Lbo, const int *
     const int mine = s * nbatch;
     int k0, k1, lo0, hi0, lo1, hi1;
     bool h0, h1;
-    level_slot<1>(W, 0, nbatch, lane, k0, h0, lo0, hi0);
+    level_slot(W, 0, nbatch, lane, k0, h0, lo0, hi0);
     PosPair c0 = load_pair(pc, k0);
-    level_slot<1>(W, 1, nbatch, lane, k1, h1, lo1, hi1);
+    level_slot(W, 1, nbatch, lane, k1, h1, lo1, hi1);
     PosPair c1 = load_pair(pc, k1);
     for (int bt = 0; bt < nbatch; bt += 2) {
         W.cover(bt);
@@ -2438,13 +2437,13 @@ __device__ __forceinline__ void position_sweep_piped(const int *Lbo, const int *
         pipe_wait(Lnext, prev, base + N.at(bt), seen);
         position_level_piped(c0, k0, h0, lo0, hi0, pc, Lpos, LminS, Lver, skip, Lflag, Lbak);
         if (bt + 1 < nbatch) pipe_publish(Lnext, me, mine + bt + 1); // the last level: after the test
-        level_slot<1>(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
+        level_slot(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
         c0 = load_pair(pc, k0);
         if (bt + 1 >= nbatch) break;
         pipe_wait(Lnext, prev, base + N.at(bt + 1), seen);
         position_level_piped(c1, k1, h1, lo1, hi1, pc, Lpos, LminS, Lver, skip, Lflag, Lbak);
         if (bt + 2 < nbatch) pipe_publish(Lnext, me, mine + bt + 2);
-        level_slot<1>(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
+        level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
         c1 = load_pair(pc, k1);
     }
 }
@@ -5001,8 +5000,8 @@ __device__ __forceinline__ void toi_pass(const Dev &d, int cur, const StepParams
     auto &s_bestPos = T.bestPos;
     int &s_err = T.err, &s_nb = T.nb, &s_np = T.np, &s_n = T.n, &s_nsnap = T.nsnap, &s_nmoved = T.nmoved, &s_ncand = T.ncand;
     const WorldDesc wd = d.W[w];
-    // the lead tier runs four waves per world, the other tiers one; the events
-    // themselves run on thread 0
+    // the lead tier and a step in one launch run four waves per world, the other tiers
+    // one; the events themselves run on wave 0
     const int tid = threadIdx.x, BS = blockDim.x, lane = tid & 63, wave = tid >> 6;
     LdsFloat2 *verts = (LdsFloat2 *)(s_verts + kVertStride * tid);
     const ToiWorld W = toi_world(d, cur, w, wd);
