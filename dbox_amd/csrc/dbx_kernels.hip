@@ -1494,7 +1494,7 @@ struct VelPair {
     float nMass0, tMass0, bias0, nMass1, tMass1, bias1, friction, tangentSpeed;
     float4 K, normalMass;
     float2 normal;
-    int pointCount;
+    int pointCount, sides; // sides: dynMask
 };
 __device__ __forceinline__ VelPair load_pair(const VelCon *vc, int k) {
     const bool odd = (threadIdx.x & 1) != 0;
@@ -1520,6 +1520,7 @@ __device__ __forceinline__ VelPair load_pair(const VelCon *vc, int k) {
     p.normalMass = v.normalMass;
     p.normal = v.normal;
     p.pointCount = v.pointCount;
+    p.sides = v.dynMask;
     return p;
 }
 // The relative velocity at the point with this lane's lever r.
@@ -2021,8 +2022,8 @@ __device__ __forceinline__ float colour_sweep(const int *Lbo, int nbatch, const 
 // levels (the largest need(l) - l, plus one), so N = levels / lag waves keep every
 // wave busy and more would only wait.  In a pile some body's contacts spread over
 // half the levels or more (two waves); in a tall stack a body meets its two
-// neighbours in consecutive levels, and eight sweeps run at once: 128 stack worlds
-// iterated to a residual take 5.4 ms a step in one wave's sweeps and 0.9 in eight's.
+// neighbours in consecutive levels, and eight sweeps could run at once: 128 stack worlds
+// iterated to a residual take 4.73 ms a step in one wave's sweeps and 0.97 in four's.
 __device__ __forceinline__ void pipe_wait(const int *Lnext, int other, int need, int &seen) {
     while (seen < need)
         seen = __builtin_amdgcn_readfirstlane(__hip_atomic_load(Lnext + 64 * other + (threadIdx.x & 63),
@@ -2116,9 +2117,9 @@ __device__ __forceinline__ float velocity_sweep_far(const int *Lbo, int nbatch, 
 }
 
 // One sweep s of the overlapped velocity phase; Lneed holds need(l) per level, prev
-// is the wave of sweep s - 1.  Returns the lane's residual (kMode 2).
+// is the wave of sweep s - 1.
 template <int kMode>
-__device__ __forceinline__ float velocity_sweep_piped(const int *Lbo, const int *Lneed, int nbatch,
+__device__ __forceinline__ void velocity_sweep_piped(const int *Lbo, const int *Lneed, int nbatch,
                                                      const VelCon *__restrict__ vc, float4 *Lvel, float4 *Limp,
                                                      int lane, int s, int endProgress, int *Lnext, int me,
                                                      int prev, int &seen) {
@@ -2150,17 +2151,14 @@ __device__ __forceinline__ float velocity_sweep_piped(const int *Lbo, const int 
         level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
         c1 = load_pair(vc, k1);
     }
-    return lres;
 }
 
 // The warm start (when warm is set) and nvel velocity iterations, overlapped on the
 // workgroup's first nact waves.  Lnext: 64 ints of LDS per wave that hold 0 on entry.
-// kMode 2: Lres[i] receives iteration i's residual.  Stamps the warm start's end (or
-// the velocity phase's start) through prof.
-template <int kMode>
+// Stamps the warm start's end (or the velocity phase's start) through prof.
 __device__ __forceinline__ void velocity_piped(const int *Lbo, const int *Lneed, int nbatch,
                                                const VelCon *__restrict__ vc, float4 *Lvel, float4 *Limp, int *Lnext,
-                                               int nact, bool warm, int nvel, float *Lres, const ProfStamp &prof) {
+                                               int nact, bool warm, int nvel, const ProfStamp &prof) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nsweeps = (warm ? 1 : 0) + nvel, prev = wave > 0 ? wave - 1 : nact - 1;
     int seen = 0;
@@ -2172,15 +2170,135 @@ __device__ __forceinline__ void velocity_piped(const int *Lbo, const int *Lneed,
             velocity_sweep_piped<0>(Lbo, Lneed, nbatch, vc, Lvel, Limp, lane, s, endProgress, Lnext, wave, prev, seen);
             prof.at(kProfVel0);
         } else {
-            float r = velocity_sweep_piped<kMode>(Lbo, Lneed, nbatch, vc, Lvel, Limp, lane, s, endProgress, Lnext, wave,
-                                                  prev, seen);
-            if (kMode == 2) {
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) r = fmaxr(r, __shfl_xor(r, o, 64));
-                if (lane == 0) Lres[s - (warm ? 1 : 0)] = r;
-            }
+            velocity_sweep_piped<1>(Lbo, Lneed, nbatch, vc, Lvel, Limp, lane, s, endProgress, Lnext, wave, prev, seen);
         }
     }
+}
+
+// Overlapped sweeps of the residual mode.  A sweep's residual is known at its end, when the
+// later sweeps are under way, so each wave keeps velocities and impulses of its own: sweep
+// s reads a body before its first update, and a constraint's impulses, from the wave of
+// sweep s - 1 and leaves the rest to itself.  The sweep that ends the step leaves its
+// number in Lstop (the least of them counts); a later one gives up when it next looks, and
+// what it wrote belongs to nobody.  A wave's own values last until its next sweep, which
+// it does not begin after the sweep that ends the step, and which, by the waits, writes a
+// body or impulse only after the sweep in between has read it.  (With one set of values for all waves, and a copy of it from
+// before each batch of N sweeps to run a batch again that went too far, a step that ended
+// after its first iteration ran two batches: 300 containers of 125 bodies took 756 us where
+// one sweep after the other takes 613 and this 618, 64 of 90 bodies 500, 415 and 418; 128
+// stack worlds that need some 64 iterations took 1.10 ms and take 0.97.)
+struct SweepState {
+    float4 *L;             // LDS; the rest are places in it
+    int base;              // the velocities before the first sweep, and those of bodies that no sweep changes
+    int prevVel, prevImp;  // of the sweep before
+    int vel, imp;          // of this sweep
+};
+template <int kMode>
+__device__ __forceinline__ void velocity_level_owned(const VelPair &p, int k, bool have, int lo, int hi,
+                                                     const VelCon *__restrict__ vc, const SweepState &S, float &lres) {
+    // bits of a record's sides: 0 and 1 the body is dynamic, 2 and 3 this is its first update
+    const int base = S.base, dPrev = S.prevVel - S.base, dVel = S.vel - S.base;
+    const auto from = [=](int bits) { return base + (bits & 1 ? (bits & 4 ? dPrev : dVel) : 0); };
+    if (hi - lo <= 32) {
+        if (have) {
+            const int bits = p.sides >> (threadIdx.x & 1);
+            float4 vel = S.L[from(bits) + p.index], im = S.L[S.prevImp + k];
+            asm volatile("" ::"v"(vel.x), "v"(im.x)); // one LDS round trip
+            if (kMode == 0) warm_start_pair(p, im, vel);
+            else lres = fmaxr(lres, solve_velocity_pair<true>(p, im, vel));
+            S.L[S.imp + k] = im;
+            if (bits & 1) S.L[S.vel + p.index] = vel;
+        }
+        return;
+    }
+    for (int c = lo; c < hi; c += 64) { // a lane per constraint, as in velocity_level
+        const int j = c + (int)(threadIdx.x & 63);
+        if (j >= hi) continue;
+        const VelCon v = vc[j];
+        const int a = v.dynMask, b = v.dynMask >> 1;
+        float4 va = S.L[from(a) + v.indexA], vb = S.L[from(b) + v.indexB], im = S.L[S.prevImp + j];
+        if (kMode == 0) warm_start_core(v, im, va, vb);
+        else lres = fmaxr(lres, solve_velocity_core<true>(v, im, va, vb));
+        S.L[S.imp + j] = im;
+        if (a & 1) S.L[S.vel + v.indexA] = va;
+        if (b & 1) S.L[S.vel + v.indexB] = vb;
+    }
+}
+// One sweep s of it; false when it gave up.  lres: the lane's residual (kMode 2).
+template <int kMode>
+__device__ __forceinline__ bool velocity_sweep_owned(const int *Lbo, const int *Lneed, int nbatch,
+                                                     const VelCon *__restrict__ vc, const SweepState &S, int lane, int s,
+                                                     int endProgress, int *Lnext, int me, int prev, int &seen,
+                                                     const int *Lstop, float &lres) {
+    LevelWindow W{Lbo, nbatch + 1, 0, 0}, N{Lneed, nbatch, 0, 0};
+    W.load(0);
+    N.load(0);
+    const int base = s > 0 ? (s - 1) * nbatch + 1 : INT_MIN / 2;
+    const int mine = s * nbatch;
+    int k0, k1, lo0, hi0, lo1, hi1;
+    bool h0, h1;
+    level_slot(W, 0, nbatch, lane, k0, h0, lo0, hi0);
+    VelPair c0 = load_pair(vc, k0);
+    level_slot(W, 1, nbatch, lane, k1, h1, lo1, hi1);
+    VelPair c1 = load_pair(vc, k1);
+    for (int bt = 0; bt < nbatch; bt += 2) {
+        if ((bt & 7) == 0 && __builtin_amdgcn_readfirstlane(__hip_atomic_load(Lstop, __ATOMIC_RELAXED,
+                                                                              __HIP_MEMORY_SCOPE_WORKGROUP)) < s)
+            return false;
+        W.cover(bt);
+        N.cover(bt);
+        pipe_wait(Lnext, prev, base + N.at(bt), seen);
+        velocity_level_owned<kMode>(c0, k0, h0, lo0, hi0, vc, S, lres);
+        pipe_publish(Lnext, me, bt + 1 < nbatch ? mine + bt + 1 : endProgress);
+        level_slot(W, bt + 2, nbatch, lane, k0, h0, lo0, hi0);
+        c0 = load_pair(vc, k0);
+        if (bt + 1 >= nbatch) break;
+        pipe_wait(Lnext, prev, base + N.at(bt + 1), seen);
+        velocity_level_owned<kMode>(c1, k1, h1, lo1, hi1, vc, S, lres);
+        pipe_publish(Lnext, me, bt + 2 < nbatch ? mine + bt + 2 : endProgress);
+        level_slot(W, bt + 3, nbatch, lane, k1, h1, lo1, hi1);
+        c1 = load_pair(vc, k1);
+    }
+    return true;
+}
+// The warm start (when warm is set) and up to iters iterations until the residual is at
+// most tol, on the workgroup's first nact waves.  S: base, and prevVel and prevImp of the
+// state before; each wave's velocities (nb of them) and impulses (nc) lie at own + wave *
+// (nb + nc).  Lres: each wave's last residual; Lstop holds INT_MAX on entry, Lnext 0.
+__device__ __forceinline__ void velocity_to_residual(const int *Lbo, const int *Lneed, int nbatch,
+                                                     const VelCon *__restrict__ vc, SweepState S, int own, int nb, int nc,
+                                                     int *Lnext, int nact, bool warm, int iters, float tol, float *Lres,
+                                                     int *Lstop, const ProfStamp &prof) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int nsweeps = (warm ? 1 : 0) + iters, prev = wave > 0 ? wave - 1 : nact - 1;
+    int seen = 0;
+    if (!warm) prof.at(kProfVel0);
+    if (wave >= nact) return;
+    S.vel = own + wave * (nb + nc);
+    S.imp = S.vel + nb;
+    for (int s = wave; s < nsweeps; s += nact) {
+        const int endProgress = s + nact < nsweeps ? (s + nact) * nbatch : INT_MAX;
+        if (s > 0) {
+            S.prevVel = own + prev * (nb + nc);
+            S.prevImp = S.prevVel + nb;
+        }
+        float r = 0.0f;
+        if (warm && s == 0) {
+            velocity_sweep_owned<0>(Lbo, Lneed, nbatch, vc, S, lane, s, endProgress, Lnext, wave, prev, seen, Lstop, r);
+            prof.at(kProfVel0);
+            continue;
+        }
+        if (!velocity_sweep_owned<2>(Lbo, Lneed, nbatch, vc, S, lane, s, endProgress, Lnext, wave, prev, seen, Lstop, r))
+            break;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) r = fmaxr(r, __shfl_xor(r, o, 64));
+        if (lane == 0) {
+            Lres[wave] = r;
+            if (r <= tol) atomicMin(Lstop, s);
+        }
+        if (r <= tol) break;
+    }
+    pipe_publish(Lnext, wave, INT_MAX); // nobody waits for a sweep that gave up or will not be
 }
 
 // A position constraint of a TOI event gets two lanes (an even lane and the odd
@@ -3355,7 +3473,7 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
     // overlapped sweeps: several waves, per body the level of its last constraint
     // (Llast), per level need(l) (Lneed) and the published progress (Lnext)
     __shared__ float s_res[kMaxSolveWaves];
-    __shared__ int s_worst;
+    __shared__ int s_worst, s_stop;
     const int iters = residualMode ? sp.maxIterations : sp.velocityIterations;
     const size_t pipeBytes = isl_align(4 * (size_t)nb) + isl_align(4 * (size_t)nbatch) + 16 + 4 * (size_t)BS;
     const bool piped = !coloured && (sp.flags & kStepPiped) && BS >= 128 && nbatch > 0 &&
@@ -3387,6 +3505,12 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
     int *Lmin2 = (int *)p; p += isl_align(4 * (size_t)nisl);
     int *Lver = (int *)p; p += isl_align(4 * (size_t)nisl);
     int *Lnext2 = (int *)p;
+    // the residual mode's overlapped sweeps: velocities and impulses per wave, in the place
+    // of the position iterations' arrays from Lbak1 on
+    const size_t ownAt = solve_lds_bytes(nb, nc, nbatch, nisl) + pipeBytes + isl_align(4 * (size_t)nb) + isl_align(4 * (size_t)nc);
+    const int ownWaves =
+        residualMode && piped && ownAt < (size_t)ldsBytes ? (int)(((size_t)ldsBytes - ownAt) / (16 * ((size_t)nb + nc))) : 0;
+    const bool firsts = pipedPos || ownWaves > 1;
 
     Contact *cont = d.cont[cur] + wd.contactBase;
     const float *ctan = d.ctan[cur] + wd.contactBase;
@@ -3424,10 +3548,8 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
         Lnext[tid] = 0;
         if (tid == 0) Llag[0] = 0;
     }
-    if (pipedPos) {
+    if (firsts)
         for (int b = tid; b < nb; b += BS) Lfirst[b] = INT_MAX;
-        Lnext2[tid] = 0;
-    }
     // Integrate velocities with damping (b2island.d:82-116) while staging the bodies.
     for (int b = tid; b < nb; b += BS) {
         const float4 pos = bpos[b], vel = bvel[b];
@@ -3470,7 +3592,7 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
             const int l = cbatch[k];
             if (v.dynMask & 1) atomicMax(&Llast[v.indexA], l);
             if (v.dynMask & 2) atomicMax(&Llast[v.indexB], l);
-            if (pipedPos) {
+            if (firsts) {
                 if (v.dynMask & 1) atomicMin(&Lfirst[v.indexA], l);
                 if (v.dynMask & 2) atomicMin(&Lfirst[v.indexB], l);
             }
@@ -3489,69 +3611,48 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
             const int e = max((dm & 1) ? Llast[ia] : 0, (dm & 2) ? Llast[ib] : 0);
             atomicMax(&Lneed[l], e);
             atomicMax(Llag, e - l);
+            if (ownWaves > 1) // SweepState's bits
+                vc[j].dynMask = dm | ((dm & 1) && Lfirst[ia] == l ? 4 : 0) | ((dm & 2) && Lfirst[ib] == l ? 8 : 0);
             if (pipedPos) { // the position constraint's bodies, in its own order
                 const int pm = pc[j].dynMask, pa = pc[j].indexA, pb = pc[j].indexB;
                 Lflag[j] = ((pm & 1) && Lfirst[pa] == l ? 1 : 0) | ((pm & 2) && Lfirst[pb] == l ? 2 : 0);
             }
         }
         __syncthreads();
-        // a sweep starts at least lag levels after the one before it and `waves`
-        // sweeps after it on the same wave: overlapped only when that gains a tenth.
-        // The residual mode overlaps one sweep per wave and keeps its start in the
-        // position phase's first backup.
+        // overlapped where that gains a tenth (overlap_gains)
         const int lag = __builtin_amdgcn_readfirstlane(Llag[0]) + 1;
         const int waves =
             (sp.flags & kStepPipedAlways) ? BS / 64 : max(2, min(BS / 64, (nbatch + lag - 1) / lag));
         auto gains = [&](long long sweeps, int n) {
             return (sp.flags & kStepPipedAlways) || overlap_gains(sweeps, n, lag, nbatch);
         };
-        const int ns = ((sp.flags & 1u) ? 1 : 0) + sp.velocityIterations;
-        if (residualMode ? pipedPos && iters > 1 && gains(waves, waves) : ns > 1 && gains(ns, waves)) nact = waves;
+        const long long ns = ((sp.flags & 1u) ? 1ll : 0ll) + iters;
+        const int velWaves = residualMode ? min(waves, ownWaves) : waves;
+        if (velWaves > 1 && ns > 1 && gains(ns, velWaves)) nact = velWaves;
         posWaves = pipedPos && gains(3, min(waves, 3)) ? min(waves, 3) : 0;
+        if (tid == 0) s_stop = INT_MAX;
+        __syncthreads();
     }
     if (nact > 0 && !residualMode) {
-        velocity_piped<1>(Lbo, Lneed, nbatch, vc, Lvel, Limp, Lnext, nact, (sp.flags & 1u) != 0, sp.velocityIterations,
-                          nullptr, prof);
+        velocity_piped(Lbo, Lneed, nbatch, vc, Lvel, Limp, Lnext, nact, (sp.flags & 1u) != 0, sp.velocityIterations, prof);
         if (tid == 0) {
             d.S[w].iterations = sp.velocityIterations;
             d.S[w].residual = -1.0f;
         }
         if (timed && lane == 0 && wave < 2) d.ktime[6 + wave] = __builtin_amdgcn_s_memtime(); // its last sweep done
     } else if (nact > 0) {
-        // Residual mode, a batch of one iteration per wave at a time: the batch runs
-        // past the iteration whose residual ends the step, if it holds one, so its start
-        // is kept (velocities in Lbak1, impulses in the constraint records) and a batch
-        // that went too far is run again from there up to that iteration.
-        int used = 0;
-        float lastRes = 0.0f;
-        bool warm = (sp.flags & 1u) != 0;
-        while (used < iters) {
-            const int n = min(nact, iters - used);
-            for (int b = tid; b < nb; b += BS) Lbak1[b] = Lvel[b];
-            for (int k = tid; k < nc; k += BS) *reinterpret_cast<float4 *>(&vc[k].nImp0) = Limp[k];
-            __syncthreads();
-            velocity_piped<2>(Lbo, Lneed, nbatch, vc, Lvel, Limp, Lnext, nact, warm, n, s_res,
-                              used == 0 ? prof : ProfStamp{});
-            __syncthreads();
-            int last = 0;
-            while (last < n && !(s_res[last] <= sp.residualTol)) ++last;
-            const bool stop = last < n;
-            lastRes = s_res[stop ? last : n - 1];
-            Lnext[tid] = 0;
-            if (stop && last + 1 < n) {
-                for (int b = tid; b < nb; b += BS) Lvel[b] = Lbak1[b];
-                for (int k = tid; k < nc; k += BS) Limp[k] = *reinterpret_cast<const float4 *>(&vc[k].nImp0);
-                __syncthreads();
-                velocity_piped<1>(Lbo, Lneed, nbatch, vc, Lvel, Limp, Lnext, nact, warm, last + 1, nullptr, ProfStamp{});
-            }
-            used += stop ? last + 1 : n;
-            warm = false;
-            __syncthreads();
-            if (stop) break;
-        }
+        const int warm = (sp.flags & 1u) ? 1 : 0, own = (int)(ownAt / 16), imp0 = (int)(Limp - Lvel);
+        velocity_to_residual(Lbo, Lneed, nbatch, vc, SweepState{Lvel, 0, 0, imp0, 0, 0}, own, nb, nc, Lnext, nact, warm != 0,
+                             iters, sp.residualTol, s_res, &s_stop, prof);
+        __syncthreads();
+        const int last = min(s_stop, warm + iters - 1);
+        const float4 *vel = Lvel + own + last % nact * (nb + nc), *imp = vel + nb;
+        for (int b = tid; b < nb; b += BS)
+            if (Llast[b] >= 0) Lvel[b] = vel[b];
+        for (int k = tid; k < nc; k += BS) Limp[k] = imp[k];
         if (tid == 0) {
-            d.S[w].iterations = used;
-            d.S[w].residual = lastRes;
+            d.S[w].iterations = last - warm + 1;
+            d.S[w].residual = s_res[last % nact];
         }
         if (timed && tid == 0) d.ktime[6] = d.ktime[7] = __builtin_amdgcn_s_memtime();
     } else if (coloured) {
@@ -3642,13 +3743,15 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
         Lvel[b] = make_float4(v.x, v.y, wv, 0.0f);
     }
     for (int i = tid; i < nisl; i += BS) Lsol[i] = 0;
-    if (posWaves)
+    if (posWaves) {
+        Lnext2[tid] = 0;
         for (int i = tid; i < nisl; i += BS) {
             Lmin[i] = f2ord(0.0f);
             Lmin1[i] = f2ord(0.0f);
             Lmin2[i] = f2ord(0.0f);
             Lver[i] = 0;
         }
+    }
     __syncthreads();
     prof.at(kProfPos0);
     if (posWaves) {

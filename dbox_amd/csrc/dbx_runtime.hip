@@ -1352,6 +1352,14 @@ static int solve_waves(const dbx_handle *h, const Tier &T, bool lead) {
     return lead ? std::max(w, 2) : w;
 }
 
+// LDS that the exact-order solve in the residual mode is launched with, at least `lds`:
+// its overlapped sweeps keep velocities and impulses per wave, and the worlds at once on
+// a CU have 8 waves between them (solve_waves), so a wave's share of the LDS is an eighth.
+static int residual_lds(const dbx_handle *h, const StepParams &sp, uint32_t flags, int waves, int lds) {
+    if (!(flags & DBX_STEP_ORDERED) || !(sp.flags & (1u << 5)) || waves < 2) return lds;
+    return std::max(lds, std::min(h->ldsMax - 1024, h->ldsMax / 8 * waves - 1024));
+}
+
 // The step chain of one tier (b2World.Step, b2world.d:367-434, for its worlds).
 // part bits: 1 = FindNewContacts (when fixtures were added), 2 = Collide, 4 = the
 // island search and everything after it.
@@ -1370,7 +1378,7 @@ static dbx_status step_tier(dbx_handle *h, int t, const StepParams &sp, uint32_t
         const int what = ((part & 2) ? kStepCollide : 0) | ((part & 4) && sp.dt > 0.0f ? kStepSolve : 0) |
                          ((flags & DBX_STEP_ORDERED) ? kStepOrdered : 0) | ((flags & DBX_STEP_CCD) ? kStepToi : 0);
         if (what & (kStepCollide | kStepSolve))
-            DBX_HIP(h, launch_step(d, cin, sp, T.first, T.count, T.stepLds, what, lead, s));
+            DBX_HIP(h, launch_step(d, cin, sp, T.first, T.count, residual_lds(h, sp, flags, 4, T.stepLds), what, lead, s));
         return DBX_OK;
     }
     if (part & 2) DBX_HIP(h, launch_collide(d, cin, T.first, T.count, lds1, T.block, lead, s, wide, T.wideCount));
@@ -1389,11 +1397,13 @@ static dbx_status step_tier(dbx_handle *h, int t, const StepParams &sp, uint32_t
         // Without that LDS the coloured mode, whose other worlds take little time, solves the
         // joint worlds in a launch of their own: 3.4 ms for the 1,500 worlds of 200 bodies, 4.4 in one.
         if (T.mixedLds && (ordered || T.mixedLds >= T.jointLds)) {
-            DBX_HIP(h, launch_solve_mixed(d, cout, sp, T.first, T.count, waves, T.mixedLds, lead, s));
+            DBX_HIP(h, launch_solve_mixed(d, cout, sp, T.first, T.count, waves, residual_lds(h, sp, flags, waves, T.mixedLds),
+                                          lead, s));
         } else {
             if (T.jointWorlds < T.count) {
                 if (T.wideCount < T.count)
-                    DBX_HIP(h, launch_solve_wave(d, cout, sp, T.first, T.count, waves, lds1, lead, s));
+                    DBX_HIP(h, launch_solve_wave(d, cout, sp, T.first, T.count, waves,
+                                                 residual_lds(h, sp, flags, waves, lds1), lead, s));
                 else
                     DBX_HIP(h, launch_solve(d, cout, sp, T.first, T.count, ordered ? 256 : T.block, ordered ? lds1 : 0,
                                             lead, s));
