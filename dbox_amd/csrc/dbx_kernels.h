@@ -46,11 +46,11 @@ hipError_t launch_step(const Dev &d, int cin, const StepParams &sp, int worldOff
 // a tier in which some worlds have joints, in one launch (waves as for launch_solve_wave)
 hipError_t launch_solve_mixed(const Dev &d, int cur, const StepParams &sp, int worldOffset, int nworlds, int waves,
                               int ldsBytes, bool lead, hipStream_t s);
-// the joint worlds [first, first + nworlds) of Dev.jointOrder (launch_solve and
-// launch_solve_wave skip joint worlds)
+// the joint worlds [first, first + nworlds) of Dev.jointOrder, 64 to 256 threads each
+// (launch_solve and launch_solve_wave skip joint worlds)
 size_t solve_joint_lds_bytes(int bodies, int constraints, int joints);
-hipError_t launch_solve_joint(const Dev &d, int cur, const StepParams &sp, int first, int nworlds, int ldsBytes, bool lead,
-                              hipStream_t s);
+hipError_t launch_solve_joint(const Dev &d, int cur, const StepParams &sp, int first, int nworlds, int threads,
+                              int ldsBytes, bool lead, hipStream_t s);
 size_t broadphase_scratch_bytes(int proxies);
 
 // A world whose broadphase scratch does not fit in one workgroup's LDS: its pairs

@@ -3433,7 +3433,7 @@ __global__ __launch_bounds__(256) void k_solve(Dev d, int cur, StepParams sp, in
 // a body, constraint or joint: they lie in LDS where they fit, and the islands are dealt
 // over the waves, since the lanes of one wave wait for each other's joint kinds.  64
 // worlds of some 44 bodies and 25 joints: 312 us a step from global memory with the
-// islands on one wave, 197 so.
+// islands on one wave, 197 so (joint_launch in the runtime chooses waves and LDS).
 template <bool kLead>
 __global__ __launch_bounds__(256) void k_solve_joint(Dev d, int cur, StepParams sp, int first, int ldsBytes) {
     extern __shared__ __align__(16) char lds[];
@@ -6389,10 +6389,11 @@ hipError_t launch_solve_mixed(const Dev &d, int cur, const StepParams &sp, int w
 size_t solve_joint_lds_bytes(int bodies, int constraints, int joints) {
     return joint_lds_bytes(bodies, constraints, joints);
 }
-hipError_t launch_solve_joint(const Dev &d, int cur, const StepParams &sp, int first, int nworlds, int ldsBytes, bool lead,
-                              hipStream_t s) {
+hipError_t launch_solve_joint(const Dev &d, int cur, const StepParams &sp, int first, int nworlds, int threads,
+                              int ldsBytes, bool lead, hipStream_t s) {
     if (nworlds <= 0) return hipSuccess;
-    DBX_LAUNCH(k_solve_joint, lead, dim3(nworlds), dim3(256), ldsBytes, s, d, cur, sp, first, ldsBytes);
+    if (threads < 64 || threads > 256 || (threads & 63)) return hipErrorInvalidValue;
+    DBX_LAUNCH(k_solve_joint, lead, dim3(nworlds), dim3(threads), ldsBytes, s, d, cur, sp, first, ldsBytes);
     return hipGetLastError();
 }
 size_t broadphase_scratch_bytes(int proxies) { return bp_bytes(proxies); }

@@ -632,6 +632,34 @@ bool build_world(const dbx_body_def *bodies, int nb, const dbx_fixture_def *fx, 
 // state does not fit there runs from global memory instead), and each tier
 // runs its whole step chain on its own stream, so that the many small worlds
 // proceed while the few largest ones, which set the step time, are solved.
+// Threads per workgroup and LDS of a launch of n joint worlds, whose state takes `state`
+// bytes of LDS at most and which can count on `least` bytes.  With its state in LDS a world
+// takes two thirds of the time, and its islands spread over four waves a little less than
+// on one; but 8 waves fit a CU, and LDS for its state leaves one or two workgroups there, so
+// a tier of more worlds than the device has room for takes the form that needs the fewest
+// rounds for its time.  Microseconds a step with state in LDS and four waves, and with the
+// form chosen here: 512 worlds of 92 bodies 867 and the same, 512 of 132 2,620 and 2,180
+// (global memory, four waves), 700 of 132 3,680 and 2,510 (two waves), 1,500 of 72 1,360
+// and 1,045 (one wave).
+struct JointLaunch {
+    int threads = 256, lds = 0;
+};
+JointLaunch joint_launch(int n, int state, int least, int cus, int ldsMax) {
+    JointLaunch best;
+    double bestCost = 0.0;
+    for (int lds : {state, std::min(state, least)})
+        for (int t : {256, 128, 64}) {
+            const int atOnce = std::max(cus, 1) * std::min(512 / t, ldsMax / std::max(lds, 1));
+            const double one = (lds < state ? 1.36 : 1.0) * (t == 256 ? 1.0 : t == 128 ? 1.04 : 1.09);
+            const double cost = one * ((n + atOnce - 1) / atOnce);
+            if (bestCost > 0.0 && cost >= bestCost) continue;
+            bestCost = cost;
+            best.threads = t;
+            best.lds = lds;
+        }
+    return best;
+}
+
 struct Tier {
     int first = 0, count = 0; // range in the launch order
     int lds = 0;
@@ -641,7 +669,8 @@ struct Tier {
     hipEvent_t done = nullptr;
     hipEvent_t t0 = nullptr, t1 = nullptr; // chain timing while autotuning
     bool own = false;         // stream and event created for this tier
-    int jointLds = 0;         // LDS of its joint solve (0: no world of it has joints)
+    int jointLds = 0;         // LDS that holds the joint solve's state (0: no world of it has joints)
+    JointLaunch joint;        // launch of the joint worlds alone
     int mixedLds = 0;         // LDS of the launch that solves its worlds with and without joints (0: all or none have joints)
     int stepLds = 0;          // LDS of its one-launch step (0: a launch per phase)
     int jointFirst = 0, jointWorlds = 0; // its worlds with joints (range in Dev.jointOrder)
@@ -1068,6 +1097,7 @@ dbx_status dbx_finalize(dbx_handle *h) {
             }
             T.wideCount = (int)h->wide.size() - T.wideFirst;
             T.jointWorlds = (int)jointOrder.size() - T.jointFirst;
+            if (T.jointWorlds > 0) T.joint = joint_launch(T.jointWorlds, T.jointLds, lds1, h->cuCount, h->ldsMax);
             // Joint worlds beside the others in one launch (both sides measured at k_solve_mixed),
             // with LDS for the joint worlds' state where the extra rounds of workgroups that it
             // means cost the others less than it saves the joint worlds, some 3 to 5 us a body and
@@ -1408,7 +1438,7 @@ static dbx_status step_tier(dbx_handle *h, int t, const StepParams &sp, uint32_t
                     DBX_HIP(h, launch_solve(d, cout, sp, T.first, T.count, ordered ? 256 : T.block, ordered ? lds1 : 0,
                                             lead, s));
             }
-            DBX_HIP(h, launch_solve_joint(d, cout, sp, T.jointFirst, T.jointWorlds, T.jointLds, lead, s));
+            DBX_HIP(h, launch_solve_joint(d, cout, sp, T.jointFirst, T.jointWorlds, T.joint.threads, T.joint.lds, lead, s));
         }
         if (ordered && T.wideCount && d.iwParent && (sp.flags & kStepGrouped))
             DBX_HIP(h, launch_solve_groups(d, cout, sp, wide, T.wideCount, lds1, lead, s));

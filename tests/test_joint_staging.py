@@ -79,3 +79,25 @@ def test_joint_worlds_among_others_equal_them_alone(mix, mode):
         assert mixed.solver_stats()[0][w] == alone.solver_stats()[0][0] and mixed.residuals()[w] == alone.residuals()[0]
         alone.close()
     mixed.close()
+
+
+# joint worlds alone, as many as each form of their launch is chosen for: state in LDS, from
+# global memory on four, two and one wave
+@pytest.mark.parametrize("worlds,debris", [(300, 60), (512, 100), (700, 100), (1500, 40)])
+def test_many_joint_worlds_equal_them_alone(worlds, debris):
+    print(f"case: {worlds} joint worlds with {debris} pieces of debris", flush=True)
+    kinds = [_scattered(debris + k) for k in range(4)]
+    hs = []
+    for ws in [[kinds[k % 4] for k in range(worlds)]] + [[k] for k in kinds]:
+        h = native.StepWorlds(contacts_per_fixture=16)
+        for s in ws:
+            h.add_scene(s)
+        h.finalize()
+        h.step(DT, 8, 3, native.WARM | native.SLEEP | native.ORDERED, n=12)
+        h.sync()
+        hs.append(h)
+    for w in [0, 1, 2, 3, worlds - 4, worlds - 3, worlds - 2, worlds - 1]:
+        for read in ("bodies", "contacts", "joints"):
+            assert getattr(hs[0], read)(w).tobytes() == getattr(hs[1 + w % 4], read)(0).tobytes(), (w, read)
+    for h in hs:
+        h.close()
