@@ -624,14 +624,6 @@ bool build_world(const dbx_body_def *bodies, int nb, const dbx_fixture_def *fx, 
 
 } // namespace
 
-// ---------------------------------------------------------------------------
-// handle
-// ---------------------------------------------------------------------------
-// Worlds are launched in tiers of similar size, largest first.  A tier's island
-// search, solver and broadphase workgroups get `lds` bytes of LDS (a world whose
-// state does not fit there runs from global memory instead), and each tier
-// runs its whole step chain on its own stream, so that the many small worlds
-// proceed while the few largest ones, which set the step time, are solved.
 // Threads per workgroup and LDS of a launch of n joint worlds, whose state takes `state`
 // bytes of LDS at most and which can count on `least` bytes.  With its state in LDS a world
 // takes two thirds of the time, and its islands spread over four waves a little less than
@@ -644,7 +636,7 @@ bool build_world(const dbx_body_def *bodies, int nb, const dbx_fixture_def *fx, 
 struct JointLaunch {
     int threads = 256, lds = 0;
 };
-JointLaunch joint_launch(int n, int state, int least, int cus, int ldsMax) {
+static JointLaunch joint_launch(int n, int state, int least, int cus, int ldsMax) {
     JointLaunch best;
     double bestCost = 0.0;
     for (int lds : {state, std::min(state, least)})
@@ -660,6 +652,14 @@ JointLaunch joint_launch(int n, int state, int least, int cus, int ldsMax) {
     return best;
 }
 
+// ---------------------------------------------------------------------------
+// handle
+// ---------------------------------------------------------------------------
+// Worlds are launched in tiers of similar size, largest first.  A tier's island
+// search, solver and broadphase workgroups get `lds` bytes of LDS (a world whose
+// state does not fit there runs from global memory instead), and each tier
+// runs its whole step chain on its own stream, so that the many small worlds
+// proceed while the few largest ones, which set the step time, are solved.
 struct Tier {
     int first = 0, count = 0; // range in the launch order
     int lds = 0;
