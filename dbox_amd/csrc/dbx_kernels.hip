@@ -2023,7 +2023,7 @@ __device__ __forceinline__ float colour_sweep(const int *Lbo, int nbatch, const 
 // wave busy and more would only wait.  In a pile some body's contacts spread over
 // half the levels or more (two waves); in a tall stack a body meets its two
 // neighbours in consecutive levels, and eight sweeps could run at once: 128 stack worlds
-// iterated to a residual take 4.73 ms a step in one wave's sweeps and 0.97 in four's.
+// iterated to a residual take 4.73 ms a step in one wave's sweeps and 0.97 in eight's.
 __device__ __forceinline__ void pipe_wait(const int *Lnext, int other, int need, int &seen) {
     while (seen < need)
         seen = __builtin_amdgcn_readfirstlane(__hip_atomic_load(Lnext + 64 * other + (threadIdx.x & 63),
