@@ -1,5 +1,5 @@
-"""Read-backs and body writes through pinned memory: writes that fill the staging
-memory several times over, reads that outgrow it, and short output buffers."""
+"""Read-backs and body writes through pinned memory: writes back to back, and so many that
+they fill the staging memory several times over, reads that outgrow it, and short output buffers."""
 import ctypes as C
 
 import numpy as np
@@ -41,6 +41,32 @@ def test_writes_back_to_back_equal_writes_one_at_a_time(forces):
         h.sync()
     for w in range(0, 300, 7):
         assert a.bodies(w).tobytes() == b.bodies(w).tobytes()
+    a.close()
+    b.close()
+
+
+def test_writes_without_a_read_between_them_wrap_and_grow_the_staging_memory():
+    # 300 small worlds and one whose states alone outgrow the first 256 KiB, four times over
+    ws = [scenes.pyramid(5, seed=w) for w in range(300)] + [scenes.mixed_container(5000, 100.0, 120.0, 3)]
+    order = list(range(150)) + [300] + list(range(150, 300))
+    a, b = _handle(ws), _handle(ws)
+    states = [b.bodies(w) for w in range(len(ws))]
+    print(f"case: {4 * sum(s.nbytes for s in states) >> 10} KiB of body states written without a read", flush=True)
+    rng = np.random.default_rng(4)
+    for k in range(4):
+        for w in order:
+            st = states[w]
+            st["vx"][1:] = rng.uniform(-1, 1, len(st) - 1).astype(np.float32)
+            f = rng.uniform(-5, 5, (len(st), 3)).astype(np.float32) if (w + k) % 3 == 0 else None
+            a.write_bodies(w, st, f)
+            b.write_bodies(w, st, f)
+            b.sync()
+            st["vx"][1:] = 99.0  # the calls have copied their input
+    for h in (a, b):
+        h.step(flags=FLAGS & ~native.CCD, n=2)
+        h.sync()
+    for w in range(len(ws)):
+        assert a.bodies(w).tobytes() == b.bodies(w).tobytes(), w
     a.close()
     b.close()
 

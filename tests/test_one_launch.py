@@ -71,6 +71,23 @@ def test_one_launch_equals_separate_launches(mode, graph):
     assert events > 0 or not flags & native.CCD
 
 
+@pytest.mark.parametrize("bodies", [127, 128, 129, 130])  # up to 128 a world alone steps in one launch
+def test_worlds_around_the_body_limit(bodies):
+    print(f"case: a world of {bodies} bodies alone and among others", flush=True)
+    s = scenes.mixed_container(bodies - 1, 2.0 + bodies ** 0.5, 4.0 + 2.0 * bodies ** 0.5, bodies)
+    assert len(s.bodies) == bodies
+    one, many = _handle([s]), _handle([s], fill=1100)
+    for mode in ("default", "coloured", "residual"):
+        for h in (one, many):
+            h.set_residual(1e-3, 30)
+            h.step(DT, 8, 3, MODES[mode], n=12)
+            h.sync()
+        for read in ("bodies", "contacts", "events", "fat_aabbs", "pairs"):
+            assert getattr(one, read)(0).tobytes() == getattr(many, read)(0).tobytes(), (mode, read)
+    one.close()
+    many.close()
+
+
 def test_profile_of_a_one_launch_step():
     h = _handle([scenes.mixed_container(40, 14.0, 30.0, 3)])
     for _ in range(3):
