@@ -167,6 +167,7 @@ struct Dev {
     int nworlds;
     const int *order;       // launch order of worlds (largest first)
     const int *jointOrder;  // the worlds with joints in that order
+    const int *mixedOrder;  // launch order with each tier's worlds with joints before its others
     const WorldDesc *W;
     WorldState *S;
     // bodies

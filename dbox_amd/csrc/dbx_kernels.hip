@@ -3455,7 +3455,7 @@ __global__ __launch_bounds__(256) void k_solve_grp(Dev d, int cur, StepParams sp
 // (kStepColoured) every thread solves a constraint of each colour from
 // LDS; from global memory 256 containers' largest world took 190 us a step, so 128.
 constexpr int kMaxSolveWaves = 8;
-__device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const StepParams &sp, int worldOffset, int w,
+__device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const StepParams &sp, bool first, int w,
                                                  char *lds, int ldsBytes, ProfStamp prof) {
     const WorldDesc wd = d.W[w];
     if (solve_grouped(d, sp, wd) || wd.jointCount > 0) return;
@@ -3465,7 +3465,7 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
     const int nisl = d.S[w].islandCount;
     const bool coloured = (sp.flags & kStepColoured) != 0;
     if (solve_lds_bytes(nb, nc, nbatch, nisl) > (size_t)ldsBytes) {
-        solve_world_global<false>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, coloured ? 0 : ldsBytes, prof);
+        solve_world_global<false>(d, cur, sp, w, first, lds, coloured ? 0 : ldsBytes, prof);
         return;
     }
     const int tid = threadIdx.x, BS = blockDim.x, lane = tid & 63, wave = tid >> 6;
@@ -3536,7 +3536,7 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
     PosCon *pc = d.pc + wd.contactBase;
     const float h = sp.dt;
 
-    const bool timed = d.ktime && worldOffset + blockIdx.x == 0;
+    const bool timed = d.ktime && first;
     if (timed && tid == 0) {
         d.ktime[4] = __builtin_amdgcn_s_memtime();
         d.ktime[12] = __builtin_amdgcn_s_memrealtime();
@@ -3574,7 +3574,7 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
         Lvel[b] = make_float4(vx, vy, wv, vw);
     }
     __syncthreads();
-    if (tid == 0) prof.begin(d, worldOffset + blockIdx.x == 0);
+    if (tid == 0) prof.begin(d, first);
     // Constraints are stored in schedule order (slot j holds constraint sched[j]),
     // so a level's constraints are a contiguous range of slots.
     const int *cbatch = d.cbatch + wd.contactBase;
@@ -3886,23 +3886,25 @@ __device__ __forceinline__ void solve_wave_world(const Dev &d, int cur, const St
 template <bool kLead>
 __global__ __launch_bounds__(64 * kMaxSolveWaves) void k_solve_wave(Dev d, int cur, StepParams sp, int worldOffset, int ldsBytes) {
     extern __shared__ __align__(16) char lds[];
-    solve_wave_world(d, cur, sp, worldOffset, d.order[worldOffset + blockIdx.x], lds, ldsBytes, ProfStamp{});
+    solve_wave_world(d, cur, sp, worldOffset + blockIdx.x == 0, d.order[worldOffset + blockIdx.x], lds, ldsBytes,
+                     ProfStamp{});
 }
 
 // A tier in which some worlds have joints: both solves in one launch, so that the long
-// chains of the joint worlds run beside the other worlds' sweeps.  300 worlds of 90 bodies
-// and one of joints: 574 us a step with the joints in k_solve_wave's own kernel, from global
-// memory, 660 with k_solve_joint after k_solve_wave, 428 so; 1,500 of 320 bodies and one of
-// 400 pieces: 14.7, 20.7 and 14.2 ms.
+// chains of the joint worlds, which come first, run beside the other worlds' sweeps.  300
+// worlds of 90 bodies and one of joints: 574 us a step with the joints in k_solve_wave's own
+// kernel, from global memory, 670 with k_solve_joint after k_solve_wave, 434 so; 1,500 of
+// 320 bodies and one of 400 pieces: 14.4, 20.7 and 14.0 ms.  In the worlds' own order, where
+// a smaller joint world may start last, 1,500 of 200 bodies and one of 182 with joints take
+// 5.2 ms instead of 3.7 (exact order, state in LDS).
 template <bool kLead>
 __global__ __launch_bounds__(64 * kMaxSolveWaves) void k_solve_mixed(Dev d, int cur, StepParams sp, int worldOffset,
                                                                      int ldsBytes) {
     extern __shared__ __align__(16) char lds[];
-    const int w = d.order[worldOffset + blockIdx.x];
-    if (d.W[w].jointCount > 0)
-        solve_world_global<true>(d, cur, sp, w, worldOffset + blockIdx.x == 0, lds, ldsBytes, ProfStamp{});
-    else
-        solve_wave_world(d, cur, sp, worldOffset, w, lds, ldsBytes, ProfStamp{});
+    const int w = d.mixedOrder[worldOffset + blockIdx.x];
+    const bool first = w == d.order[0];
+    if (d.W[w].jointCount > 0) solve_world_global<true>(d, cur, sp, w, first, lds, ldsBytes, ProfStamp{});
+    else solve_wave_world(d, cur, sp, first, w, lds, ldsBytes, ProfStamp{});
 }
 
 // ---------------------------------------------------------------------------
@@ -5452,7 +5454,7 @@ __global__ __launch_bounds__(256) void k_step(Dev d, int cin, StepParams sp, int
     __syncthreads();
     prof.at(kProfSearched);
     if (d.W[w].jointCount > 0) solve_world_global<true>(d, cout, sp, w, first, lds, ldsBytes, prof);
-    else solve_wave_world(d, cout, sp, worldOffset, w, lds, ldsBytes, prof);
+    else solve_wave_world(d, cout, sp, first, w, lds, ldsBytes, prof);
     __syncthreads();
     prof.at(kProfSolved);
     broadphase_world(d, cout, w, first, lds, ldsBytes);

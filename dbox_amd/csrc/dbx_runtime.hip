@@ -635,17 +635,21 @@ bool build_world(const dbx_body_def *bodies, int nb, const dbx_fixture_def *fx, 
 // and 1,045 (one wave).
 struct JointLaunch {
     int threads = 256, lds = 0;
+    double cost = 0.0; // its time in that of one world with state in LDS and four waves
 };
+// A joint world's time grows by this where its state is in global memory, and with fewer
+// waves than four.
+constexpr double kJointGlobal = 1.36, kJointTwoWaves = 1.04, kJointOneWave = 1.09;
 static JointLaunch joint_launch(int n, int state, int least, int cus, int ldsMax) {
     JointLaunch best;
-    double bestCost = 0.0;
     for (int lds : {state, std::min(state, least)})
         for (int t : {256, 128, 64}) {
             const int atOnce = std::max(cus, 1) * std::min(512 / t, ldsMax / std::max(lds, 1));
-            const double one = (lds < state ? 1.36 : 1.0) * (t == 256 ? 1.0 : t == 128 ? 1.04 : 1.09);
+            const double one = (lds < state ? kJointGlobal : 1.0) *
+                               (t == 256 ? 1.0 : t == 128 ? kJointTwoWaves : kJointOneWave);
             const double cost = one * ((n + atOnce - 1) / atOnce);
-            if (bestCost > 0.0 && cost >= bestCost) continue;
-            bestCost = cost;
+            if (best.cost > 0.0 && cost >= best.cost) continue;
+            best.cost = cost;
             best.threads = t;
             best.lds = lds;
         }
@@ -671,9 +675,10 @@ struct Tier {
     bool own = false;         // stream and event created for this tier
     int jointLds = 0;         // LDS that holds the joint solve's state (0: no world of it has joints)
     JointLaunch joint;        // launch of the joint worlds alone
-    int mixedLds = 0;         // LDS of the launch that solves its worlds with and without joints (0: all or none have joints)
     int stepLds = 0;          // LDS of its one-launch step (0: a launch per phase)
     int jointFirst = 0, jointWorlds = 0; // its worlds with joints (range in Dev.jointOrder)
+    int jointBodies = 0, otherBodies = 0; // of its largest world with and without joints
+    long long jointSum = 0, otherSum = 0; // of all its worlds with and without joints
     int wideFirst = 0, wideCount = 0; // its worlds whose broadphase runs device-wide (range in the handle's list)
 };
 
@@ -1051,7 +1056,7 @@ dbx_status dbx_finalize(dbx_handle *h) {
     std::vector<int> order(nw);
     for (int w = 0; w < nw; ++w) order[w] = w;
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return need[a] > need[b]; });
-    std::vector<int> jointOrder;
+    std::vector<int> jointOrder, mixedOrder;
     {
         std::vector<int> sizes = {h->ldsMax};
         for (int l : {81920, 40960, 20480})
@@ -1077,12 +1082,12 @@ dbx_status dbx_finalize(dbx_handle *h) {
             const int lds1 = std::min(T.lds, h->ldsMax - 1024);
             T.wideFirst = (int)h->wide.size();
             T.jointFirst = (int)jointOrder.size();
-            int jointBodies = 0, otherBodies = 0; // of its largest world with and without joints
             for (int i = T.first; i < T.first + T.count; ++i) {
                 WorldDesc &D = h->W[order[i]];
                 if (D.jointCount > 0) jointOrder.push_back(order[i]);
-                int &most = D.jointCount > 0 ? jointBodies : otherBodies;
+                int &most = D.jointCount > 0 ? T.jointBodies : T.otherBodies;
                 most = std::max(most, D.bodyCount);
+                (D.jointCount > 0 ? T.jointSum : T.otherSum) += D.bodyCount;
                 if (D.jointCount > 0) // room for two solved contacts per fixture
                     T.jointLds = std::max(T.jointLds, (int)std::min<size_t>(h->ldsMax - 1024,
                                                           solve_joint_lds_bytes(D.bodyCount, 2 * D.fixCount, D.jointCount)));
@@ -1097,21 +1102,10 @@ dbx_status dbx_finalize(dbx_handle *h) {
             }
             T.wideCount = (int)h->wide.size() - T.wideFirst;
             T.jointWorlds = (int)jointOrder.size() - T.jointFirst;
+            mixedOrder.insert(mixedOrder.end(), jointOrder.begin() + T.jointFirst, jointOrder.end());
+            for (int i = T.first; i < T.first + T.count; ++i)
+                if (h->W[order[i]].jointCount == 0) mixedOrder.push_back(order[i]);
             if (T.jointWorlds > 0) T.joint = joint_launch(T.jointWorlds, T.jointLds, lds1, h->cuCount, h->ldsMax);
-            // Joint worlds beside the others in one launch (both sides measured at k_solve_mixed),
-            // with LDS for the joint worlds' state where the extra rounds of workgroups that it
-            // means cost the others less than it saves the joint worlds, some 3 to 5 us a body and
-            // round against 10 to 15 us a body: 1,500 worlds of 60 bodies and 60 of joints, two
-            // rounds more, step in 884 us with it and 1,181 without; 1,500 of 200 bodies and one of
-            // 184 with joints, three more, in 5.25 ms and 4.83.
-            if (T.jointWorlds > 0 && T.jointWorlds < T.count) {
-                const int lds = std::max(lds1, T.jointLds);
-                const auto rounds = [&](int bytes) {
-                    const int atOnce = std::max(h->cuCount, 1) * (h->ldsMax / bytes);
-                    return (T.count + atOnce - 1) / atOnce;
-                };
-                T.mixedLds = (long long)(rounds(lds) - rounds(lds1)) * otherBodies <= 3ll * jointBodies ? lds : lds1;
-            }
         }
         // Collide and broadphase take a contact or proxy per thread and pass, so a tier of
         // bigger worlds that leaves CUs idle takes the widest workgroup: 64 worlds of 400
@@ -1139,17 +1133,20 @@ dbx_status dbx_finalize(dbx_handle *h) {
 
     Dev &d = h->d;
     d.nworlds = nw;
-    int *dOrder, *dJointOrder;
+    int *dOrder, *dJointOrder, *dMixedOrder;
     WorldDesc *dW;
     DBX_HIP(h, dalloc(h, &dOrder, nw));
     DBX_HIP(h, dalloc(h, &dJointOrder, jointOrder.size()));
     DBX_HIP(h, upload(h, dJointOrder, jointOrder));
+    DBX_HIP(h, dalloc(h, &dMixedOrder, mixedOrder.size()));
+    DBX_HIP(h, upload(h, dMixedOrder, mixedOrder));
     DBX_HIP(h, dalloc(h, &dW, nw));
     DBX_HIP(h, dalloc(h, &d.S, nw));
     DBX_HIP(h, hipMemcpyAsync(dOrder, order.data(), nw * sizeof(int), hipMemcpyHostToDevice, h->stream));
     DBX_HIP(h, hipMemcpyAsync(dW, h->W.data(), nw * sizeof(WorldDesc), hipMemcpyHostToDevice, h->stream));
     d.order = dOrder;
     d.jointOrder = dJointOrder;
+    d.mixedOrder = dMixedOrder;
     d.W = dW;
     // bodies
     std::vector<uint32_t> bflags;
@@ -1382,6 +1379,34 @@ static int solve_waves(const dbx_handle *h, const Tier &T, bool lead) {
     return lead ? std::max(w, 2) : w;
 }
 
+// LDS of the launch that solves a mixed tier's worlds with and without joints together
+// (k_solve_mixed), or 0 for a launch each.  Three forms: together with LDS for the joint
+// worlds' state, which leaves fewer workgroups at once on the device; together without it,
+// the joint worlds from global memory; one after the other, each launch as it is best.  Their
+// times are estimated from a world's, 8 us a body with joints (and joint_launch's factors), 3
+// without in the exact order and 0.8 coloured: the longest world or all of them over the
+// workgroups at once.  Microseconds a step in the three forms: 1,500 worlds of 60 bodies and
+// 60 of 72 with joints 882, 1,160 and 1,040; 1,000 of 60 and 700 of 132 with joints 4,860,
+// 3,500 and 3,630; 1,500 of 320 and one of 432 with joints 13,900, 14,100 and 20,800; 1,500
+// of 200 and one of 182 with joints, for which the estimate misses the first, 3,690, 4,280
+// and 4,460 (coloured 3,200, 4,310 and 3,460).
+static int mixed_lds(const dbx_handle *h, const Tier &T, bool ordered, int waves, int lds1) {
+    if (T.jointWorlds == 0 || T.jointWorlds == T.count) return 0;
+    const double other = ordered ? 3.0 : 0.8, joint = 8.0;
+    const auto atOnce = [&](int lds) { return std::max(h->cuCount, 1) * std::min(std::max(8 / waves, 1), h->ldsMax / lds); };
+    const auto time = [&](double one, double all, int lds) { return std::max(one, all / atOnce(lds)); };
+    const double fewer = waves >= 4 ? 1.0 : waves >= 2 ? kJointTwoWaves : kJointOneWave;
+    const auto together = [&](int lds) {
+        const double j = joint * fewer * (lds < T.jointLds ? kJointGlobal : 1.0);
+        return time(std::max(j * T.jointBodies, other * T.otherBodies), j * T.jointSum + other * T.otherSum, lds);
+    };
+    const int staged = std::max(lds1, T.jointLds);
+    const double with = together(staged), without = together(lds1);
+    const double apart = time(other * T.otherBodies, other * T.otherSum, lds1) + joint * T.joint.cost * T.jointBodies + 30.0;
+    if (apart < with && apart < without) return 0;
+    return with <= without ? staged : lds1;
+}
+
 // LDS that the exact-order solve in the residual mode is launched with, at least `lds`:
 // its overlapped sweeps keep velocities and impulses per wave, and the worlds at once on
 // a CU have 8 waves between them (solve_waves), so a wave's share of the LDS is an eighth.
@@ -1424,11 +1449,8 @@ static dbx_status step_tier(dbx_handle *h, int t, const StepParams &sp, uint32_t
         // with the device-wide broadphase): island groups in the exact order, colour
         // batches from global memory in the coloured mode.
         const int waves = ordered ? solve_waves(h, T, lead) : std::min(T.block / 64, 8);
-        // Without that LDS the coloured mode, whose other worlds take little time, solves the
-        // joint worlds in a launch of their own: 3.4 ms for the 1,500 worlds of 200 bodies, 4.4 in one.
-        if (T.mixedLds && (ordered || T.mixedLds >= T.jointLds)) {
-            DBX_HIP(h, launch_solve_mixed(d, cout, sp, T.first, T.count, waves, residual_lds(h, sp, flags, waves, T.mixedLds),
-                                          lead, s));
+        if (const int lds = mixed_lds(h, T, ordered, waves, lds1)) {
+            DBX_HIP(h, launch_solve_mixed(d, cout, sp, T.first, T.count, waves, residual_lds(h, sp, flags, waves, lds), lead, s));
         } else {
             if (T.jointWorlds < T.count) {
                 if (T.wideCount < T.count)

@@ -43,11 +43,14 @@ def test_joint_worlds_equal_the_oracle(sizes, warm):
             assert m is None, f"{label}: {m}"
 
 
-# joint worlds beside others in the same tier: (other worlds, their bodies, debris of the joint worlds)
+# joint worlds beside others in the same tier: (other worlds, their bodies, debris of the joint
+# worlds), so that each form of the solve is chosen: together with LDS for the joint worlds'
+# state, together without it, a launch each
 MIXES = {
     "few": (300, 20, [0, 12, 40]),
     "larger LDS for all": (280, 200, [150, 170]),
-    "too many rounds for that": (2000, 200, [150, 170]),  # joints from global memory, or (coloured) a launch of their own
+    "too many rounds for that": (2000, 200, [150, 170]),
+    "many joint worlds": (1000, 60, [96 + k % 4 for k in range(700)]),
 }
 
 
@@ -57,7 +60,8 @@ def test_joint_worlds_among_others_equal_them_alone(mix, mode):
     print(f"case: joint worlds in a mixed tier, {mix}, {mode}", flush=True)
     others, size, debris = MIXES[mix]
     box = [scenes.mixed_container(size, 3.0 + size ** 0.5, 6.0 + 2.0 * size ** 0.5, k) for k in range(4)]
-    ws = [_scattered(n) for n in debris] + [box[k % 4] for k in range(others)]
+    joint = {n: _scattered(n) for n in debris}
+    ws = [joint[n] for n in debris] + [box[k % 4] for k in range(others)]
     flags = native.WARM | native.SLEEP | {"exact": native.ORDERED, "coloured": 0,
                                           "residual": native.ORDERED | native.RESIDUAL}[mode]
 
@@ -72,7 +76,7 @@ def test_joint_worlds_among_others_equal_them_alone(mix, mode):
         return h
 
     mixed = run(ws)
-    for w in range(len(debris) + 4):
+    for w in [*range(0, len(debris), max(1, len(debris) // 8)), *range(len(debris), len(debris) + 4)]:
         alone = run([ws[w]])
         for read in ("bodies", "contacts", "joints"):
             assert getattr(mixed, read)(w).tobytes() == getattr(alone, read)(0).tobytes(), f"world {w}: {read}"
